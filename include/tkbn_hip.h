@@ -110,14 +110,16 @@ typedef struct tkbn_interp_desc {
   int64_t klength;
   int32_t omega_batched;
   int32_t flags; /* TKBN_PLAN_REUSE or 0 */
-  /* Tuning of the sample-lane binned kernels (fewer than 32 coil rows, or 1-D / 3-D,
-   * or complex128): 0 = the library's choice.  tile[d] is the grid-tile edge along
+  /* Tuning of the sample-lane binned kernels (1-D / 3-D, complex128, and 2-D complex64
+   * of fewer than 32 coil rows): 0 = the library's choice, which for 2-D complex64 and
+   * numpoints <= 6 is the separable kernels; any other value asks for the sample-lane
+   * ones.  tile[d] is the grid-tile edge along
    * dimension d (raised to numpoints[d] - 1, lowered to grid_size[d]; a tile whose
    * one-row LDS staging exceeds 60 KiB is refused: prod_d (tile[d] + numpoints[d] - 1)
    * complex values for the gather, prod_d tile[d] * 16 bytes for the spread); work_target is the number of (sample, tile) entries per work
    * item of the atomic spread and per work item of the gather (>= 16).  Both are part
-   * of the plan: a workspace's plan is rebuilt when they change.  The multi-coil
-   * kernels and the unbinned gather ignore them. */
+   * of the plan: a workspace's plan is rebuilt when they change.  The separable kernels
+   * from 32 coil rows on, the 3-D multi-coil kernels and the unbinned gather ignore them. */
   int32_t tile[3];
   int32_t work_target;
 } tkbn_interp_desc;
@@ -201,9 +203,8 @@ TKBN_API int tkbn_interp_adj_noalloc(const tkbn_interp_desc* desc, const void* k
  *
  * Every problem is complex64, of the same ndim and numpoints class (all <= 6 or all
  * <= 16), with an unbatched trajectory and fewer than 32 coil rows, or fewer than 4 in
- * 3-D (the sample-lane kernels; larger problems take the multi-coil kernels, one call
- * each).  The caller
- * first makes one tkbn_interp_fwd and one tkbn_interp_adj call per problem with its
+ * 3-D (larger problems take the multi-coil kernels, one call each).  Problems on the
+ * separable and on the sample-lane kernels may mix.  The caller first makes one tkbn_interp_fwd and one tkbn_interp_adj call per problem with its
  * two workspaces (this builds the plans; the forward needs its workspace), then:
  *   tkbn_batch_create     describes the problems once: their descriptors (`adj_descs`, or
  *                         NULL for `descs`, may differ from `descs` in the tuning fields

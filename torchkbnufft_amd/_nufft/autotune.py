@@ -5,6 +5,7 @@ and adjoint fork over the batch and gather / index_add per sample,
 ``_nufft/interp.py:235-265,587-726``).  Here the binned gather and spread cut the grid
 into tiles and the hot tiles into work items of ``work_target`` entries; the best
 tile edge and target depend on the grid, the sample density and the number of rows.
+(For 2-D complex64 the default is the separable kernels, which take no tuning.)
 ``tune`` times every candidate on one problem of a geometry with HIP events (plan
 built once, then reused: plan cost is not part of the choice), keeps the fastest,
 and caches it per geometry class in this process (and, when ``TKBN_AUTOTUNE_CACHE``

@@ -8,8 +8,7 @@ problem.  Here
   their oversampled FFTs run as one fused launch over a stacked buffer;
 * every problem keeps its own trajectory plan in workspaces it owns, built once at
   the first call (the trajectories are fixed at construction);
-* when every problem takes the sample-lane kernels (complex64, fewer than 32 coil
-  rows), the interpolations of ALL problems run as one gather launch and one spread
+* when every problem has fewer than 32 coil rows (complex64), the interpolations of ALL problems run as one gather launch and one spread
   launch (``tkbn_batch_interp_fwd`` / ``_adj``): a device table holds each problem's
   geometry, plans and buffers, and each block finds its (problem, work item) from
   offsets computed on the device.  Otherwise each problem is its own launch, dealt
@@ -167,8 +166,9 @@ class BatchedKbNufft(torch.nn.Module):
         return op._tables(), op.n_shift, op.numpoints, op.table_oversamp, op.offsets
 
     def _tune(self, det: bool) -> None:
-        """Autotune each size group on its median-length problem (sample-lane kernels
-        only: from 32 coil rows the multi-coil kernels run, which take no tuning)."""
+        """Autotune each size group on its median-length problem (a tuned tile or target
+        selects the sample-lane kernels, and is kept where they beat the default; from 32
+        coil rows the multi-coil kernels run, which take no tuning)."""
         for g, members in enumerate(self.groups):
             if self.coils >= 32:
                 break

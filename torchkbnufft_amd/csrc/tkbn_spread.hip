@@ -47,6 +47,7 @@ struct TileGeom {
   int target;      // candidate samples per split
   int CC;          // coil rows per work-group
   int64_t maxwork; // work items per trajectory (upper bound)
+  int rec_entry;   // separable spread: a record per entry, else one per sample
   int64_t maxent;  // (sample, tile) entries per trajectory (upper bound)
   int own_only;    // forward plans: each sample only in the tile of its base cell
   int R[3];        // forward: staged region per dimension (T + J - 1)
@@ -59,6 +60,7 @@ struct TileGeom {
   int64_t nkeys;           // multi-coil plan: (tile, footprint column) keys
   int64_t o_hot, o_cold;   // multi-coil plan: scans of split / unsplit tiles
   int64_t o_rec_bytes;     // multi-coil plan: byte offset of the entry records
+  int64_t plan_stride;     // multi-coil plan: ints from one trajectory's plan to the next
   int64_t o_meta, o_tmp, o_sort, o_scratch;  // 3-D register-tile plan: counts, scan scratch, sort
   int64_t o_sw, o_sb;                        // 3-D register-tile plan: per-sample tap weights, bases
   int64_t pool_off_bytes, pool_slots;        // 3-D register-tile plan: piece partials
@@ -640,35 +642,14 @@ __global__ void __launch_bounds__(spread_tiles_threads(D))
 }
 
 // ---------------------------------------------------------------------------
-// multi-coil spread geometry (2-D, complex64, J <= 6; the kernel is spread_sep_kernel)
-//   One group (8 waves) per (16 x 16 tile, split, chunk of 32 coil rows); half-wave h
-//   of wave w owns tile row 2w + h of its coil row in registers, so every cell has
-//   exactly one writer and no atomics are needed.  Entries (sample, tile) are staged
-//   64 at a time and walked c0 value by c0 value (one ballot each): inside a group the
-//   column offsets are compile-time constants, so every accumulator index is fixed.
-//   Footprints are contiguous inside a tile when every grid extent is at least
-//   tile + J - 1 cells (a wrapped footprint then never meets one tile twice);
-//   smaller grids use the sample-lane kernel.
+// separable spread geometry (2-D, complex64, J <= 6; the kernel is spread_sep_kernel):
+//   entries (sample, 16 x 16 tile its footprint meets).  Footprints are contiguous inside a
+//   tile when every grid extent is at least tile + J - 1 cells (a wrapped footprint then
+//   never meets one tile twice); smaller grids use the sample-lane kernel.
 // ---------------------------------------------------------------------------
-constexpr int kRegCoils = 32;  // coil rows per work item (lanes of a wave slice)
-constexpr int kRegRowsPerWave = 64 / kRegCoils;  // tile rows of a wave: one per slice
-constexpr int kRegWaves = 8;
-constexpr int kRegThreads = 64 * kRegWaves;
-constexpr int kRegT0 = kRegRowsPerWave * kRegWaves;
-constexpr int kRegT1 = 16;
-constexpr int kRegBatch = 64;  // staged entries
-constexpr int kRegPitch = kRegCoils + 1;  // float2 per staged entry (+1: bank spread)
+constexpr int kRegT0 = 16, kRegT1 = 16;
 constexpr int kRegMinC0 = -5;  // first footprint column relative to the tile, J <= 6
 constexpr int kRegKeys = kRegT1 - kRegMinC0;  // c0 values per tile: -5 .. 15
-// A tile with more entries than kRegMaxUnsplit is split into pieces of kRegHotTarget
-// entries (their groups then add into a pre-zeroed tile); the pieces are listed
-// first so the longest work starts first.  Other tiles are one work item each.
-constexpr int kRegMaxUnsplit = 768;
-constexpr int kRegHotTarget = 768;
-
-__host__ __device__ inline int reg_splits(int v) {
-  return v <= kRegMaxUnsplit ? 1 : (v + kRegHotTarget - 1) / kRegHotTarget;
-}
 
 // Tiles met along one dimension by the footprint bm .. bm+J-1 (mod K), in footprint
 // order, with the footprint's first cell relative to each tile's origin.  The runs of
@@ -721,26 +702,19 @@ __device__ __forceinline__ void coil_sample_tiles(const Geom<float>& g, const Ti
 }
 
 // ---------------------------------------------------------------------------
-// multi-coil forward gather geometry (2-D, complex64, J <= 6; the kernel is
+// separable forward gather geometry (2-D, complex64, J <= 6; the kernel is
 // gather_sep_kernel)
 //   The plan bins every sample once, into the tile of its base cell (the footprint's
-//   first cell), keeping trajectory order inside a tile.  One group (8 waves) per
-//   (16 x 16 tile, split, chunk of 16 coil rows) stages the tile and its J-1 halo
-//   (21 x 21 cells, wrapped) in LDS with the coil row fastest.  Each quarter-wave takes
-//   one entry (lanes = the chunk's 16 rows), so a tap read by a wave is four runs of
-//   16 consecutive LDS words and conflict-free.  Short row chunks allow large tiles:
-//   the region is 1.7x the tile's cells, and each staging round covers many samples.
+//   first cell), keeping trajectory order inside a tile.  One group per (16 x 16 tile,
+//   split, chunk of coil rows) stages the tile and its J-1 halo (21 x 21 cells, wrapped) in
+//   LDS with the coil row fastest; the lanes of an entry are the chunk's rows, so a tap
+//   read by a wave is a few runs of consecutive LDS words.
 // ---------------------------------------------------------------------------
 constexpr int kGatT0 = 16, kGatT1 = 16;     // tile edges
 constexpr int kGatR0 = kGatT0 + 5;          // staged region edges (J <= 6)
 constexpr int kGatR1 = kGatT1 + 5;
 constexpr int kGatCells = kGatR0 * kGatR1;  // 441
-constexpr int kGatRows = 16;                // coil rows per work item
-constexpr int kGatPerWave = 64 / kGatRows;  // entries a wave takes at once
-constexpr int kGatPitch = kGatRows + 1;     // float2 per staged cell (odd: staging stores spread over banks)
-constexpr int kGatThreads = 512;
 constexpr int kGatTarget = 512;             // entries per work item
-static_assert(kGatCells * kGatPitch * 8 * 2 <= 160 * 1024, "two groups per CU");
 
 __device__ __forceinline__ int gat_base_tile(const Geom<float>& g, const TileGeom& tg, const float* om, int m, int* l) {
   int key = 0;
@@ -940,7 +914,7 @@ __global__ void __launch_bounds__((fwd_tiled_threads<T, JM>()))
 }
 
 // ---------------------------------------------------------------------------
-// separable multi-coil kernels (2-D, complex64, J <= 6)
+// separable kernels (2-D, complex64, J <= 6)
 //   The reference's table for dimension d holds t[i] = KB(u) exp(-i pi (N-1) u / K)
 //   at u = (i - J L / 2) / L (_nufft/utils.py:122-179), and the taps j of one sample
 //   read t[i_0 - j L] (the float32 index arithmetic of _nufft/interp.py:129-131 gives
@@ -953,11 +927,14 @@ __global__ void __launch_bounds__((fwd_tiled_threads<T, JM>()))
 //   (a table of another form, N unknown, a non-finite sample, or a rounding case) are
 //   flagged by the plan and applied with complex weights in the rotated frame, so the
 //   result is the reference's for every table.
+//   Every phase of the frame is evaluated in double and rounded once at the end: with float
+//   phases the results of few-row problems were further from 64-bit sums than those of the
+//   complex-weight kernels (12 rows, 256^2 adjoint: 1.26e-7 against 1.12e-7; now 1.07e-7).
 // ---------------------------------------------------------------------------
 struct SepGeom {
   int L[2];            // table oversampling
   int64_t o_rtab[2];   // int offsets of the real tables in the plan
-  int64_t o_ptab[2];   // int offsets of the cell phases P_d(k), k < K_d (float2) in the plan
+  int64_t o_ptab[2];   // int offsets of the cell phases P_d(k), k < K_d (double2) in the plan
   int64_t o_nm1;       // int offset of N_d - 1 (2 ints), found from the tables by the plan
 };
 
@@ -971,38 +948,41 @@ __device__ __forceinline__ int sep_nm1_estimate(const Geom<float>& g, int d) {
   return (int)llrint(-ang * (double)g.K[d] * g.Lf[d] / 3.141592653589793);
 }
 
-// exp(i pi a / q) for an integer a of any sign and q > 0; a is reduced modulo 2q first,
-// so the float angle lies in [0, 2 pi)
-__device__ __forceinline__ float2 pi_phase(int64_t a, int64_t q) {
+// exp(i pi a / q) for an integer a of any sign and q > 0; a is reduced modulo 2q first.
+// In double: a float angle in [0, 2 pi) is off by up to 1.9e-7, which was the largest error
+// of the rotated frame (only plans evaluate phases).
+__device__ __forceinline__ double2 pi_phase_d(int64_t a, int64_t q) {
   int64_t r = a % (2 * q);
   if (r < 0) r += 2 * q;
-  // r and q are exact floats below 2^24, and the float division is correctly rounded
-  const float x = q < (1 << 23) ? (float)r / (float)q : (float)((double)r / (double)q);
-  float s, c;
-  sincospif(x, &s, &c);
-  return make_float2(c, s);
+  double s, c;
+  sincospi((double)r / (double)q, &s, &c);
+  return make_double2(c, s);
 }
 
 // P(p) = exp(i pi (N - 1) p / K) for a cell coordinate p >= 0 that may run past the
 // grid's end (the gather's staged halo): P(p) = P(p - K) (-1)^(N - 1), from the plan's
 // table of P(k), k < K.
-__device__ __forceinline__ float2 sep_cell_phase(const float2* P, int K, int nm1, int p) {
+__device__ __forceinline__ float2 sep_cell_phase(const double2* P, int K, int nm1, int p) {
   bool flip = false;
   while (p >= K) {
     p -= K;
     flip = flip != ((nm1 & 1) != 0);
   }
-  const float2 v = P[p];
-  return flip ? make_float2(-v.x, -v.y) : v;
+  const double2 v = P[p];
+  return flip ? make_float2((float)-v.x, (float)-v.y) : make_float2((float)v.x, (float)v.y);
 }
 
-// Plan record of one (sample, tile) entry (64 bytes).  Forward: the sample's base cell
-// relative to the tile; adjoint: the footprint's first cell relative to the tile.
+// Plan record of one sample (64 bytes).  The forward keeps them in tile order; the adjoint,
+// whose samples have an entry in every tile that they reach, in sample order, and lists a
+// tile's samples in perm (80 bytes a sample; a record per entry took up to 272, and was
+// written 1.7 times).
 struct SepRec {
-  int me;      // sample index | exception flag << 31
-  int rc;      // (p0 + 8) | (p1 + 8) << 8
+  int me;      // forward: sample index; adjoint: first cell of the footprint along dimension 0;
+               // exception flag << 31
+  int rc;      // forward: base cell relative to the tile, (p0 + 8) | (p1 + 8) << 8; adjoint:
+               // first cell along dimension 1
   float2 F;    // forward: shift phase * B_0 * B_1 (exceptions: the shift phase alone);
-               // adjoint: the conjugate
+               // adjoint: the conjugate, for the wrapped footprint's first cell
   float w0[6]; // R_0 of taps 0..5 along dimension 0
   float w1[6]; // R_1 along dimension 1
 };
@@ -1053,30 +1033,17 @@ __device__ __forceinline__ float2 sep_tap_weight(const Geom<float>& g, int d, fl
   return g.table[d][ti];
 }
 
-// Complex weights of a forward exception entry in the rotated frame (same index as its
-// record): t_d[i_j] conj(P_d(p_d + j)).
-struct SepX {
-  float2 w0[6];
-  float2 w1[6];
-};
-static_assert(sizeof(SepX) == 96, "exception record is 96 bytes");
-
-__device__ __forceinline__ void sep_exception_weights(const Geom<float>& g, const int (&nm1)[2], float om0, float om1,
-                                                      int64_t p0, int64_t p1, SepX& x) {
-#pragma unroll
-  for (int j = 0; j < 6; ++j) {
-    x.w0[j] = cmul_conj(sep_tap_weight(g, 0, om0, j), pi_phase((int64_t)nm1[0] * (p0 + j), g.K[0]));
-    x.w1[j] = cmul_conj(sep_tap_weight(g, 1, om1, j), pi_phase((int64_t)nm1[1] * (p1 + j), g.K[1]));
-  }
+// Angle of a tap's phase B_d = exp(-i pi (N-1) n / (L K)) over pi, n = (i_0 - J L / 2) + L p
+// (p: tap 0's cell in the tile frame), reduced modulo 2
+__device__ __forceinline__ double sep_turn(const Geom<float>& g, const SepGeom& sg, int nm1, int d, int ti0, int64_t p) {
+  const int64_t q = (int64_t)sg.L[d] * g.K[d];
+  return (double)((int64_t)nm1 * ((int64_t)(ti0 - g.center[d]) + (int64_t)sg.L[d] * p) % (2 * q)) / (double)q;
 }
-
-// B_d = exp(-i pi (N-1) n / (L K)), n = (i_0 - J L / 2) + L p (p: tap 0's cell in the
-// tile frame)
-__device__ __forceinline__ float2 sep_b(const Geom<float>& g, const SepGeom& sg, int nm1, int d, int ti0, int64_t p) {
-  const int64_t L = sg.L[d];
-  const int64_t n = (int64_t)(ti0 - g.center[d]) + L * p;
-  const float2 e = pi_phase((int64_t)nm1 * n, L * g.K[d]);
-  return make_float2(e.x, -e.y);
+// exp(i (theta - pi turns)), evaluated in double and rounded once
+__device__ __forceinline__ float2 sep_factor(float theta, double turns) {
+  double s, c;
+  sincos((double)theta - turns * 3.14159265358979323846, &s, &c);
+  return make_float2((float)c, (float)s);
 }
 
 // Real tables R_d[i] = Re(t_d[i] exp(i pi (N-1)(i - J L / 2) / (L K))) into the plan;
@@ -1094,9 +1061,9 @@ __device__ __forceinline__ void sep_table_prep(const Geom<float>& g, const SepGe
     const int d = i < n0 ? 0 : 1;
     const int m = (int)(d == 0 ? i : i - n0);
     const float2 t = g.table[d][m];
-    const float2 p = pi_phase((int64_t)nm1[d] * (m - g.center[d]), (int64_t)sg.L[d] * g.K[d]);
-    const float re = t.x * p.x - t.y * p.y;
-    const float im = t.x * p.y + t.y * p.x;
+    const double2 p = pi_phase_d((int64_t)nm1[d] * (m - g.center[d]), (int64_t)sg.L[d] * g.K[d]);
+    const float re = (float)((double)t.x * p.x - (double)t.y * p.y);
+    const float im = (float)((double)t.x * p.y + (double)t.y * p.x);
     reinterpret_cast<float*>(plan + sg.o_rtab[d])[m] = re;
     if (!(fabsf(im) <= 0x1p-19f * (fabsf(t.x) + fabsf(t.y)))) atomicOr(flag, 1);
   }
@@ -1104,7 +1071,7 @@ __device__ __forceinline__ void sep_table_prep(const Geom<float>& g, const SepGe
        i += (int64_t)gridDim.x * blockDim.x) {
     const int d = i < g.K[0] ? 0 : 1;
     const int k = (int)(d == 0 ? i : i - g.K[0]);
-    reinterpret_cast<float2*>(plan + sg.o_ptab[d])[k] = pi_phase((int64_t)nm1[d] * k, g.K[d]);
+    reinterpret_cast<double2*>(plan + sg.o_ptab[d])[k] = pi_phase_d((int64_t)nm1[d] * k, g.K[d]);
   }
 }
 
@@ -1115,12 +1082,85 @@ __device__ __forceinline__ void sep_gat_record(const Geom<float>& g, const TileG
 __device__ __forceinline__ void sep_spr_scatter_item(const Geom<float>& g, const TileGeom& tg, const SepGeom& sg,
                                                      const float* __restrict__ omega, int* __restrict__ ws, int m);
 
+// Scan of per-tile counts into tile starts and the work list, longest work first: tiles
+// above `target` entries, cut into pieces of `target`, then the others by size class (above
+// 1/2, 1/4, 1/8 of the target, the rest), so that no long tile starts late (16 coils x 4,
+// 320^2 radial: the spread's waves were 1.2 per SIMD on average with the tiles in grid
+// order, 2 fit).  Empty tiles get no item when `skip_empty`.
+constexpr int kSepClasses = 4;
+__device__ __forceinline__ void sep_plan_scan(const TileGeom& tg, int* __restrict__ plan, bool skip_empty, int* sbuf) {
+  const int target = tg.target;
+  const int* count = plan + tg.o_count;
+  int* start = plan + tg.o_start;
+  int* cursor = plan + tg.o_cursor;
+  int* wstart = plan + tg.o_wstart;
+  int* work = plan + tg.o_work;
+  int* hot = plan + tg.o_hot;
+  int* rank = plan + tg.o_cold;
+  const int NB = tg.NB;
+  const auto size_class = [&](int v) {  // 0: split; kSepClasses + 1: no item
+    if (v > target) return 0;
+    if (v == 0 && skip_empty) return kSepClasses + 1;
+    return 2 * v > target ? 1 : 4 * v > target ? 2 : 8 * v > target ? 3 : 4;
+  };
+  block_exclusive_scan(count, start, NB, sbuf);
+  for (int t = threadIdx.x; t < NB; t += blockDim.x) {
+    cursor[t] = start[t];
+    const int v = count[t];
+    work[t] = v > target ? (v + target - 1) / target : 0;
+  }
+  __syncthreads();
+  block_exclusive_scan(work, hot, NB, sbuf);
+  int nwork = hot[NB];
+  __syncthreads();  // `work` and `cursor` are the scans' scratch below
+  for (int t = threadIdx.x; t < NB; t += blockDim.x)
+    if (size_class(count[t]) == 0) wstart[t] = hot[t];
+  for (int c = 1; c <= kSepClasses; ++c) {
+    for (int t = threadIdx.x; t < NB; t += blockDim.x) work[t] = size_class(count[t]) == c ? 1 : 0;
+    __syncthreads();
+    block_exclusive_scan(work, rank, NB, sbuf);
+    for (int t = threadIdx.x; t < NB; t += blockDim.x)
+      if (size_class(count[t]) == c) wstart[t] = nwork + rank[t];
+    nwork += rank[NB];
+    __syncthreads();
+  }
+  const int cap = (int)tg.maxwork;
+  for (int t = threadIdx.x; t < NB; t += blockDim.x) {
+    const int c = size_class(count[t]);
+    if (c > kSepClasses) continue;
+    const int items = c == 0 ? hot[t + 1] - hot[t] : 1;
+    const int a = wstart[t], e = min(a + items, cap);
+    for (int w = a; w < e; ++w) work[w] = t;
+  }
+  if (threadIdx.x == 0) plan[tg.o_nwork] = min(nwork, cap);
+}
+
+// The count kernels' end: the last block of a trajectory to finish scans its counts (its
+// own launch for the scan cost 5 us of every call, also where the plan is kept).  The
+// counts are device-scope atomics, and each wave waits for its own before its block signs
+// off; nothing else is read here (a release fence by every block wrote the L2 back 800
+// times: 69 instead of 62 us for 206 000 new samples).
+__device__ __forceinline__ void sep_scan_if_last(const TileGeom& tg, int* __restrict__ plan, bool skip_empty) {
+  __shared__ int sbuf[256];
+  __shared__ bool last;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) last = atomicAdd(plan + tg.o_count + tg.NB + 1, 1) == (int)gridDim.x - 1;
+  __syncthreads();
+  if (!last) return;
+  __threadfence();
+  sep_plan_scan(tg, plan, skip_empty, sbuf);
+}
+
 // Forward: each sample once, in the 16 x 16 tile of its base cell (trajectory order
 // within a tile as far as the building atomics keep it); count[NB] is the table flag.
+// blockIdx.y: the trajectory (one plan each).
 __global__ void __launch_bounds__(256)
     sep_gat_count_kernel(const Geom<float> g, const TileGeom tg, const SepGeom sg, const float* __restrict__ omega,
                          int* __restrict__ ws, const CacheHdr* cache) {
   if (cache_hit(cache)) return;  // cached plan reused
+  omega += (int64_t)blockIdx.y * 2 * g.M;
+  ws += (int64_t)blockIdx.y * tg.plan_stride;
   sep_table_prep(g, sg, ws, ws + tg.o_count + tg.NB);
   for (int m0 = blockIdx.x * blockDim.x; m0 < g.M; m0 += gridDim.x * blockDim.x) {
     const int m = m0 + threadIdx.x;
@@ -1129,12 +1169,15 @@ __global__ void __launch_bounds__(256)
     const int key = live ? gat_base_tile(g, tg, omega, m, l) : 0;
     wave_aggregated_add(ws + tg.o_count, key, live);
   }
+  sep_scan_if_last(tg, ws, true);
 }
 
 __global__ void __launch_bounds__(256)
     sep_gat_scatter_kernel(const Geom<float> g, const TileGeom tg, const SepGeom sg, const float* __restrict__ omega,
                            int* __restrict__ ws, const CacheHdr* cache) {
   if (cache_hit(cache)) return;  // cached plan reused
+  omega += (int64_t)blockIdx.y * 2 * g.M;
+  ws += (int64_t)blockIdx.y * tg.plan_stride;
   for (int m0 = blockIdx.x * blockDim.x; m0 < g.M; m0 += gridDim.x * blockDim.x) {
     const int m = m0 + threadIdx.x;
     const bool live = m < g.M;
@@ -1154,7 +1197,7 @@ __device__ __forceinline__ void sep_gat_record(const Geom<float>& g, const TileG
   const float om0 = omega[m], om1 = omega[g.M + m];
   const SepTaps a = sep_taps(g, 0, om0), b = sep_taps(g, 1, om1);
   const float theta = sample_theta<float, 2>(g, omega, m);
-  float2 F = make_float2(cosf(theta), sinf(theta));
+  double turns = 0.;
   SepRec rec;
   const bool exc = !(tab_ok && a.regular && b.regular);
   const float* R0 = reinterpret_cast<const float*>(ws + sg.o_rtab[0]);
@@ -1168,19 +1211,12 @@ __device__ __forceinline__ void sep_gat_record(const Geom<float>& g, const TileG
     // tap 0's cell in the tile frame is the wrapped base (the staged region continues
     // past the grid's end without wrapping its coordinates)
     const int o0 = (key / tg.bstride[0]) % tg.nb[0] * kGatT0, o1 = (key / tg.bstride[1]) % tg.nb[1] * kGatT1;
-    F = cmul(F, cmul(sep_b(g, sg, nm10, 0, a.ti0, o0 + l[0]), sep_b(g, sg, nm11, 1, b.ti0, o1 + l[1])));
+    turns = sep_turn(g, sg, nm10, 0, a.ti0, o0 + l[0]) + sep_turn(g, sg, nm11, 1, b.ti0, o1 + l[1]);
   }
   rec.me = m | (exc ? (int)0x80000000u : 0);
   rec.rc = (l[0] + 8) | ((l[1] + 8) << 8);
-  rec.F = F;
+  rec.F = sep_factor(theta, turns);
   reinterpret_cast<SepRec*>(reinterpret_cast<char*>(ws) + tg.o_rec_bytes)[pos] = rec;
-  if (exc) {
-    const int o0 = (key / tg.bstride[0]) % tg.nb[0] * kGatT0, o1 = (key / tg.bstride[1]) % tg.nb[1] * kGatT1;
-    const int nm1[2] = {nm10, nm11};
-    SepX x;
-    sep_exception_weights(g, nm1, om0, om1, o0 + l[0], o1 + l[1], x);
-    reinterpret_cast<SepX*>(reinterpret_cast<char*>(ws) + tg.o_rec_bytes + tg.maxent * (int64_t)sizeof(SepRec))[pos] = x;
-  }
 }
 
 // Adjoint: one entry per (sample, 16 x 16 tile its footprint meets); count[NB] is the
@@ -1190,6 +1226,8 @@ __global__ void __launch_bounds__(256)
     sep_spr_count_kernel(const Geom<float> g, const TileGeom tg, const SepGeom sg, const float* __restrict__ omega,
                          int* __restrict__ ws, const CacheHdr* cache) {
   if (cache_hit(cache)) return;  // cached plan reused
+  omega += (int64_t)blockIdx.y * 2 * g.M;
+  ws += (int64_t)blockIdx.y * tg.plan_stride;
   sep_table_prep(g, sg, ws, ws + tg.o_count + tg.NB);
   for (int m0 = blockIdx.x * blockDim.x; m0 < g.M; m0 += gridDim.x * blockDim.x) {
     const int m = m0 + threadIdx.x;
@@ -1202,17 +1240,36 @@ __global__ void __launch_bounds__(256)
       wave_aggregated_add(count, tkey, valid);
     });
   }
+  sep_scan_if_last(tg, ws, false);
 }
 
+// Zeroes tile t of rows [r0, r1) if its pieces add into the grid
+__device__ __forceinline__ void sep_zero_hot_item(const Geom<float>& g, const TileGeom& tg, const int* plan,
+                                                  float2* __restrict__ grid, int t, int64_t r0, int64_t r1);
+
+// Blocks x < nscatter write the records of a new plan (trajectory blockIdx.y), the others
+// clear what the spread adds into, on every call: block nscatter + t + NB * y, tile t and
+// rows [64 y, 64 y + 64).
 __global__ void __launch_bounds__(256)
     sep_spr_scatter_kernel(const Geom<float> g, const TileGeom tg, const SepGeom sg, const float* __restrict__ omega,
-                           int* __restrict__ ws, const CacheHdr* cache) {
+                           int* __restrict__ ws, const CacheHdr* cache, int nscatter, float2* __restrict__ grid) {
+  if ((int)blockIdx.x >= nscatter) {
+    const int64_t b = blockIdx.y;
+    const int x = (int)blockIdx.x - nscatter, y = x / tg.NB;
+    const int64_t nrows = g.batched ? g.C : g.B * g.C, rowbase = g.batched ? b * g.C : 0;
+    const int64_t r0 = (int64_t)y * 64;
+    const int64_t r1 = r0 + 64 < nrows ? r0 + 64 : nrows;
+    sep_zero_hot_item(g, tg, ws + b * tg.plan_stride, grid, x - y * tg.NB, rowbase + r0, rowbase + r1);
+    return;
+  }
   if (cache_hit(cache)) return;  // cached plan reused
-  for (int m0 = blockIdx.x * blockDim.x; m0 < g.M; m0 += gridDim.x * blockDim.x)
+  omega += (int64_t)blockIdx.y * 2 * g.M;
+  ws += (int64_t)blockIdx.y * tg.plan_stride;
+  for (int m0 = blockIdx.x * blockDim.x; m0 < g.M; m0 += nscatter * blockDim.x)
     sep_spr_scatter_item(g, tg, sg, omega, ws, m0 + threadIdx.x);
 }
 
-// the adjoint entries of sample m (m >= M: a dead lane that still takes part in the
+// the adjoint's record and entries of sample m (m >= M: a dead lane that still takes part in the
 // wave-aggregated cursor increments)
 __device__ __forceinline__ void sep_spr_scatter_item(const Geom<float>& g, const TileGeom& tg, const SepGeom& sg,
                                                      const float* __restrict__ omega, int* __restrict__ ws, int m) {
@@ -1220,13 +1277,12 @@ __device__ __forceinline__ void sep_spr_scatter_item(const Geom<float>& g, const
   int tl[2][3], off[2][3], n[2];
   coil_sample_tiles(g, tg, omega, m, live, tl, off, n);
   SepTaps a{}, b{};
-  float2 ns = make_float2(0.f, 0.f);
+  float theta = 0.f;
   bool regular = false;
   if (live) {
     a = sep_taps(g, 0, omega[m]);
     b = sep_taps(g, 1, omega[g.M + m]);
-    const float theta = sample_theta<float, 2>(g, omega, m);
-    ns = make_float2(cosf(theta), sinf(theta));
+    theta = sample_theta<float, 2>(g, omega, m);
     regular = ws[tg.o_count + tg.NB] == 0 && a.regular && b.regular;
   }
   const float* R0 = reinterpret_cast<const float*>(ws + sg.o_rtab[0]);
@@ -1234,83 +1290,48 @@ __device__ __forceinline__ void sep_spr_scatter_item(const Geom<float>& g, const
   const int nm10 = ws[sg.o_nm1], nm11 = ws[sg.o_nm1 + 1];
   int* plan = ws;
   SepRec* recs = reinterpret_cast<SepRec*>(reinterpret_cast<char*>(ws) + tg.o_rec_bytes);
-  coil_for_each_entry(tg, tl, off, n, live, [&](int key, int ai, int ci, bool valid) {
-    const int tkey = valid ? (key - (off[1][ci] - kRegMinC0)) / kRegKeys : 0;
-    const int pos = wave_aggregated_inc(plan + tg.o_cursor, tkey, valid);
-    if (valid) {
-      SepRec rec;
-      float2 F = ns;
-      if (regular) {
-        const int o0 = (tkey / tg.bstride[0]) % tg.nb[0] * kRegT0, o1 = (tkey / tg.bstride[1]) % tg.nb[1] * kRegT1;
-        F = cmul(F, cmul(sep_b(g, sg, nm10, 0, a.ti0, (int64_t)o0 + off[0][ai]),
-                         sep_b(g, sg, nm11, 1, b.ti0, (int64_t)o1 + off[1][ci])));
-      }
+  const int c0 = live ? (int)sample_base_wrapped<float>(g, 0, omega[m]) : 0;
+  const int c1 = live ? (int)sample_base_wrapped<float>(g, 1, omega[g.M + m]) : 0;
+  SepRec rec;
+  const float2 F = sep_factor(
+      theta, regular ? sep_turn(g, sg, nm10, 0, a.ti0, c0) + sep_turn(g, sg, nm11, 1, b.ti0, c1) : 0.);
 #pragma unroll
-      for (int j = 0; j < 6; ++j) {
-        rec.w0[j] = (regular && j < g.J[0]) ? R0[a.ti0 - j * sg.L[0]] : 0.f;
-        rec.w1[j] = (regular && j < g.J[1]) ? R1[b.ti0 - j * sg.L[1]] : 0.f;
-      }
-      rec.me = m | (regular ? 0 : (int)0x80000000u);
-      rec.rc = (off[0][ai] + 8) | ((off[1][ci] + 8) << 8);
-      rec.F = make_float2(F.x, -F.y);
-      plan[tg.o_perm + pos] = rec.me;
-      recs[pos] = rec;
-    }
+  for (int j = 0; j < 6; ++j) {
+    rec.w0[j] = (regular && j < g.J[0]) ? R0[a.ti0 - j * sg.L[0]] : 0.f;
+    rec.w1[j] = (regular && j < g.J[1]) ? R1[b.ti0 - j * sg.L[1]] : 0.f;
+  }
+  rec.me = c0 | (regular ? 0 : (int)0x80000000u);
+  rec.rc = c1;
+  rec.F = make_float2(F.x, -F.y);
+  coil_for_each_entry(tg, tl, off, n, live, [&](int key, int, int c, bool valid) {
+    const int tkey = valid ? (key - (off[1][c] - kRegMinC0)) / kRegKeys : 0;
+    const int pos = wave_aggregated_inc(plan + tg.o_cursor, tkey, valid);
+    if (!valid) return;
+    plan[tg.o_perm + pos] = m;
+    if (tg.rec_entry) recs[pos] = rec;
   });
-}
-
-// Scan of per-tile counts into tile starts and the work list: tiles above `maxunsplit`
-// entries are cut into pieces of `target`, listed first (longest work first); empty
-// tiles get no item when `skip_empty`.
-__global__ void __launch_bounds__(1024) sep_plan_scan_kernel(const TileGeom tg, int* __restrict__ ws,
-                                                            const CacheHdr* cache, int maxunsplit, int target,
-                                                            int skip_empty) {
-  if (cache_hit(cache)) return;  // cached plan reused
-  __shared__ int sbuf[1024];
-  int* plan = ws;
-  const int* count = plan + tg.o_count;
-  int* start = plan + tg.o_start;
-  int* cursor = plan + tg.o_cursor;
-  int* wstart = plan + tg.o_wstart;
-  int* work = plan + tg.o_work;
-  int* hot = plan + tg.o_hot;
-  int* cold = plan + tg.o_cold;
-  const int NB = tg.NB;
-  block_exclusive_scan(count, start, NB, sbuf);
-  for (int t = threadIdx.x; t < NB; t += blockDim.x) {
-    cursor[t] = start[t];
-    const int v = count[t];
-    const int ns = v <= maxunsplit ? 1 : (v + target - 1) / target;
-    work[t] = ns > 1 ? ns : 0;
-    wstart[t] = (ns == 1 && (v > 0 || !skip_empty)) ? 1 : 0;
-  }
-  __syncthreads();
-  block_exclusive_scan(work, hot, NB, sbuf);
-  block_exclusive_scan(wstart, cold, NB, sbuf);
-  const int nhot = hot[NB];
-  const int cap = (int)tg.maxwork;
-  for (int t = threadIdx.x; t < NB; t += blockDim.x) {
-    const int ns = hot[t + 1] - hot[t];
-    wstart[t] = ns > 0 ? hot[t] : nhot + cold[t];
-  }
-  __syncthreads();
-  for (int t = threadIdx.x; t < NB; t += blockDim.x) {
-    const int ns = hot[t + 1] - hot[t];
-    const int items = ns > 0 ? ns : cold[t + 1] - cold[t];
-    const int a = wstart[t], e = min(a + items, cap);
-    for (int w = a; w < e; ++w) work[w] = t;
-  }
-  if (threadIdx.x == 0) plan[tg.o_nwork] = min(nhot + cold[NB], cap);
+  if (live && !tg.rec_entry) recs[m] = rec;
 }
 
 // ---- forward gather ------------------------------------------------------------------
-// A group per 16 x 16 tile, piece and chunk of 16 coil rows; the tile and its halo are
-// staged in LDS with the coil row fastest, rotated: region = grid * P_0 * P_1; a
-// quarter-wave per entry computes
+// A group per 16 x 16 tile, piece and chunk of ROWS coil rows; the tile and its halo are
+// staged in LDS with the coil row fastest, rotated: region = grid * P_0 * P_1; ROWS lanes
+// per entry compute
 //   y = F * sum_i w0[i] sum_j w1[j] region[l0 + i][l1 + j]
-// with real w0, w1; exception entries use complex weights t_d * conj(P_d).
+// with real w0, w1; exception entries use the table's complex weights and the cells
+// rotated back.
+// ROWS: 16 from 9 coil rows on (the records are read once per 16 rows), else the smallest of
+// 8, 4, 2, 1 that holds them: fewer idle lanes, and 64 / ROWS entries share a wave.
+template <int ROWS>
+struct GatShape {
+  static constexpr int kPitch = ROWS > 1 ? ROWS + 1 : 1;  // float2 per staged cell (odd: stores spread over banks)
+  static constexpr int kThreads = ROWS == 16 ? 512 : 256;
+};
+
+template <int ROWS>
 __device__ __forceinline__ float2 sep_gat_real(const float (&w0)[6], const float (&w1)[6], const float2* L0, int J0,
                                                int J1, bool fixed6) {
+  constexpr int kPitch = GatShape<ROWS>::kPitch;
   if (fixed6) {
     // J = 6: all 36 taps are read before any is used (a scheduling barrier keeps the
     // sums behind the reads, so the LDS latency is paid once per entry)
@@ -1318,7 +1339,7 @@ __device__ __forceinline__ float2 sep_gat_real(const float (&w0)[6], const float
 #pragma unroll
     for (int j0 = 0; j0 < 6; ++j0)
 #pragma unroll
-      for (int j1 = 0; j1 < 6; ++j1) X[j0][j1] = L0[j0 * (kGatR1 * kGatPitch) + j1 * kGatPitch];
+      for (int j1 = 0; j1 < 6; ++j1) X[j0][j1] = L0[j0 * (kGatR1 * kPitch) + j1 * kPitch];
     __builtin_amdgcn_sched_barrier(0);
     float2 acc = make_float2(0.f, 0.f);
 #pragma unroll
@@ -1337,13 +1358,13 @@ __device__ __forceinline__ float2 sep_gat_real(const float (&w0)[6], const float
   float2 acc = make_float2(0.f, 0.f);
 #pragma unroll
   for (int j0 = 0; j0 < 6; ++j0) {
-    if (fixed6 || j0 < J0) {
-      const float2* L = L0 + j0 * (kGatR1 * kGatPitch);
+    if (j0 < J0) {
+      const float2* L = L0 + j0 * (kGatR1 * kPitch);
       float2 p = make_float2(0.f, 0.f);
 #pragma unroll
       for (int j1 = 0; j1 < 6; ++j1) {
-        if (fixed6 || j1 < J1) {
-          const float2 x = L[j1 * kGatPitch];
+        if (j1 < J1) {
+          const float2 x = L[j1 * kPitch];
           p.x = fmaf(w1[j1], x.x, p.x);
           p.y = fmaf(w1[j1], x.y, p.y);
         }
@@ -1355,30 +1376,33 @@ __device__ __forceinline__ float2 sep_gat_real(const float (&w0)[6], const float
   return acc;
 }
 
-__device__ __forceinline__ float2 sep_gat_complex(const SepX* x, const float2* L0, int J0, int J1) {
+// exception entry: the table's weights on the cells rotated back by conj(P_0 P_1)
+template <int ROWS>
+__device__ __forceinline__ float2 sep_gat_complex(const Geom<float>& g, float om0, float om1, const float2* L0,
+                                                  const float2* p0, const float2* p1) {
+  constexpr int kPitch = GatShape<ROWS>::kPitch;
   float2 acc = make_float2(0.f, 0.f);
-  for (int j0 = 0; j0 < J0; ++j0) {
-    const float2* L = L0 + j0 * (kGatR1 * kGatPitch);
+  for (int j0 = 0; j0 < g.J[0]; ++j0) {
+    const float2* L = L0 + j0 * (kGatR1 * kPitch);
     float2 p = make_float2(0.f, 0.f);
-    for (int j1 = 0; j1 < J1; ++j1) cmac(p, x->w1[j1], L[j1 * kGatPitch]);
-    cmac(acc, x->w0[j0], p);
+    for (int j1 = 0; j1 < g.J[1]; ++j1) cmac(p, sep_tap_weight(g, 1, om1, j1), cmul_conj(L[j1 * kPitch], p1[j1]));
+    cmac(acc, sep_tap_weight(g, 0, om0, j0), cmul_conj(p, p0[j0]));
   }
   return acc;
 }
 
-template <int JF>
-__global__ void __launch_bounds__(kGatThreads)
-    gather_sep_kernel(const Geom<float> g, const TileGeom tg, const SepGeom sg, const float2* __restrict__ grid,
-                      const int* ws, float2* kdata, int nchunk) {
-  __shared__ __attribute__((aligned(16))) float2 region[kGatCells * kGatPitch];
-  __shared__ float2 cph[kGatCells];
+// One work item: tile piece wi, chunk of ROWS coil rows; `plan`, `omega` and rows
+// [rowbase, rowbase + nrows) belong to one trajectory.  `region`: kGatCells * kPitch cells,
+// `ph`: the phases P_0 of the region's rows and P_1 of its columns.
+template <int JF, int ROWS>
+__device__ __forceinline__ void gather_sep_item(const Geom<float>& g, const TileGeom& tg, const SepGeom& sg,
+                                                const float2* __restrict__ grid, const float* __restrict__ omega,
+                                                const int* plan, float2* kdata, int64_t rowbase, int64_t nrows,
+                                                int64_t wi, int chunk, float2* region, float2* ph) {
+  constexpr int kPitch = GatShape<ROWS>::kPitch, kThreads = GatShape<ROWS>::kThreads;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int half = lane / kGatRows, row = lane % kGatRows;  // entry slot, coil row
-  const int* plan = ws;
-  const int64_t item = xcd_work_item(blockIdx.x, kXcdTiles * nchunk);
-  const int64_t wi = item / nchunk;
-  const int chunk = (int)(item - wi * nchunk);
+  const int slot = lane / ROWS, row = lane % ROWS;  // entry slot, coil row
   if (wi >= plan[tg.o_nwork]) return;
   const int t = plan[tg.o_work + wi];
   const int split = (int)(wi - plan[tg.o_wstart + t]);
@@ -1386,58 +1410,87 @@ __global__ void __launch_bounds__(kGatThreads)
   const int i0 = split * tg.target;
   const int i1 = min(i0 + tg.target, V);
   if (i0 >= i1) return;
-  const int64_t nrows = g.B * g.C;
-  const int64_t rbase = (int64_t)chunk * kGatRows;
-  const int ncc = (int)((rbase + kGatRows < nrows ? rbase + kGatRows : nrows) - rbase);
+  const int64_t rbase = (int64_t)chunk * ROWS;
+  const int ncc = (int)((rbase + ROWS < nrows ? rbase + ROWS : nrows) - rbase);
+  const int64_t row0 = rowbase + rbase;
   const int o0 = ((t / tg.bstride[0]) % tg.nb[0]) * kGatT0;
   const int o1 = ((t / tg.bstride[1]) % tg.nb[1]) * kGatT1;
-  const int nm1[2] = {plan[sg.o_nm1], plan[sg.o_nm1 + 1]};
-  const float2* P0 = reinterpret_cast<const float2*>(plan + sg.o_ptab[0]);
-  const float2* P1 = reinterpret_cast<const float2*>(plan + sg.o_ptab[1]);
+  float2* const p0 = ph;
+  float2* const p1 = ph + kGatR0;
+  const auto phases = [&](int i) {  // i-th of the kGatR0 + kGatR1 phases
+    const int d = i < kGatR0 ? 0 : 1;
+    const int nm1 = plan[sg.o_nm1 + d];
+    const double2* P = reinterpret_cast<const double2*>(plan + sg.o_ptab[d]);
+    ph[i] = sep_cell_phase(P, g.K[d], nm1, d == 0 ? o0 + i : o1 + i - kGatR0);
+  };
 
-  // Stage: thread (coil row sr, region column sl1) of the first 16 x 21 threads loads
-  // that column's 21 region rows (consecutive threads read consecutive grid columns;
-  // the row index steps by one and wraps), while the other threads compute the cell
-  // phases; then every loaded value is stored rotated.
-  constexpr int kStageThreads = kGatRows * kGatR1;  // 336
-  static_assert(kStageThreads < kGatThreads, "spare threads compute the phases");
-  const int sr = (int)threadIdx.x / kGatR1, sl1 = (int)threadIdx.x - sr * kGatR1;
-  float2 v[kGatR0];
-  if ((int)threadIdx.x < kStageThreads) {
-    int k1 = o1 + sl1;
-    while (k1 >= g.K[1]) k1 -= g.K[1];
-    int k0 = o0;  // a tile origin lies inside the grid
-    const bool live = sr < ncc;
-    const float2* src = grid + (rbase + (live ? sr : 0)) * g.G + k1;
+  if constexpr (ROWS == 16) {
+    // Stage: thread (coil row sr, region column sl1) of the first 16 x 21 threads loads
+    // that column's 21 region rows (consecutive threads read consecutive grid columns;
+    // the row index steps by one and wraps), while the other threads look up the phases;
+    // then every loaded value is stored rotated.
+    constexpr int kStageThreads = ROWS * kGatR1;  // 336
+    static_assert(kStageThreads + kGatR0 + kGatR1 <= kThreads, "spare threads look up the phases");
+    const int sr = (int)threadIdx.x / kGatR1, sl1 = (int)threadIdx.x - sr * kGatR1;
+    float2 v[kGatR0];
+    if ((int)threadIdx.x < kStageThreads) {
+      int k1 = o1 + sl1;
+      while (k1 >= g.K[1]) k1 -= g.K[1];
+      int k0 = o0;  // a tile origin lies inside the grid
+      const bool live = sr < ncc;
+      const float2* src = grid + (row0 + (live ? sr : 0)) * g.G + k1;
 #pragma unroll
-    for (int l0 = 0; l0 < kGatR0; ++l0) {
-      v[l0] = live ? src[(int64_t)k0 * g.stride[0]] : make_float2(0.f, 0.f);
-      k0 = k0 + 1 == g.K[0] ? 0 : k0 + 1;
+      for (int l0 = 0; l0 < kGatR0; ++l0) {
+        v[l0] = live ? src[(int64_t)k0 * g.stride[0]] : make_float2(0.f, 0.f);
+        k0 = k0 + 1 == g.K[0] ? 0 : k0 + 1;
+      }
+    } else if ((int)threadIdx.x - kStageThreads < kGatR0 + kGatR1) {
+      phases((int)threadIdx.x - kStageThreads);
+    }
+    lds_barrier();
+    if ((int)threadIdx.x < kStageThreads) {
+      const float2 pc = p1[sl1];
+#pragma unroll
+      for (int l0 = 0; l0 < kGatR0; ++l0)
+        region[(l0 * kGatR1 + sl1) * kPitch + sr] = cmul(v[l0], cmul(p0[l0], pc));
     }
   } else {
-    for (int c = (int)threadIdx.x - kStageThreads; c < kGatCells; c += kGatThreads - kStageThreads) {
-      const int l0 = c / kGatR1, l1 = c - l0 * kGatR1;
-      cph[c] = cmul(sep_cell_phase(P0, g.K[0], nm1[0], o0 + l0), sep_cell_phase(P1, g.K[1], nm1[1], o1 + l1));
-    }
-  }
-  lds_barrier();
-  if ((int)threadIdx.x < kStageThreads) {
+    // cell by cell: all of a thread's loads in flight before their stores
+    constexpr int kN = ROWS * kGatCells, kU = (kN + kThreads - 1) / kThreads;
+    float2 v[kU];
+    const auto place = [&](int i, int& r, int& l0, int& l1) {
+      r = i / kGatCells;
+      const int c = i - r * kGatCells;
+      l0 = c / kGatR1;
+      l1 = c - l0 * kGatR1;
+    };
 #pragma unroll
-    for (int l0 = 0; l0 < kGatR0; ++l0) {
-      const int cell = l0 * kGatR1 + sl1;
-      region[cell * kGatPitch + sr] = cmul(v[l0], cph[cell]);
+    for (int u = 0; u < kU; ++u) {
+      int r, l0, l1;
+      place(min((int)threadIdx.x + u * kThreads, kN - 1), r, l0, l1);
+      int k0 = o0 + l0, k1 = o1 + l1;
+      while (k0 >= g.K[0]) k0 -= g.K[0];
+      while (k1 >= g.K[1]) k1 -= g.K[1];
+      v[u] = grid[(row0 + min(r, ncc - 1)) * g.G + (int64_t)k0 * g.stride[0] + k1];
+    }
+    if ((int)threadIdx.x < kGatR0 + kGatR1) phases((int)threadIdx.x);
+    lds_barrier();
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      int r, l0, l1;
+      const int i = (int)threadIdx.x + u * kThreads;
+      place(min(i, kN - 1), r, l0, l1);
+      if (i < kN) region[(l0 * kGatR1 + l1) * kPitch + r] = cmul(v[u], cmul(p0[l0], p1[l1]));
     }
   }
   __syncthreads();
 
   // Records one entry ahead, alternating between two register sets (unconditional,
-  // clamped loads).  Half-wave h of wave w takes entries i0 + 4w + h, stepping by 32.
-  const float4* recs = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(ws) + tg.o_rec_bytes) +
+  // clamped loads).  Slot h of wave w takes entries i0 + kPer w + h, stepping by kStep.
+  constexpr int kPer = 64 / ROWS, kStep = kPer * (kThreads / 64);
+  const float4* recs = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(plan) + tg.o_rec_bytes) +
                        (int64_t)plan[tg.o_start + t] * 4;
-  const SepX* xrecs = reinterpret_cast<const SepX*>(reinterpret_cast<const char*>(ws) + tg.o_rec_bytes +
-                                                    tg.maxent * (int64_t)sizeof(SepRec));
   const int J0 = g.J[0], J1 = g.J[1];
-  constexpr int kStep = kGatPerWave * (kGatThreads / 64);
   float4 ra[4], rb[4];
   auto load_rec = [&](float4 (&r)[4], int e) {
     const int ec = e < i1 ? e : i1 - 1;
@@ -1447,23 +1500,24 @@ __global__ void __launch_bounds__(kGatThreads)
   auto finish = [&](const float4 (&r)[4], int e) {
     if (e < i1) {
       const int me = __float_as_int(r[0].x), rc = __float_as_int(r[0].y);
+      const int m = me & 0x7fffffff;
       const int l0 = (rc & 255) - 8, l1 = ((rc >> 8) & 255) - 8;
       const float2 F = make_float2(r[0].z, r[0].w);
-      const float2* L0 = region + (l0 * kGatR1 + l1) * kGatPitch + row;
+      const float2* L0 = region + (l0 * kGatR1 + l1) * kPitch + row;
       float2 acc;
       if (me >= 0) {
         const float w0[6] = {r[1].x, r[1].y, r[1].z, r[1].w, r[2].x, r[2].y};
         const float w1[6] = {r[2].z, r[2].w, r[3].x, r[3].y, r[3].z, r[3].w};
-        acc = sep_gat_real(w0, w1, L0, J0, J1, JF == 6);
+        acc = sep_gat_real<ROWS>(w0, w1, L0, J0, J1, JF == 6);
       } else {
-        acc = sep_gat_complex(xrecs + (e + (int64_t)plan[tg.o_start + t]), L0, J0, J1);
+        acc = sep_gat_complex<ROWS>(g, omega[m], omega[g.M + m], L0, p0 + l0, p1 + l1);
       }
-      if (row < ncc) kdata[(rbase + row) * g.M + (me & 0x7fffffff)] = cmul(acc, F);
+      if (row < ncc) kdata[(row0 + row) * g.M + m] = cmul(acc, F);
     }
   };
-  load_rec(ra, i0 + kGatPerWave * wave + half);
-  for (int eb = i0 + kGatPerWave * wave; eb < i1; eb += 2 * kStep) {
-    const int e = eb + half;
+  load_rec(ra, i0 + kPer * wave + slot);
+  for (int eb = i0 + kPer * wave; eb < i1; eb += 2 * kStep) {
+    const int e = eb + slot;
     load_rec(rb, e + kStep);
     finish(ra, e);
     load_rec(ra, e + 2 * kStep);
@@ -1471,269 +1525,434 @@ __global__ void __launch_bounds__(kGatThreads)
   }
 }
 
-// ---- adjoint spread --------------------------------------------------------------------
-// A group per 16 x 16 tile, split and chunk of 32 coil rows; half-wave h of wave w owns
-// tile row 2w + h of its coil row in registers.  In the rotated frame: the staged data
-// are s = kdata * F, a tap adds s * w0[i] * w1[j] with real weights, and the flush
-// multiplies each cell by conj(P_0 P_1).  Exception entries have zero real weights
-// here; after the flush the group adds them with their complex weights conj(t_d)
-// (looked up from omega) and atomics.
-struct SepLds {
-  float w0r[6];  // R_0 of taps 0..5 (zero for exception entries)
-  float w1r[6];  // R_1
-  int r0, c0, pad[2];
-};
-static_assert(sizeof(SepLds) == 64, "staged record is 64 bytes");
-
-// Two staged entries a, b of one footprint column group at once (b may be the zero
-// dummy entry): ja / jb = the lane's tap row of each (any value; rows outside 0..J0-1
-// add nothing).  Branch-free, so the LDS reads of both entries are in flight together;
-// the adds into each accumulator keep the order a then b.
-template <int C0>
-__device__ __forceinline__ void sep_entry2(float2 (&acc)[kRegT1], const SepLds* ra, const SepLds* rb,
-                                           const float2 sa, const float2 sb, int ja, int jb, unsigned J0) {
-  float w1a[6], w1b[6];
-#pragma unroll
-  for (int j = 0; j < 6; ++j) {
-    w1a[j] = ra->w1r[j];
-    w1b[j] = rb->w1r[j];
-  }
-  const float wa = ra->w0r[min(max(ja, 0), 5)], wb = rb->w0r[min(max(jb, 0), 5)];
-  const bool va = (unsigned)ja < J0, vb = (unsigned)jb < J0;
-  const float2 ua = va ? make_float2(sa.x * wa, sa.y * wa) : make_float2(0.f, 0.f);
-  const float2 ub = vb ? make_float2(sb.x * wb, sb.y * wb) : make_float2(0.f, 0.f);
-#pragma unroll
-  for (int j = 0; j < 6; ++j) {
-    if (C0 + j >= 0 && C0 + j < kRegT1) {
-      acc[C0 + j].x = fmaf(ua.x, w1a[j], acc[C0 + j].x);
-      acc[C0 + j].y = fmaf(ua.y, w1a[j], acc[C0 + j].y);
-      acc[C0 + j].x = fmaf(ub.x, w1b[j], acc[C0 + j].x);
-      acc[C0 + j].y = fmaf(ub.y, w1b[j], acc[C0 + j].y);
-    }
-  }
+template <int JF, int ROWS>
+__global__ void __launch_bounds__(GatShape<ROWS>::kThreads)
+    gather_sep_kernel(const Geom<float> g, const TileGeom tg, const SepGeom sg, const float2* __restrict__ grid,
+                      const float* __restrict__ omega, const int* ws, float2* kdata, int nchunk) {
+  __shared__ __attribute__((aligned(16))) float2 region[kGatCells * GatShape<ROWS>::kPitch];
+  __shared__ float2 ph[kGatR0 + kGatR1];
+  const int64_t b = blockIdx.y;  // trajectory
+  const int64_t item = xcd_work_item(blockIdx.x, kXcdTiles * nchunk);
+  const int64_t wi = item / nchunk;
+  gather_sep_item<JF, ROWS>(g, tg, sg, grid, omega + b * 2 * g.M, ws + b * tg.plan_stride, kdata,
+                            g.batched ? b * g.C : 0, g.batched ? g.C : g.B * g.C, wi, (int)(item - wi * nchunk), region,
+                            ph);
 }
 
-__global__ void __launch_bounds__(kRegThreads) __attribute__((amdgpu_waves_per_eu(6)))
-    spread_sep_kernel(const Geom<float> g, const TileGeom tg, const SepGeom sg, const float2* __restrict__ kdata,
-                      const float* __restrict__ omega, const int* __restrict__ ws, float2* __restrict__ grid,
-                      int nchunk) {
-  // two staging buffers (batch k in buffer k & 1: one barrier per batch), each with a
-  // zero dummy entry kRegBatch; buffer 0 is also the flush's transposition space
-  __shared__ __attribute__((aligned(16))) float2 vals[2][(kRegBatch + 1) * kRegPitch];
-  __shared__ __attribute__((aligned(16))) SepLds brec[2][kRegBatch + 1];
-  __shared__ float2 rph[kRegT0], cphs[kRegT1];  // conj(P_0) of the tile rows, conj(P_1) of its columns
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  const int coil = lane & (kRegCoils - 1), hh = lane / kRegCoils;
+// ---- adjoint spread --------------------------------------------------------------------
+// On the matrix cores: in the rotated frame every tap of an entry adds s * w0[i] * w1[j]
+// with real w0, w1 (s = kdata * F), so a tile's sum over its entries is a matrix product
+// with the entries as the inner dimension.  A wave takes four entries of a 16 x 16 tile per
+// 16x16x4 float32 MFMA; their weights and data pass through its own part of LDS, without
+// work-group barriers.  A tile (or a piece of its entries) belongs to one wave, or, where
+// tiles are dense, to the four waves of a group, which split its entries and add their sums
+// through LDS at the end: a tile's entries are a serial chain, and cutting it into more
+// pieces would cost atomics (about 160 G lanes a second: with 128-entry pieces nearly every
+// tile of a 434 x 362 grid with 130 000 entries and 39 rows was split, 153 us).
+//   rows form (G = 8, 16 coil rows): per tile row r and 8 coil rows,  D_r[component][column]
+//     += s[component][entry] * (w0[entry][r] w1[entry][column]); the 16 components are the
+//     real and imaginary parts of the 8 rows, and tile rows that none of the four entries
+//     reaches are skipped (neighbouring samples of a trajectory share most rows);
+//   outer form (G = 1, 2, 4 coil rows): per row and component, D[row][column] +=
+//     (w0[entry][row] s[entry]) * w1[entry][column].
+// Every cell of the tile has one owner, so nothing is added atomically except the pieces of
+// split tiles.  The flush multiplies each cell by conj(P_0 P_1).
+// Entries with complex weights, and entries whose data are not finite (0 * inf would reach
+// the whole tile), are left out of the products and added with atomics after the flush,
+// tap by tap over their own footprint.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 
-  const int* plan = ws;
-  const int64_t wi = blockIdx.x / nchunk;
-  const int chunk = (int)(blockIdx.x - wi * nchunk);
+constexpr int kMmBatch = 32;   // entries staged at once by a wave
+constexpr int kMmWaves = 4;    // waves per work-group
+constexpr int kMmWPitch = 20;  // floats per staged row of 16 weights (+4: spreads the banks, takes what falls outside)
+constexpr int kMmExc = 32;     // entries left to the atomic pass that a wave remembers
+// rows per chunk of a form, and waves per SIMD of its kernel
+__host__ __device__ constexpr int mm_rows(int G) { return G; }
+constexpr int mm_waves(int G) { return G >= 8 ? 2 : G > 2 ? 3 : 4; }
+// floats per staged entry's data (two components a row; +2 spreads the banks)
+constexpr int mm_spitch(int G) { return 2 * G + 2; }
+
+// Dense tiles add hundreds of entries to a cell, and one float32 chain over them was the
+// spread's largest error (8 rows, 256^2: image off by 1.8e-7; 64-bit integer sums: 1.6e-7).
+// So each batch's 32 entries have a chain of their own, and the batches are added up outside
+// the matrix cores: in double for one or two rows, in float32 for more (1.6e-7 again).  16
+// rows leave no registers for it; with 12 rows one chain is as good as the integer sums
+// (1.1e-7 both).
+__host__ __device__ constexpr bool mm_two_level(int G) { return G <= 8; }
+template <bool Double>
+struct MmSum {
+  typedef f32x4 vec;
+  typedef float one;
+};
+template <>
+struct MmSum<true> {
+  typedef f64x4 vec;
+  typedef double one;
+};
+
+template <int G>
+struct __attribute__((aligned(16))) MmLds {  // one wave's staging
+  float w0[kMmBatch * kMmWPitch];  // weights of the tile's rows (zero outside the footprint)
+  float w1[kMmBatch * kMmWPitch];  // weights of the tile's columns
+  float s[kMmBatch * mm_spitch(G)];
+  int exc[kMmExc];
+};
+
+// a tile of more than `target` entries is cut into pieces of `target`, listed first
+__host__ __device__ inline int mm_splits(int v, int target) { return v <= target ? 1 : (v + target - 1) / target; }
+
+// LDS writes of this wave's lanes are visible to its other lanes after this
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+
+// a b with nearly one rounding a component (the rounding of each second product is added back)
+__device__ __forceinline__ float2 cmul_once(float2 a, float2 b) {
+  const float p = a.y * b.y, q = a.y * b.x;
+  return make_float2(fmaf(a.x, b.x, -p) - fmaf(a.y, b.y, -p), fmaf(a.x, b.y, q) + fmaf(a.y, b.x, -q));
+}
+
+// One work item: tile piece wi, chunk of coil rows, for one wave (ks = 1) or the whole group
+// (ks = kMmWaves, this wave its part `part`); `plan`, `omega` and rows [rowbase, rowbase +
+// nrows) belong to one trajectory.
+template <int G>
+__device__ __forceinline__ void spread_sep_item(const Geom<float>& g, const TileGeom& tg, const SepGeom& sg,
+                                                const float2* __restrict__ kdata, const float* __restrict__ omega,
+                                                const int* __restrict__ plan, float2* __restrict__ grid,
+                                                int64_t rowbase, int64_t nrows, int64_t wi, int chunk, int ks, int part,
+                                                MmLds<G>* group_lds, MmLds<G>& lds) {
+  constexpr int kRows = mm_rows(G), kSP = mm_spitch(G);
+  constexpr int kGroups = G >= 8 ? G / 8 : 0;  // rows form: 8 coil rows each
+  constexpr int kLoads = kRows > 1 ? kRows / 2 : 1;  // rows staged by a half-wave
+  const int lane = threadIdx.x & 63;
+  const int n16 = lane & 15, k4 = lane >> 4;  // matrix operands: outer index, inner index (entry)
   if (wi >= plan[tg.o_nwork]) return;
   const int t = plan[tg.o_work + wi];
   const int split = (int)(wi - plan[tg.o_wstart + t]);
-  const int64_t nrows = g.B * g.C;
-  const int64_t rbase = (int64_t)chunk * kRegCoils;
-  const int ncc = (int)((rbase + kRegCoils < nrows ? rbase + kRegCoils : nrows) - rbase);
+  const int64_t rbase = (int64_t)chunk * kRows;
+  const int ncc = (int)((rbase + kRows < nrows ? rbase + kRows : nrows) - rbase);
+  const int64_t row0 = rowbase + rbase;
   const int o0 = ((t / tg.bstride[0]) % tg.nb[0]) * kRegT0;
   const int o1 = ((t / tg.bstride[1]) % tg.nb[1]) * kRegT1;
   const int cstart = plan[tg.o_start + t];
   const int V = plan[tg.o_start + t + 1] - cstart;
-  const int nsplit = reg_splits(V);
-  const int i0 = nsplit > 1 ? split * kRegHotTarget : 0;
-  const int i1 = nsplit > 1 ? min(i0 + kRegHotTarget, V) : V;
+  const int nsplit = mm_splits(V, tg.target);
+  int i0 = nsplit > 1 ? split * tg.target : 0;
+  int i1 = nsplit > 1 ? min(i0 + tg.target, V) : V;
+  if (ks > 1) {  // this wave's batches
+    const int nb = (i1 - i0 + kMmBatch - 1) / kMmBatch;
+    const int b0 = i0 + (nb * part / kMmWaves) * kMmBatch, b1 = i0 + (nb * (part + 1) / kMmWaves) * kMmBatch;
+    i0 = min(b0, i1);
+    i1 = min(b1, i1);
+  }
+  const SepRec* recs = reinterpret_cast<const SepRec*>(reinterpret_cast<const char*>(plan) + tg.o_rec_bytes);
   const int* perm = plan + tg.o_perm + cstart;
-  const SepRec* recs = reinterpret_cast<const SepRec*>(reinterpret_cast<const char*>(ws) + tg.o_rec_bytes) + cstart;
+  const int odd0 = plan[sg.o_nm1] & 1, odd1 = plan[sg.o_nm1 + 1] & 1;
+  // a footprint's first cell relative to the tile, below 0 where it starts before the tile
+  // or past the grid's end
+  const auto rel = [](int cell, int o, int T, int K) { return cell - o < T ? cell - o : cell - o - K; };
   const int J0 = g.J[0];
-  const int wrow = wave * kRegRowsPerWave;
 
-  // cells past the grid's end are never flushed: any phase will do there
-  if (threadIdx.x < kRegT0) {
-    const float2 p = reinterpret_cast<const float2*>(plan + sg.o_ptab[0])[min(o0 + (int)threadIdx.x, g.K[0] - 1)];
-    rph[threadIdx.x] = make_float2(p.x, -p.y);
-  } else if (threadIdx.x < kRegT0 + kRegT1) {
-    const float2 p =
-        reinterpret_cast<const float2*>(plan + sg.o_ptab[1])[min(o1 + (int)threadIdx.x - kRegT0, g.K[1] - 1)];
-    cphs[threadIdx.x - kRegT0] = make_float2(p.x, -p.y);
+  // phases of the tile's rows (lane n16: row n16) and of this lane's column, for the flush
+  const double2 pr16 = reinterpret_cast<const double2*>(plan + sg.o_ptab[0])[min(o0 + n16, g.K[0] - 1)];
+  const double2 pc = reinterpret_cast<const double2*>(plan + sg.o_ptab[1])[min(o1 + n16, g.K[1] - 1)];
+
+  constexpr int kAcc = kGroups > 0 ? kGroups * kRegT0 : 2 * kRows;
+  f32x4 acc[kAcc];
+#pragma unroll
+  for (int c = 0; c < kAcc; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // Sums of the batches' sums
+  typedef typename MmSum<(G <= 2)>::vec Sum;
+  typedef typename MmSum<(G <= 2)>::one Sum1;
+  constexpr bool kTwo = mm_two_level(G);
+  Sum tot[kTwo ? kAcc : 1];
+  if constexpr (kTwo) {
+#pragma unroll
+    for (int c = 0; c < kAcc; ++c) tot[c] = Sum{0, 0, 0, 0};
   }
-  for (int i = threadIdx.x; i < 2 * kRegPitch; i += kRegThreads)
-    vals[i / kRegPitch][kRegBatch * kRegPitch + i % kRegPitch] = make_float2(0.f, 0.f);
-  if (threadIdx.x < 2 * 16) reinterpret_cast<int*>(&brec[threadIdx.x / 16][kRegBatch])[threadIdx.x % 16] = 0;
-  lds_barrier();  // the flush reads them even when the tile has no entries
 
-  float2 acc[kRegT1];
-#pragma unroll
-  for (int c = 0; c < kRegT1; ++c) acc[c] = make_float2(0.f, 0.f);
-
-  // Software pipeline: the next batch's data (with its entry's factor F) and records
-  // are loaded into registers while a batch is processed, and the sample indices one
-  // batch further.  Thread (wave w, lane e) stages coil rows
-  // 4w .. 4w+3 of entry e; threads of waves 0..3 load one float4 of the 64-byte records.
-  constexpr int kPer = kRegCoils / kRegWaves;
-  float4 prec = make_float4(0.f, 0.f, 0.f, 0.f);
-  float2 pv[kPer];
-  float2 pF = make_float2(0.f, 0.f);
-  int pme = 0;
-  bool anyexc = false;  // an exception entry was staged (the same in every wave)
-  auto prefetch = [&](int b, int me) {
-    const int n = min(kRegBatch, i1 - b);
-    if ((int)threadIdx.x < n * 4) prec = reinterpret_cast<const float4*>(recs + b)[threadIdx.x];
-    pme = lane < n ? me : 0;
-    pF = lane < n ? recs[b + lane].F : make_float2(0.f, 0.f);
-    const int mb = me & 0x7fffffff;
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-      const int row = wave * kPer + q;
-      pv[q] = make_float2(0.f, 0.f);
-      if (lane < n && row < ncc) pv[q] = kdata[(rbase + row) * g.M + mb];
-    }
-  };
+  // Staging: lane (entry e, half h) holds the sample's header, its weights along dimension h
+  // and its data for the half's rows.  The sample indices are loaded two batches ahead, the
+  // records and the data one, so that all are in flight during a walk.
+  const int e = lane & (kMmBatch - 1), h = lane / kMmBatch;
   int mnext = 0;
-  if (i0 < i1) {
-    const int m0 = lane < min(kRegBatch, i1 - i0) ? perm[i0 + lane] : 0;
-    prefetch(i0, m0);
-    const int b1 = i0 + kRegBatch;
-    if (b1 < i1 && lane < min(kRegBatch, i1 - b1)) mnext = perm[b1 + lane];
-  }
-  int buf = 0;
-  for (int base = i0; base < i1; base += kRegBatch, buf ^= 1) {
-    const int nb = min(kRegBatch, i1 - base);
-    float2* const vb = vals[buf];
-    SepLds* const bb = brec[buf];
+  float4 head = make_float4(0.f, 0.f, 0.f, 0.f);  // me, rc, F
+  float2 wv[3], kd[kLoads];
+  const auto stage_row = [&](int c) { return kRows > 1 ? h * kLoads + c : 0; };
+  int at = 0;  // position of the entry that mnext belongs to
+  const auto load_index = [&](int base) {
+    at = min(base + e, i1 - 1);
+    mnext = perm[at];
+  };
+  const auto load_sample = [&] {
+    const int m = mnext;
+    const float2* r = reinterpret_cast<const float2*>(recs + (tg.rec_entry ? cstart + at : m));
+    head = *reinterpret_cast<const float4*>(r);
 #pragma unroll
-    for (int q = 0; q < kPer; ++q) vb[lane * kRegPitch + wave * kPer + q] = cmul(pv[q], pF);
-    anyexc = anyexc || __ballot(pme < 0) != 0;
-    // records: float4 q of entry e holds (me, rc, F) for q = 0, then w0[0..3],
-    // w0[4..5] w1[0..1], w1[2..5]: the latter three are the first 48 bytes of SepLds
-    if ((int)threadIdx.x < nb * 4) {
-      const int e = threadIdx.x >> 2, q = threadIdx.x & 3;
-      if (q == 0) {
-        const int rc = __float_as_int(prec.y);
-        bb[e].r0 = (rc & 255) - 8;
-        bb[e].c0 = ((rc >> 8) & 255) - 8;
-      } else {
-        reinterpret_cast<float4*>(bb + e)[q - 1] = prec;
+    for (int q = 0; q < 3; ++q) wv[q] = r[2 + 3 * h + q];
+#pragma unroll
+    for (int c = 0; c < kLoads; ++c) kd[c] = kdata[(row0 + min(stage_row(c), ncc - 1)) * g.M + m];
+  };
+  int nexc = 0;  // entries left to the atomic pass
+  // operands of entries 4 k .. 4 k + 3: rows form: the tile's 16 row weights, outer form: the
+  // weight of row n16; the weight of column n16; the data
+  struct Operands {
+    f32x4 w0[kGroups > 0 ? 4 : 1];
+    float w1, a[kGroups > 0 ? kGroups : 2 * kRows];
+  };
+  const auto read_ops = [&](int k) {
+    Operands o;
+    const int en = 4 * k + k4;
+    o.w1 = lds.w1[en * kMmWPitch + n16];
+    if constexpr (kGroups > 0) {
+#pragma unroll
+      for (int u = 0; u < kGroups; ++u) o.a[u] = lds.s[en * kSP + 16 * u + n16];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) o.w0[q] = *reinterpret_cast<const f32x4*>(&lds.w0[en * kMmWPitch + 4 * q]);
+    } else {
+      o.w0[0][0] = lds.w0[en * kMmWPitch + n16];
+#pragma unroll
+      for (int c = 0; c < kRows; ++c) {
+        const float2 sv = *reinterpret_cast<const float2*>(&lds.s[en * kSP + 2 * c]);
+        o.a[2 * c] = sv.x;
+        o.a[2 * c + 1] = sv.y;
       }
     }
-    // The other buffer was last read in the previous batch's walk, which every wave
-    // finished before this barrier; global loads stay in flight across it.
-    lds_barrier();
-    const int r0l = lane < nb ? bb[lane].r0 : 1000, c0l = lane < nb ? bb[lane].c0 : 1000;
-    const int b1 = base + kRegBatch;
-    if (b1 < i1) {
-      prefetch(b1, mnext);
-      const int b2 = b1 + kRegBatch;
-      mnext = (b2 < i1 && lane < min(kRegBatch, i1 - b2)) ? perm[b2 + lane] : 0;
+    return o;
+  };
+  if (i0 < i1) {  // loads past the end read the last entry again
+    load_index(i0);
+    load_sample();
+    load_index(i0 + kMmBatch);
+  }
+  for (int base = i0; base < i1; base += kMmBatch) {
+    const bool live = base + e < i1;
+    const int me = __float_as_int(head.x);
+    const int b0 = me & 0x7fffffff, b1 = __float_as_int(head.y);
+    const int r0 = rel(b0, o0, kRegT0, g.K[0]), c0 = rel(b1, o1, kRegT1, g.K[1]);
+    // one grid period before the wrapped cell: F times (-1)^(N - 1)
+    const bool flip = ((b0 - o0 >= kRegT0 ? odd0 : 0) ^ (b1 - o1 >= kRegT1 ? odd1 : 0)) != 0;
+    const float2 F = flip ? make_float2(-head.z, -head.w) : make_float2(head.z, head.w);
+    const bool use = live && me >= 0;  // others get zero weights
+    float2 s[kLoads];
+    float probe = 0.f;  // NaN once any value is not finite
+#pragma unroll
+    for (int c = 0; c < kLoads; ++c) {
+      s[c] = cmul_once(kd[c], F);
+      probe = fmaf(s[c].x, 0.f, probe);
+      probe = fmaf(s[c].y, 0.f, probe);
     }
-    const int jal = wrow - r0l;
-    const unsigned long long hits = __ballot(jal + kRegRowsPerWave > 0 && jal < J0);
-#define TKBN_SEP_GROUP(C0)                                                                        \
-  {                                                                                               \
-    unsigned long long mk = __ballot(c0l == (C0)) & hits;                                         \
-    while (mk) {                                                                                  \
-      const int ca = __ffsll(mk) - 1;                                                             \
-      mk &= mk - 1;                                                                               \
-      int cb = kRegBatch;                                                                         \
-      if (mk) {                                                                                   \
-        cb = __ffsll(mk) - 1;                                                                     \
-        mk &= mk - 1;                                                                             \
-      }                                                                                           \
-      const int ja = wrow + hh - __builtin_amdgcn_readlane(r0l, ca);                              \
-      const int jb = wrow + hh - __builtin_amdgcn_readlane(r0l, cb & 63);                         \
-      sep_entry2<C0>(acc, bb + ca, bb + cb, vb[ca * kRegPitch + coil], vb[cb * kRegPitch + coil], \
-                     ja, jb, (unsigned)J0);                                                       \
-    }                                                                                             \
+    const bool finite = probe == 0.f;
+    const bool bad = live && (me < 0 || !finite);
+    const unsigned long long bb = __ballot(bad || !finite);
+    if (bb) {  // rare: zero what is not finite, remember the first kMmExc entries left out
+#pragma unroll
+      for (int c = 0; c < kLoads; ++c)
+        if (!(isfinite(s[c].x) && isfinite(s[c].y))) s[c] = make_float2(0.f, 0.f);
+      const unsigned long long bb = __ballot(bad);
+      const unsigned both = (unsigned)bb | (unsigned)(bb >> 32);
+      const int at = nexc + __popc(both & ((1u << e) - 1u));
+      if (h == 0 && ((both >> e) & 1u) && at < kMmExc) lds.exc[at] = base + e;
+      nexc += __popc(both);
+    }
+    {
+      // the row's zeros, then its six weights; what falls outside the tile goes to slot 16
+      float* w = (h == 0 ? lds.w0 : lds.w1) + e * kMmWPitch;
+      const int off = use ? (h == 0 ? r0 : c0) : 16;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) reinterpret_cast<float4*>(w)[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+      const float wj[6] = {wv[0].x, wv[0].y, wv[1].x, wv[1].y, wv[2].x, wv[2].y};
+#pragma unroll
+      for (int j = 0; j < 6; ++j) w[min((unsigned)(off + j), 16u)] = wj[j];
+    }
+#pragma unroll
+    for (int c = 0; c < kLoads; ++c)
+      if (kRows > 1 || h == 0) *reinterpret_cast<float2*>(&lds.s[e * kSP + 2 * stage_row(c)]) = s[c];
+    // tile rows that entries 4 k .. 4 k + 3 reach, in lane 4 k
+    unsigned mask = use ? ((((1u << J0) - 1u) << (r0 + 5)) >> 5) & 0xffffu : 0u;
+    mask |= (unsigned)__builtin_amdgcn_mov_dpp((int)mask, 0xb1, 0xf, 0xf, true);  // lane ^ 1
+    mask |= (unsigned)__builtin_amdgcn_mov_dpp((int)mask, 0x4e, 0xf, 0xf, true);  // lane ^ 2
+    wave_lds_sync();
+    load_sample();
+    load_index(base + 2 * kMmBatch);
+    // Four entries at a time; the operands of the next four are read from LDS (all of them,
+    // before the branches that skip rows) while this four's products run.
+    Operands op = read_ops(0);
+#pragma unroll
+    for (int k = 0; k < kMmBatch / 4; ++k) {
+      const unsigned mk = __builtin_amdgcn_readlane(mask, 4 * k);
+      Operands nxt = op;
+      if (k + 1 < kMmBatch / 4) nxt = read_ops(k + 1);
+      asm volatile("" ::: "memory");  // keeps the reads here
+      if constexpr (kGroups > 0) {
+#pragma unroll
+        for (int r = 0; r < kRegT0; ++r) {
+          if ((mk >> r) & 1u) {
+            const float w = op.w0[r / 4][r % 4] * op.w1;
+#pragma unroll
+            for (int u = 0; u < kGroups; ++u)
+              acc[u * kRegT0 + r] = __builtin_amdgcn_mfma_f32_16x16x4f32(op.a[u], w, acc[u * kRegT0 + r], 0, 0, 0);
+          }
+        }
+      } else if (mk != 0) {
+#pragma unroll
+        for (int c = 0; c < kRows; ++c) {
+          acc[2 * c] = __builtin_amdgcn_mfma_f32_16x16x4f32(op.w0[0][0] * op.a[2 * c], op.w1, acc[2 * c], 0, 0, 0);
+          acc[2 * c + 1] =
+              __builtin_amdgcn_mfma_f32_16x16x4f32(op.w0[0][0] * op.a[2 * c + 1], op.w1, acc[2 * c + 1], 0, 0, 0);
+        }
+      }
+      op = nxt;
+    }
+    wave_lds_sync();  // the next batch overwrites the staging
+    if constexpr (kTwo) {
+#pragma unroll
+      for (int c = 0; c < kAcc; ++c) {
+        tot[c] += __builtin_convertvector(acc[c], Sum);
+        acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
   }
-    TKBN_SEP_GROUP(-5) TKBN_SEP_GROUP(-4) TKBN_SEP_GROUP(-3) TKBN_SEP_GROUP(-2) TKBN_SEP_GROUP(-1)
-    TKBN_SEP_GROUP(0) TKBN_SEP_GROUP(1) TKBN_SEP_GROUP(2) TKBN_SEP_GROUP(3) TKBN_SEP_GROUP(4)
-    TKBN_SEP_GROUP(5) TKBN_SEP_GROUP(6) TKBN_SEP_GROUP(7) TKBN_SEP_GROUP(8) TKBN_SEP_GROUP(9)
-    TKBN_SEP_GROUP(10) TKBN_SEP_GROUP(11) TKBN_SEP_GROUP(12) TKBN_SEP_GROUP(13) TKBN_SEP_GROUP(14)
-    TKBN_SEP_GROUP(15)
-#undef TKBN_SEP_GROUP
-  }
-  lds_barrier();  // the flush reuses buffer 0
+  Sum(&sum)[kAcc] = [&]() -> Sum(&)[kAcc] {
+    if constexpr (kTwo) return tot;
+    else return acc;
+  }();
 
-  // Flush: every owned cell inside the grid is written (split tiles were zeroed first
-  // and add), rotated back by conj(P_0 P_1).  The rows go out through LDS in rounds of
-  // kRound tile rows so that each store instruction writes 16 consecutive cells (128 B)
-  // of every coil row; LDS-only barriers keep the stores in flight.
-  constexpr int kRound = 4;
-  constexpr int kRoundWaves = kRound / kRegRowsPerWave;
-  for (int round = 0; round < kRegT0 / kRound; ++round) {
-    if (wave / kRoundWaves == round) {
-      const int slot = (wave % kRoundWaves) * kRegRowsPerWave + hh;
-      const float2 pr = rph[kRound * round + slot];
+  const int exc = lane < kMmExc ? lds.exc[lane] : 0;  // (the staging is reused)
+
+  // A group's waves add their sums, in wave order: wave q collects the q-th kQ accumulators.
+  constexpr int kQ = kAcc / kMmWaves > 2 ? kAcc / kMmWaves : 2, kRounds = kAcc / kQ;
+  static_assert((kMmWaves - 1) * kQ * 64 * sizeof(Sum) <= kMmWaves * sizeof(MmLds<G>), "the sums fit the staging");
+  if (ks > 1) {
+    Sum* const sums = reinterpret_cast<Sum*>(group_lds);  // [wave, the collecting one left out][kQ][lane]
 #pragma unroll
-      for (int c = 0; c < kRegT1; ++c) vals[0][(slot * kRegT1 + c) * kRegPitch + coil] = cmul(acc[c], cmul(pr, cphs[c]));
+    for (int q = 0; q < kRounds; ++q) {
+      lds_barrier();  // the staging, or the last round's sums, are read
+      if (part != q) {
+        Sum* const mine = sums + (part - (part > q ? 1 : 0)) * (kQ * 64) + lane;
+#pragma unroll
+        for (int i = 0; i < kQ; ++i) mine[i * 64] = sum[q * kQ + i];
+      }
+      lds_barrier();
+      if (part == q) {
+#pragma unroll
+        for (int i = 0; i < kQ; ++i) {
+          Sum s = q == 0 ? sum[i] : sums[i * 64 + lane];
+#pragma unroll
+          for (int w = 1; w < kMmWaves; ++w) s += w == q ? sum[q * kQ + i] : sums[((w - (w > q ? 1 : 0)) * kQ + i) * 64 + lane];
+          sum[q * kQ + i] = s;
+        }
+      }
     }
-    lds_barrier();
+  }
+  const auto mine = [&](int a) { return ks == 1 || a / kQ == part; };  // accumulators this wave flushes
+
+  // Flush: lane n16 holds column n16 of the tile; every cell inside the grid is written
+  // (split tiles were zeroed first and add), 128 contiguous bytes of a row per 16 lanes.
+  const int k1 = o1 + n16;
+  const auto phase = [&](int r) {  // of this lane's cell in tile row r
+    return cmul(make_double2(__shfl(pr16.x, r, 64), __shfl(pr16.y, r, 64)), pc);
+  };
+  const auto put = [&](int row, int r, double2 p, Sum1 re, Sum1 im) {  // the rotated cell of tile row r
+    const int k0 = o0 + r;
+    if (row < ncc && k0 < g.K[0] && k1 < g.K[1]) {
+      const double2 vd = cmul_conj(make_double2((double)re, (double)im), p);
+      const float2 v = make_float2((float)vd.x, (float)vd.y);
+      float2* dst = grid + (row0 + row) * g.G + (int64_t)k0 * g.stride[0] + k1;
+      if (nsplit == 1) {
+        *dst = v;
+      } else {
+        unsafeAtomicAdd(&dst->x, v.x);
+        unsafeAtomicAdd(&dst->y, v.y);
+      }
+    }
+  };
+  if constexpr (kGroups > 0) {
 #pragma unroll
-    for (int q = 0; q < (kRound * kRegT1 * kRegCoils) / kRegThreads; ++q) {
-      const int e = threadIdx.x + q * kRegThreads;
-      const int c = e & (kRegT1 - 1), cl = (e / kRegT1) & (kRegCoils - 1), slot = e / (kRegT1 * kRegCoils);
-      const int k0 = o0 + kRound * round + slot, k1 = o1 + c;
-      if (cl < ncc && k0 < g.K[0] && k1 < g.K[1]) {
-        const float2 v = vals[0][(slot * kRegT1 + c) * kRegPitch + cl];
-        float2* dst = grid + (rbase + cl) * g.G + (int64_t)k0 * g.stride[0] + k1;
-        if (nsplit == 1) {
-          *dst = v;
-        } else {
+    for (int r = 0; r < kRegT0; ++r) {
+      const double2 p = phase(r);
+#pragma unroll
+      for (int u = 0; u < kGroups; ++u) {
+        if (!mine(u * kRegT0 + r)) continue;
+        const Sum a = sum[u * kRegT0 + r];
+        put(8 * u + 2 * k4, r, p, a[0], a[1]);
+        put(8 * u + 2 * k4 + 1, r, p, a[2], a[3]);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const double2 p = phase(4 * k4 + v);
+#pragma unroll
+      for (int c = 0; c < kRows; ++c)
+        if (mine(2 * c)) put(c, 4 * k4 + v, p, sum[2 * c][v], sum[2 * c + 1][v]);
+    }
+  }
+
+  // Entries left out of the products: lane (tap row i, coil row) adds
+  // kdata * conj(phase) * conj(t0[i] t1[j]) over the row's taps inside the tile.  The
+  // remembered ones, or (more than fit) a walk over all entries of the item.
+  // The tile's stores come first: they and the atomics meet in this XCD's L2 (a device-scope
+  // fence would write the whole L2 back).
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (ks > 1) __syncthreads();
+  if (nexc == 0) return;
+  const bool listed = nexc <= kMmExc;
+  const int n = listed ? nexc : i1 - i0;
+  for (int x = 0; x < n; ++x) {
+    const int ei = listed ? __shfl(exc, x, 64) : i0 + x;
+    const int m = perm[ei];
+    const SepRec& rec = recs[tg.rec_entry ? cstart + ei : m];
+    const int me = rec.me;
+    const int i = lane >> 3;
+    const int r = rel(me & 0x7fffffff, o0, kRegT0, g.K[0]) + i, c0 = rel(rec.rc, o1, kRegT1, g.K[1]);
+    if (i >= J0 || r < 0 || r >= kRegT0 || o0 + r >= g.K[0]) continue;
+    const float2 F = rec.F;
+    for (int row = lane & 7; row < ncc; row += 8) {
+      const float2 kv = kdata[(row0 + row) * g.M + m];
+      const float2 s = cmul(kv, F);
+      if (me >= 0 && isfinite(s.x) && isfinite(s.y)) continue;
+      const float om0 = omega[m], om1 = omega[g.M + m];
+      const float theta = sample_theta<float, 2>(g, omega, m);
+      const float2 u = cmul_conj(cmul_conj(kv, make_float2(cosf(theta), sinf(theta))), sep_tap_weight(g, 0, om0, i));
+      for (int j = 0; j < g.J[1]; ++j) {
+        const int c = c0 + j;
+        if (c >= 0 && c < kRegT1 && o1 + c < g.K[1]) {
+          const float2 v = cmul_conj(u, sep_tap_weight(g, 1, om1, j));
+          float2* dst = grid + (row0 + row) * g.G + (int64_t)(o0 + r) * g.stride[0] + (o1 + c);
           unsafeAtomicAdd(&dst->x, v.x);
           unsafeAtomicAdd(&dst->y, v.y);
         }
       }
     }
-    lds_barrier();
-  }
-
-  // Exception entries (complex weights; none for the reference's own tables except
-  // rare rounding cases) are added with atomics after the tile's stores are complete:
-  // thread (tap row i, coil row) adds s * w0[i] * w1[j] over the row's in-tile taps.
-  if (!anyexc) return;
-  __syncthreads();  // waits for the flush stores
-  for (int base = i0; base < i1; base += 64) {
-    const int e = base + lane;
-    const unsigned long long exc = __ballot(e < i1 && perm[min(e, i1 - 1)] < 0);
-    unsigned long long mk = exc;
-    while (mk) {
-      const int c = __ffsll(mk) - 1;
-      mk &= mk - 1;
-      const int ei = base + c;
-      const int m = perm[ei] & 0x7fffffff;
-      const int i = threadIdx.x >> 5;  // tap row 0..15 (0..5 used)
-      if (i < J0 && coil < ncc) {
-        const SepRec& r = recs[ei];
-        const int r0 = (r.rc & 255) - 8, c0 = ((r.rc >> 8) & 255) - 8;
-        const int k0 = r0 + i;
-        if (k0 >= 0 && k0 < kRegT0 && o0 + k0 < g.K[0]) {
-          const float om0 = omega[m], om1 = omega[g.M + m];
-          const float2 t0 = sep_tap_weight(g, 0, om0, i);
-          const float2 u = cmul(cmul(kdata[(rbase + coil) * g.M + m], r.F), make_float2(t0.x, -t0.y));
-          for (int j = 0; j < g.J[1]; ++j) {
-            const int k1 = c0 + j;
-            if (k1 >= 0 && k1 < kRegT1 && o1 + k1 < g.K[1]) {
-              const float2 t1 = sep_tap_weight(g, 1, om1, j);
-              const float2 v = cmul(u, make_float2(t1.x, -t1.y));
-              float2* dst = grid + (rbase + coil) * g.G + (int64_t)(o0 + k0) * g.stride[0] + (o1 + k1);
-              unsafeAtomicAdd(&dst->x, v.x);
-              unsafeAtomicAdd(&dst->y, v.y);
-            }
-          }
-        }
-      }
-    }
   }
 }
 
-// zeroes the tiles whose pieces add into the grid
-__global__ void __launch_bounds__(256)
-    sep_zero_hot_kernel(const Geom<float> g, const TileGeom tg, const int* __restrict__ ws, float2* __restrict__ grid) {
-  const int t = blockIdx.x;
-  const int* start = ws + tg.o_start;
-  if (reg_splits(start[t + 1] - start[t]) <= 1) return;
-  const int64_t nrows = g.B * g.C;
-  const int64_t r0 = (int64_t)blockIdx.y * 64;
-  const int64_t r1 = r0 + 64 < nrows ? r0 + 64 : nrows;
+// (At least two waves per SIMD asked for: the accumulators then stay in VGPRs.  With the
+// larger register budget the compiler keeps them in AGPRs and moves them to VGPRs and back
+// around every skipped row.)
+template <int G>
+__global__ void __launch_bounds__(64 * kMmWaves) __attribute__((amdgpu_waves_per_eu(mm_waves(G))))
+    spread_sep_kernel(const Geom<float> g, const TileGeom tg, const SepGeom sg, const float2* __restrict__ kdata,
+                      const float* __restrict__ omega, const int* __restrict__ ws, float2* __restrict__ grid,
+                      int nchunk, int ks) {
+  __shared__ MmLds<G> lds[kMmWaves];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t b = blockIdx.y;  // trajectory
+  const int64_t item = ks == 1 ? (int64_t)blockIdx.x * kMmWaves + wave : (int64_t)blockIdx.x;
+  const int64_t wi = item / nchunk;
+  spread_sep_item<G>(g, tg, sg, kdata, omega + b * 2 * g.M, ws + b * tg.plan_stride, grid, g.batched ? b * g.C : 0,
+                     g.batched ? g.C : g.B * g.C, wi, (int)(item - wi * nchunk), ks, wave, lds, lds[wave]);
+}
+
+__device__ __forceinline__ void sep_zero_hot_item(const Geom<float>& g, const TileGeom& tg, const int* plan,
+                                                  float2* __restrict__ grid, int t, int64_t r0, int64_t r1) {
+  const int* start = plan + tg.o_start;
+  if (mm_splits(start[t + 1] - start[t], tg.target) <= 1) return;
   const int o0 = ((t / tg.bstride[0]) % tg.nb[0]) * kRegT0;
   const int o1 = ((t / tg.bstride[1]) % tg.nb[1]) * kRegT1;
   for (int cell = threadIdx.x; cell < kRegT0 * kRegT1; cell += blockDim.x) {
@@ -1880,6 +2099,11 @@ static int64_t spread_workspace_bytes(const tkbn_interp_desc* d, const TileGeom&
   return nplans * tg.plan_ints * 4 + 16;
 }
 
+// the sample-lane spread's workspace
+static int64_t adj_lane_bytes(const tkbn_interp_desc* d, bool det) {
+  return plan_cache_bytes(d) + spread_workspace_bytes(d, make_tile_geom(d, det));
+}
+
 static size_t spread_lds_bytes(const tkbn_interp_desc* d, const TileGeom& tg, bool det) {
   (void)d;
   (void)det;
@@ -1946,24 +2170,47 @@ int spread_launch(const Geom<T>& g, const TileGeom& tg, bool det, const void* kd
   return TKBN_OK;
 }
 
-// ---- multi-coil (lanes = coil rows) variant -------------------------------------
+// ---- separable variant ----------------------------------------------------------
+static int64_t plans_of(const tkbn_interp_desc* d) { return d->omega_batched ? d->batch : 1; }
+static int64_t rows_of(const tkbn_interp_desc* d) { return d->omega_batched ? d->coils : d->batch * d->coils; }
+// Form of the spread (see spread_sep_item): the outer form up to four rows (two products per
+// row and four entries; the rows form takes about eight per eight rows), 16 rows at once
+// where there are more than eight (the weights of four entries then serve twice the rows).
+static int mm_form(int64_t nrows) { return nrows > 8 ? 16 : nrows > 4 ? 8 : nrows > 2 ? 4 : (int)nrows; }
+
+// (sample, tile) entries of all trajectories, about: (21/16)^2 a sample
+static int64_t sep_entries(const tkbn_interp_desc* d) { return plans_of(d) * (d->klength * 7 / 4); }
+// Waves that share a tile's entries: the whole group where the tiles x chunks alone do not
+// fill the chip (4096 waves) and hold at least a batch of entries each (39 rows, 434 x 362:
+// 142 -> 77 us, 12 rows, 512^2: 75 -> 51 us; 64 rows, 640^2, the other way: 216 -> 273 us).
+static int mm_waves_per_item(int64_t entries, int64_t tiles, int64_t chunks) {
+  return tiles * chunks < 4096 && entries >= kMmBatch * tiles ? kMmWaves : 1;
+}
+
 static TileGeom make_coil_tile_geom(const tkbn_interp_desc* d) {
-  // same plan layout as the sample-lane spread, with 16 x 16 tiles
-  tkbn_interp_desc dd = *d;
-  TileGeom tg = make_tile_geom(&dd, false);
+  TileGeom tg{};
   const int TT[2] = {kRegT0, kRegT1};
   for (int i = 0; i < 2; ++i) {
+    tg.K[i] = (int)d->grid_size[i];
+    tg.J[i] = (int)d->numpoints[i];
     tg.T[i] = TT[i];
     tg.nb[i] = (int)ceil_div(d->grid_size[i], TT[i]);
   }
+  tg.K[2] = tg.J[2] = tg.nb[2] = 1;
   tg.bstride[1] = 1;
   tg.bstride[0] = tg.nb[1];
-  tg.lstride[1] = 1;
-  tg.lstride[0] = tg.T[1];
   tg.NB = tg.nb[0] * tg.nb[1];
-  tg.tcells = kRegT0 * kRegT1;
-  tg.CC = 64;
-  tg.target = 1024;
+  // Entries per piece and wave.  A wave's entries are a serial chain, and pieces add with
+  // atomics: half of what a SIMD gets if the entries of all chunks spread evenly, so that the
+  // chains end with the rest, within 128 (one coil, 256^2, 402 x 512 radial: 16.6 us, 21.1
+  // with 384) and 1024 (64 rows, 320^2 radial: 216 us at 896, 250 at 512, 277 at 384).
+  {
+    const int64_t chunks = ceil_div(rows_of(d), mm_rows(mm_form(rows_of(d))));
+    const int64_t per_simd = sep_entries(d) * chunks / 1024;
+    const int64_t half = ceil_div(per_simd / 2, kMmBatch) * kMmBatch;
+    const int ks = mm_waves_per_item(sep_entries(d), (int64_t)tg.NB * plans_of(d), chunks);
+    tg.target = ks * (int)(half < 128 ? 128 : half > 1024 ? 1024 : half);
+  }
   // tiles a footprint can meet per dimension: 2, or 3 when the last tile is shorter
   // than J - 1 (the footprint then crosses it into the first tile)
   int64_t per_sample = 1;
@@ -1971,36 +2218,28 @@ static TileGeom make_coil_tile_geom(const tkbn_interp_desc* d) {
     const int last = tg.K[i] - (tg.nb[i] - 1) * tg.T[i];
     per_sample *= last >= tg.J[i] - 1 ? 2 : 3;
   }
-  const int64_t M = d->klength;
-  tg.maxent = per_sample * M;
-  tg.maxwork = tg.NB + tg.maxent / kRegHotTarget + 1;
-  tg.nkeys = (int64_t)tg.NB * kRegKeys;
-  int64_t o = 0;
-  tg.o_key = o;
-  tg.o_perm = o; o += tg.maxent;
-  tg.o_count = o; o += tg.nkeys;
-  tg.o_start = o; o += tg.nkeys + 1;
-  tg.o_cursor = o; o += tg.nkeys;
-  tg.o_wstart = o; o += tg.NB + 1;
-  tg.o_work = o; o += (tg.maxwork > tg.NB ? tg.maxwork : tg.NB);
-  tg.o_nwork = o; o += 1;
-  tg.o_hot = o; o += tg.NB + 1;
-  tg.o_cold = o; o += tg.NB + 1;
-  o = (o + 3) & ~3LL;  // 16-byte aligned records
-  tg.plan_ints = o;
-  tg.o_rec_bytes = o * 4;
+  tg.maxent = per_sample * d->klength;
+  tg.maxwork = tg.NB + tg.maxent / tg.target + 1;  // sum of ceil(V / target)
   return tg;
 }
 
-// register-accumulation spread: complex64, 2-D, shared trajectory, J <= 6, enough
-// coil rows to fill the lanes, and grids of at least tile + J - 1 cells per dimension
-static bool coil_variant_eligible(const tkbn_interp_desc* d) {
-  if (d->dtype != TKBN_F32 || d->ndim != 2 || d->omega_batched) return false;
+// The separable kernels take complex64, 2-D, J <= 6.  From 32 coil rows on one trajectory
+// they are the only 2-D path (their tuning fields are ignored); below, a caller's tile or
+// work target asks for the sample-lane kernels, whose fields they are, and so does a
+// problem whose separable plan (about 80 bytes a sample) would pass 1 GiB.  Below 32 rows,
+// sample-lane against separable: spread 31 -> 18 us, gather 25 -> 13 us (one row, 512^2 grid,
+// 206 000 samples), spread + gather 255 -> 108 us (8 trajectories x 8 rows, 384^2).
+static bool sep_eligible(const tkbn_interp_desc* d) {
+  if (d->dtype != TKBN_F32 || d->ndim != 2) return false;
   if (d->numpoints[0] > 6 || d->numpoints[1] > 6) return false;
-  if (d->batch * d->coils < 32) return false;
-  return d->grid_size[0] >= kRegT0 + 5 && d->grid_size[1] >= kRegT1 + 5;
+  if (!d->omega_batched && d->batch * d->coils >= 32) return true;
+  if (d->tile[0] > 0 || d->tile[1] > 0 || d->work_target > 0) return false;
+  return (d->omega_batched ? d->batch : 1) * d->klength * 80 <= (1LL << 30);
 }
-
+// and the spread grids of at least tile + J - 1 cells per dimension
+static bool coil_variant_eligible(const tkbn_interp_desc* d) {
+  return sep_eligible(d) && d->grid_size[0] >= kRegT0 + 5 && d->grid_size[1] >= kRegT1 + 5;
+}
 // One-shot timing hook: events the caller asked to have recorded around the next
 // main interpolation kernel (tkbn_profile_next_kernel).
 struct ProfileHook {
@@ -2009,10 +2248,10 @@ struct ProfileHook {
 static thread_local ProfileHook g_profile;
 
 static void profile_before(hipStream_t s) {
-  if (g_profile.start) hipEventRecord(g_profile.start, s);
+  if (g_profile.start) (void)hipEventRecord(g_profile.start, s);
 }
 static void profile_after(hipStream_t s) {
-  if (g_profile.stop) hipEventRecord(g_profile.stop, s);
+  if (g_profile.stop) (void)hipEventRecord(g_profile.stop, s);
   g_profile = ProfileHook{};
 }
 
@@ -2026,9 +2265,10 @@ constexpr int kPlanSepSpread = 7;
 static void sep_finish_layout(TileGeom& tg, SepGeom& sg, int64_t o, const tkbn_interp_desc* d) {
   sg.o_nm1 = o;
   o += 2;
+  o = (o + 3) & ~3LL;
   for (int i = 0; i < 2; ++i) {
     sg.o_ptab[i] = o;
-    o += 2 * d->grid_size[i];
+    o += 4 * d->grid_size[i];
   }
   for (int i = 0; i < 2; ++i) {
     sg.o_rtab[i] = o;
@@ -2037,6 +2277,7 @@ static void sep_finish_layout(TileGeom& tg, SepGeom& sg, int64_t o, const tkbn_i
   o = (o + 15) & ~15LL;
   tg.plan_ints = o;
   tg.o_rec_bytes = o * 4;
+  tg.plan_stride = o + (tg.rec_entry ? tg.maxent : d->klength) * (int64_t)(sizeof(SepRec) / 4);
 }
 
 static SepGeom sep_phase_of(const tkbn_interp_desc* d) {
@@ -2051,7 +2292,7 @@ static TileGeom make_sep_gather_geom(const tkbn_interp_desc* d, SepGeom* sg) {
   int64_t o = 0;
   tg.o_key = o;
   tg.o_perm = o;  // unused: the records carry the sample index
-  tg.o_count = o; o += tg.NB + 1;  // + the table flag
+  tg.o_count = o; o += tg.NB + 2;  // + the table flag, finished count blocks
   tg.o_start = o; o += tg.NB + 1;
   tg.o_cursor = o; o += tg.NB;
   tg.o_wstart = o; o += tg.NB + 1;
@@ -2065,11 +2306,16 @@ static TileGeom make_sep_gather_geom(const tkbn_interp_desc* d, SepGeom* sg) {
 
 static TileGeom make_sep_spread_geom(const tkbn_interp_desc* d, SepGeom* sg) {
   TileGeom tg = make_coil_tile_geom(d);
+  // 16 rows a chunk: a record per entry is read in order (16 coils x 4, 320^2 radial: 225 us;
+  // through the sample index: 245); fewer rows, where the plan weighs more against the data,
+  // a record per sample (one row, 205 824 samples: 16 instead of 56 MB, 17.8 us both)
+  tg.rec_entry = mm_form(rows_of(d)) == 16;
+  tg.T[2] = 2 * tg.target + tg.rec_entry;  // part of the plan's key
   *sg = sep_phase_of(d);
   int64_t o = 0;
   tg.o_key = o;
   tg.o_perm = o; o += tg.maxent;
-  tg.o_count = o; o += tg.NB + 1;  // + the table flag
+  tg.o_count = o; o += tg.NB + 2;  // + the table flag, finished count blocks
   tg.o_start = o; o += tg.NB + 1;
   tg.o_cursor = o; o += tg.NB;
   tg.o_wstart = o; o += tg.NB + 1;
@@ -2081,9 +2327,67 @@ static TileGeom make_sep_spread_geom(const tkbn_interp_desc* d, SepGeom* sg) {
   return tg;
 }
 
-// records (the gather's followed by its exception records at the same indices)
-static int64_t sep_workspace_bytes(const TileGeom& tg, bool gather) {
-  return tg.o_rec_bytes + tg.maxent * (int64_t)(sizeof(SepRec) + (gather ? sizeof(SepX) : 0));
+static int64_t sep_workspace_bytes(const tkbn_interp_desc* d, const TileGeom& tg) {
+  return plans_of(d) * tg.plan_stride * 4;
+}
+
+// The plan kernels of the separable gather (grid = nullptr) or spread, one plan per
+// trajectory; the spread's last one also clears what is added into in `grid`.
+static int sep_plan_launch(const tkbn_interp_desc* d, float2* grid, const Geom<float>& g, const TileGeom& tg,
+                           const SepGeom& sg, const float* om, void* ws, int* wsi, hipStream_t s) {
+  const bool spread = grid != nullptr;
+  const int kind = spread ? kPlanSepSpread : kPlanSepGather;
+  const int64_t np = plans_of(d);
+  TKBN_REQUIRE(np < 65536, TKBN_ERR_UNSUPPORTED, "too many trajectories in one call");
+  const int64_t zero_blocks = spread ? tg.NB * ceil_div(rows_of(d), 64) : 0;
+  const bool reused = plan_reused(d);
+  const int nscatter = reused ? 0 : (int)bin_grid(g.M);
+  TKBN_REQUIRE(zero_blocks + nscatter < (1LL << 31), TKBN_ERR_UNSUPPORTED,
+               "too many coil rows x work items for one launch");
+  CacheHdr* cache = nullptr;
+  const dim3 gc((unsigned)nscatter, (unsigned)np);
+  hipError_t e1 = hipSuccess;
+  if (reused) {
+    const int st = plan_registry_require(d, kind, tg.T, ws);
+    if (st != TKBN_OK || !spread) return st;
+  } else {
+    CacheZero z;
+    z.p = wsi + tg.o_count;
+    z.n = tg.NB + 2;
+    z.stride = tg.plan_stride;
+    z.copies = np;
+    const int st = plan_cache_begin(d, kind, tg.T, om, ws, s, &cache, z);
+    if (st != TKBN_OK) return st;
+    if (spread)
+      sep_spr_count_kernel<<<gc, dim3(256), 0, s>>>(g, tg, sg, om, wsi, cache);
+    else
+      sep_gat_count_kernel<<<gc, dim3(256), 0, s>>>(g, tg, sg, om, wsi, cache);
+    e1 = hipGetLastError();
+  }
+  if (spread)
+    sep_spr_scatter_kernel<<<dim3((unsigned)(nscatter + zero_blocks), (unsigned)np), dim3(256), 0, s>>>(
+        g, tg, sg, om, wsi, cache, nscatter, grid);
+  else
+    sep_gat_scatter_kernel<<<gc, dim3(256), 0, s>>>(g, tg, sg, om, wsi, cache);
+  const hipError_t e2 = hipGetLastError();
+  if (e1 != hipSuccess || e2 != hipSuccess) {
+    if (!reused) plan_cache_invalidate(ws, s);
+    set_error("launch of the separable plan failed: %s", hipGetErrorString(e1 != hipSuccess ? e1 : e2));
+    return TKBN_ERR_HIP;
+  }
+  return TKBN_OK;
+}
+
+// coil rows per work item of the gather (see gather_sep_kernel)
+static int gat_rows(int64_t nrows) { return nrows > 8 ? 16 : nrows > 4 ? 8 : nrows > 2 ? 4 : nrows > 1 ? 2 : 1; }
+
+template <int ROWS>
+static void gather_sep_start(const Geom<float>& g, const TileGeom& tg, const SepGeom& sg, const float2* grid,
+                             const float* om, const int* wsi, float2* kdata, int nchunk, dim3 grd, hipStream_t s) {
+  if (g.J[0] == 6 && g.J[1] == 6)
+    gather_sep_kernel<6, ROWS><<<grd, dim3(GatShape<ROWS>::kThreads), 0, s>>>(g, tg, sg, grid, om, wsi, kdata, nchunk);
+  else
+    gather_sep_kernel<0, ROWS><<<grd, dim3(GatShape<ROWS>::kThreads), 0, s>>>(g, tg, sg, grid, om, wsi, kdata, nchunk);
 }
 
 static int gather_sep_launch(const tkbn_interp_desc* d, const void* grid, const void* omega, void* kdata, void* ws,
@@ -2093,41 +2397,24 @@ static int gather_sep_launch(const tkbn_interp_desc* d, const void* grid, const 
   const TileGeom tg = make_sep_gather_geom(d, &sg);
   int* wsi = reinterpret_cast<int*>(static_cast<char*>(ws) + plan_cache_bytes(d));
   const float* om = static_cast<const float*>(omega);
-  if (!plan_reused(d)) {
-    CacheHdr* cache = nullptr;
-    CacheZero z;
-    z.p = wsi + tg.o_count;
-    z.n = tg.NB + 1;
-    int st = plan_cache_begin(d, kPlanSepGather, tg.T, omega, ws, s, &cache, z);
-    if (st != TKBN_OK) return st;
-    const dim3 gc(bin_grid(g.M));
-    sep_gat_count_kernel<<<gc, dim3(256), 0, s>>>(g, tg, sg, om, wsi, cache);
-    hipError_t e1 = hipGetLastError();
-    sep_plan_scan_kernel<<<dim3(1), dim3(1024), 0, s>>>(tg, wsi, cache, tg.target, tg.target, 1);
-    hipError_t e2 = hipGetLastError();
-    sep_gat_scatter_kernel<<<gc, dim3(256), 0, s>>>(g, tg, sg, om, wsi, cache);
-    hipError_t e3 = hipGetLastError();
-    if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess) {
-      plan_cache_invalidate(ws, s);
-      set_error("launch of the separable gather plan failed: %s",
-                hipGetErrorString(e1 != hipSuccess ? e1 : (e2 != hipSuccess ? e2 : e3)));
-      return TKBN_ERR_HIP;
-    }
-  } else {
-    const int st = plan_registry_require(d, kPlanSepGather, tg.T, ws);
-    if (st != TKBN_OK) return st;
-  }
-  const int nchunk = (int)ceil_div(g.B * g.C, kGatRows);
+  const int st = sep_plan_launch(d, nullptr, g, tg, sg, om, ws, wsi, s);
+  if (st != TKBN_OK) return st;
+  const int rows = gat_rows(rows_of(d));
+  const int nchunk = (int)ceil_div(rows_of(d), rows);
   const int64_t run = (int64_t)kXcdTiles * nchunk;  // see xcd_work_item
   const int64_t groups = ceil_div(tg.maxwork * nchunk, 8 * run) * 8 * run;
   TKBN_REQUIRE(groups < (1LL << 31), TKBN_ERR_UNSUPPORTED, "too many coil rows x work items for one launch");
+  const dim3 grd((unsigned)groups, (unsigned)plans_of(d));
+  const float2* gr = static_cast<const float2*>(grid);
+  float2* kd = static_cast<float2*>(kdata);
   profile_before(s);
-  if (g.J[0] == 6 && g.J[1] == 6)
-    gather_sep_kernel<6><<<dim3((unsigned)groups), dim3(kGatThreads), 0, s>>>(
-        g, tg, sg, static_cast<const float2*>(grid), wsi, static_cast<float2*>(kdata), nchunk);
-  else
-    gather_sep_kernel<0><<<dim3((unsigned)groups), dim3(kGatThreads), 0, s>>>(
-        g, tg, sg, static_cast<const float2*>(grid), wsi, static_cast<float2*>(kdata), nchunk);
+  switch (rows) {
+    case 16: gather_sep_start<16>(g, tg, sg, gr, om, wsi, kd, nchunk, grd, s); break;
+    case 8: gather_sep_start<8>(g, tg, sg, gr, om, wsi, kd, nchunk, grd, s); break;
+    case 4: gather_sep_start<4>(g, tg, sg, gr, om, wsi, kd, nchunk, grd, s); break;
+    case 2: gather_sep_start<2>(g, tg, sg, gr, om, wsi, kd, nchunk, grd, s); break;
+    default: gather_sep_start<1>(g, tg, sg, gr, om, wsi, kd, nchunk, grd, s); break;
+  }
   profile_after(s);
   TKBN_LAUNCH_CHECK("gather_sep_kernel");
   note_kernel("gather_sep_kernel");
@@ -2141,39 +2428,25 @@ static int spread_sep_launch(const tkbn_interp_desc* d, const void* kdata, const
   const TileGeom tg = make_sep_spread_geom(d, &sg);
   int* wsi = reinterpret_cast<int*>(static_cast<char*>(ws) + plan_cache_bytes(d));
   const float* om = static_cast<const float*>(omega);
-  if (!plan_reused(d)) {
-    CacheHdr* cache = nullptr;
-    CacheZero z;
-    z.p = wsi + tg.o_count;
-    z.n = tg.NB + 1;
-    int st = plan_cache_begin(d, kPlanSepSpread, tg.T, omega, ws, s, &cache, z);
-    if (st != TKBN_OK) return st;
-    const dim3 gc(bin_grid(g.M));
-    sep_spr_count_kernel<<<gc, dim3(256), 0, s>>>(g, tg, sg, om, wsi, cache);
-    hipError_t e1 = hipGetLastError();
-    sep_plan_scan_kernel<<<dim3(1), dim3(1024), 0, s>>>(tg, wsi, cache, kRegMaxUnsplit, kRegHotTarget, 0);
-    hipError_t e2 = hipGetLastError();
-    sep_spr_scatter_kernel<<<gc, dim3(256), 0, s>>>(g, tg, sg, om, wsi, cache);
-    hipError_t e3 = hipGetLastError();
-    if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess) {
-      plan_cache_invalidate(ws, s);
-      set_error("launch of the separable spread plan failed: %s",
-                hipGetErrorString(e1 != hipSuccess ? e1 : (e2 != hipSuccess ? e2 : e3)));
-      return TKBN_ERR_HIP;
-    }
-  } else {
-    const int st = plan_registry_require(d, kPlanSepSpread, tg.T, ws);
-    if (st != TKBN_OK) return st;
-  }
-  const int64_t nrows = g.B * g.C;
-  const unsigned ychunks = (unsigned)ceil_div(nrows, 64);
-  sep_zero_hot_kernel<<<dim3((unsigned)tg.NB, ychunks, 1), dim3(256), 0, s>>>(g, tg, wsi, static_cast<float2*>(grid));
-  TKBN_LAUNCH_CHECK("sep_zero_hot_kernel");
-  const int nchunk = (int)ceil_div(nrows, kRegCoils);
-  TKBN_REQUIRE(tg.maxwork * nchunk < (1LL << 31), TKBN_ERR_UNSUPPORTED, "too many coil rows x work items for one launch");
+  const int st = sep_plan_launch(d, static_cast<float2*>(grid), g, tg, sg, om, ws, wsi, s);
+  if (st != TKBN_OK) return st;
+  const int64_t nrows = rows_of(d), np = plans_of(d);
+  const int form = mm_form(nrows);
+  const int nchunk = (int)ceil_div(nrows, mm_rows(form));
+  const int ks = mm_waves_per_item(sep_entries(d), tg.NB * plans_of(d), nchunk);
+  const int64_t groups = ceil_div(tg.maxwork * nchunk, kMmWaves / ks);
+  TKBN_REQUIRE(groups < (1LL << 31), TKBN_ERR_UNSUPPORTED, "too many coil rows x work items for one launch");
+  const dim3 grd((unsigned)groups, (unsigned)np), blk(64 * kMmWaves);
+  const float2* kd = static_cast<const float2*>(kdata);
+  float2* gr = static_cast<float2*>(grid);
   profile_before(s);
-  spread_sep_kernel<<<dim3((unsigned)(tg.maxwork * nchunk)), dim3(kRegThreads), 0, s>>>(
-      g, tg, sg, static_cast<const float2*>(kdata), om, wsi, static_cast<float2*>(grid), nchunk);
+  switch (form) {
+    case 1: spread_sep_kernel<1><<<grd, blk, 0, s>>>(g, tg, sg, kd, om, wsi, gr, nchunk, ks); break;
+    case 2: spread_sep_kernel<2><<<grd, blk, 0, s>>>(g, tg, sg, kd, om, wsi, gr, nchunk, ks); break;
+    case 4: spread_sep_kernel<4><<<grd, blk, 0, s>>>(g, tg, sg, kd, om, wsi, gr, nchunk, ks); break;
+    case 8: spread_sep_kernel<8><<<grd, blk, 0, s>>>(g, tg, sg, kd, om, wsi, gr, nchunk, ks); break;
+    default: spread_sep_kernel<16><<<grd, blk, 0, s>>>(g, tg, sg, kd, om, wsi, gr, nchunk, ks); break;
+  }
   profile_after(s);
   TKBN_LAUNCH_CHECK("spread_sep_kernel");
   note_kernel("spread_sep_kernel");
@@ -2797,9 +3070,9 @@ static int spread_dispatch(const Geom<T>& g, const TileGeom& tg, bool det, const
 
 template <typename T>
 int interp_adj_t(const tkbn_interp_desc* d, bool det, const void* kdata, const void* omega, void* grid, void* ws,
-                 hipStream_t s) {
+                 hipStream_t s, bool sep = true) {
   if (std::is_same<T, float>::value && reg3_eligible(d)) return reg3_spread_launch(d, det, kdata, omega, ws, grid, s);
-  if (std::is_same<T, float>::value && !det && coil_variant_eligible(d))
+  if (std::is_same<T, float>::value && sep && !det && coil_variant_eligible(d))
     return spread_sep_launch(d, kdata, omega, ws, grid, s);
   const Geom<T> g = make_geom<T>(d);
   const TileGeom tg = make_tile_geom(d, det);
@@ -2888,13 +3161,7 @@ int interp_fwd_tiled_t(const tkbn_interp_desc* d, const void* grid, const void* 
   return st;
 }
 
-// ---- multi-coil forward gather ---------------------------------------------------
-static bool gather_coils_eligible(const tkbn_interp_desc* d) {
-  if (d->dtype != TKBN_F32 || d->ndim != 2 || d->omega_batched) return false;
-  if (d->numpoints[0] > 6 || d->numpoints[1] > 6) return false;
-  return d->batch * d->coils >= 32;
-}
-
+// ---- separable forward gather ----------------------------------------------------
 static TileGeom make_gather_geom(const tkbn_interp_desc* d) {
   TileGeom tg{};
   const int TT[2] = {kGatT0, kGatT1};
@@ -2910,7 +3177,6 @@ static TileGeom make_gather_geom(const tkbn_interp_desc* d) {
   tg.bstride[2] = 0;
   tg.NB = tg.nb[0] * tg.nb[1];
   tg.own_only = 1;
-  tg.CC = kGatRows;
   tg.target = kGatTarget;
   const int64_t M = d->klength;
   tg.maxent = M;
@@ -2933,9 +3199,9 @@ static TileGeom make_gather_geom(const tkbn_interp_desc* d) {
 }
 
 int64_t interp_fwd_workspace_bytes(const tkbn_interp_desc* d) {
-  if (gather_coils_eligible(d)) {
+  if (sep_eligible(d)) {
     SepGeom sg;
-    return plan_cache_bytes(d) + sep_workspace_bytes(make_sep_gather_geom(d, &sg), true);
+    return plan_cache_bytes(d) + sep_workspace_bytes(d, make_sep_gather_geom(d, &sg));
   }
   const TileGeom tg = make_tile_geom(d, false, true);
   const size_t lds = (size_t)tg.CC * tg.rcells * (d->dtype == TKBN_F32 ? 8 : 16);
@@ -2945,7 +3211,7 @@ int64_t interp_fwd_workspace_bytes(const tkbn_interp_desc* d) {
 
 int interp_fwd_tiled(const tkbn_interp_desc* d, const void* grid, const void* omega, void* kdata, void* ws,
                      hipStream_t s) {
-  if (gather_coils_eligible(d)) return gather_sep_launch(d, grid, omega, kdata, ws, s);
+  if (sep_eligible(d)) return gather_sep_launch(d, grid, omega, kdata, ws, s);
   if (d->dtype == TKBN_F32) return interp_fwd_tiled_t<float>(d, grid, omega, kdata, ws, s);
   return interp_fwd_tiled_t<double>(d, grid, omega, kdata, ws, s);
 }
@@ -2969,6 +3235,8 @@ struct BatchProb {
   const float2* kdata_in;  // adjoint input
   float2* grid_out;        // adjoint output grid (fully overwritten)
   const float* omega;
+  SepGeom sf, sa;          // separable plans (sep_f, sep_a: which kind the plan above is)
+  int sep_f, sep_a;
   const int* wf;           // forward plan (past the workspace's cache header)
   const int* wa;           // adjoint plan
   void* slot;              // adjoint max|re|,|im| slot (8 bytes, cleared each call)
@@ -2978,7 +3246,9 @@ struct BatchProb {
 };
 
 // Offsets of the problems' work items: off_f[p] = sum_{q < p} nwork_f(q) * yf(q) (and
-// off_a the same for the adjoint), off[nprob] the totals; clears every adjoint slot.
+// off_a the same for the adjoint), off[nprob] the totals; clears every adjoint slot.  Both
+// kinds of problem (separable, sample-lane) are counted; each kind's launch passes over
+// the other's items.
 __global__ void __launch_bounds__(1024) batch_offsets_kernel(const BatchProb* __restrict__ probs, int nprob,
                                                              int* __restrict__ off_f, int* __restrict__ off_a,
                                                              int clear_slots) {
@@ -2992,7 +3262,7 @@ __global__ void __launch_bounds__(1024) batch_offsets_kernel(const BatchProb* __
       const BatchProb& q = probs[p0 + threadIdx.x];
       cf[threadIdx.x] = q.wf[q.tf.o_nwork] * (int)q.yf;
       ca[threadIdx.x] = q.wa[q.ta.o_nwork] * (int)q.ya;
-      if (clear_slots) *static_cast<unsigned long long*>(q.slot) = 0ull;
+      if (clear_slots && !q.sep_a) *static_cast<unsigned long long*>(q.slot) = 0ull;
     }
     __syncthreads();
     block_exclusive_scan(cf, off_f + p0, n, sbuf);  // off_f[p0 .. p0 + n]
@@ -3029,6 +3299,7 @@ __global__ void __launch_bounds__((fwd_tiled_threads<float, JM>()))
   if (item >= off[nprob]) return;
   const int p = batch_find(off, nprob, item);
   const BatchProb& q = probs[p];
+  if (q.sep_f) return;
   const int li = item - off[p];
   const int64_t wi = li / q.yf, yc = li - wi * q.yf;
   fwd_tiled_item<float, D, JM>(q.g, q.tf, q.grid_in, q.omega, q.wf, q.kdata_out, wi, yc, 0, smem_raw);
@@ -3047,6 +3318,12 @@ __global__ void __launch_bounds__(256) batch_zero_hot_kernel(const BatchProb* __
   const int64_t li = blk - q.zoff;
   const int64_t t = li / q.ya, yc = li - t * q.ya;
   if (t >= q.ta.NB) return;
+  if constexpr (D == 2) {
+    if (q.sep_a) {  // one chunk holds all rows (fewer than 32)
+      if (yc == 0) sep_zero_hot_item(q.g, q.ta, q.wa, q.grid_out, (int)t, 0, q.g.B * q.g.C);
+      return;
+    }
+  }
   zero_hot_tiles_item<float, D>(q.g, q.ta, q.wa, q.grid_out, (int)t, yc, 0);
 }
 
@@ -3054,6 +3331,7 @@ __global__ void __launch_bounds__(256) batch_zero_hot_kernel(const BatchProb* __
 // sample or trajectory value, into the problem's slot
 __global__ void __launch_bounds__(256) batch_maxabs_kernel(const BatchProb* __restrict__ probs) {
   const BatchProb& q = probs[blockIdx.y];
+  if (q.sep_a) return;  // the separable spread needs no bound
   const float* x = reinterpret_cast<const float*>(q.kdata_in);
   const int64_t n = q.g.B * q.g.C * q.g.M * 2;
   float mx = 0.f;
@@ -3086,17 +3364,57 @@ __global__ void __launch_bounds__(spread_tiles_threads(D))
   if (item >= off[nprob]) return;
   const int p = batch_find(off, nprob, item);
   const BatchProb& q = probs[p];
+  if (q.sep_a) return;
   const int li = item - off[p];
   const int64_t wi = li / q.ya, yc = li - wi * q.ya;
   spread_tiles_item<float, FIXED, D, JM>(q.g, q.ta, q.kdata_in, q.omega, q.wa, q.slot, q.grid_out, fallback, wi, yc, 0,
                                          smem_raw);
 }
 
+// the separable problems of a batch: a group (gather) or a wave (spread) per item
+template <int ROWS>
+__global__ void __launch_bounds__(GatShape<ROWS>::kThreads)
+    batch_gather_sep_kernel(const BatchProb* __restrict__ probs, int nprob, const int* __restrict__ off) {
+  __shared__ __attribute__((aligned(16))) float2 region[kGatCells * GatShape<ROWS>::kPitch];
+  __shared__ float2 ph[kGatR0 + kGatR1];
+  const int item = blockIdx.x;
+  if (item >= off[nprob]) return;
+  const int p = batch_find(off, nprob, item);
+  const BatchProb& q = probs[p];
+  if (!q.sep_f) return;
+  const int li = item - off[p];
+  const int64_t wi = li / q.yf;
+  const int yc = (int)(li - wi * q.yf);
+  if (q.g.J[0] == 6 && q.g.J[1] == 6)
+    gather_sep_item<6, ROWS>(q.g, q.tf, q.sf, q.grid_in, q.omega, q.wf, q.kdata_out, 0, q.g.B * q.g.C, wi, yc, region, ph);
+  else
+    gather_sep_item<0, ROWS>(q.g, q.tf, q.sf, q.grid_in, q.omega, q.wf, q.kdata_out, 0, q.g.B * q.g.C, wi, yc, region, ph);
+}
+
+template <int G>
+__global__ void __launch_bounds__(64 * kMmWaves) __attribute__((amdgpu_waves_per_eu(mm_waves(G))))
+    batch_spread_sep_kernel(const BatchProb* __restrict__ probs, int nprob, const int* __restrict__ off, int ks) {
+  __shared__ MmLds<G> lds[kMmWaves];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int item = ks == 1 ? blockIdx.x * kMmWaves + wave : blockIdx.x;
+  if (item >= off[nprob]) return;
+  const int p = __builtin_amdgcn_readfirstlane(batch_find(off, nprob, item));
+  const BatchProb& q = probs[p];
+  if (!q.sep_a) return;
+  const int li = item - off[p];
+  const int64_t wi = li / q.ya;
+  spread_sep_item<G>(q.g, q.ta, q.sa, q.kdata_in, q.omega, q.wa, q.grid_out, 0, q.g.B * q.g.C, wi, (int)(li - wi * q.ya),
+                     ks, wave, lds, lds[wave]);
+}
+
 }  // namespace tkbn
 
 struct tkbn_batch {
   int nprob = 0, ndim = 0, jm = 6, det = 0;
+  int gat_rows = 1, form = 1, ks = 1;              // shapes of the separable launches (the largest problem's rows)
+  int nsep_f = 0, nsep_a = 0;              // separable problems
   std::vector<tkbn::BatchProb> probs;
+  std::vector<int64_t> rows;
   std::vector<tkbn_interp_desc> descs_f, descs_a;
   std::vector<const void*> wsf, wsa;
   size_t lds_f = 0, lds_a = 0;
@@ -3108,9 +3426,10 @@ namespace tkbn {
 // the batch's plans must be the ones its workspaces hold (same check as TKBN_PLAN_REUSE)
 static int batch_plans_current(const tkbn_batch* b) {
   for (int p = 0; p < b->nprob; ++p) {
-    int st = plan_registry_require(&b->descs_f[p], kPlanFwdTiles, b->probs[p].tf.T, b->wsf[p]);
+    const BatchProb& q = b->probs[p];
+    int st = plan_registry_require(&b->descs_f[p], q.sep_f ? kPlanSepGather : kPlanFwdTiles, q.tf.T, b->wsf[p]);
     if (st != TKBN_OK) return st;
-    st = plan_registry_require(&b->descs_a[p], kPlanSpreadTiles + b->det, b->probs[p].ta.T, b->wsa[p]);
+    st = plan_registry_require(&b->descs_a[p], q.sep_a ? kPlanSepSpread : kPlanSpreadTiles + b->det, q.ta.T, b->wsa[p]);
     if (st != TKBN_OK) return st;
   }
   return TKBN_OK;
@@ -3146,7 +3465,7 @@ int tkbn_batch_create(const tkbn_interp_desc* descs, const tkbn_interp_desc* adj
   b->det = mode == TKBN_ADJ_DETERMINISTIC ? 1 : 0;
   b->ndim = descs[0].ndim;
   b->jm = max_numpoints(&descs[0]) <= 6 ? 6 : 16;
-  int64_t zoff = 0;
+  int64_t zoff = 0, entries = 0, tiles = 0;
   for (int p = 0; p < nprob; ++p) {
     const tkbn_interp_desc* d = &descs[p];
     const tkbn_interp_desc* da = adj_descs ? &adj_descs[p] : d;
@@ -3162,10 +3481,10 @@ int tkbn_batch_create(const tkbn_interp_desc* descs, const tkbn_interp_desc* adj
                 "class with unbatched trajectories", p);
       st = TKBN_ERR_UNSUPPORTED;
     }
-    if (st == TKBN_OK && (gather_coils_eligible(d) || interp_fwd_workspace_bytes(d) <= 0 ||
-                          (!b->det && coil_variant_eligible(da)) || reg3_eligible(da))) {
-      set_error("tkbn_batch_create: problem %d takes the multi-coil or unbinned path; batches run the sample-lane "
-                "kernels only (fewer than 32 coil rows)", p);
+    if (st == TKBN_OK && ((d->ndim == 2 && d->numpoints[0] <= 6 && d->numpoints[1] <= 6 && d->batch * d->coils >= 32) ||
+                          interp_fwd_workspace_bytes(d) <= 0 || reg3_eligible(da))) {
+      set_error("tkbn_batch_create: problem %d takes a path of its own or is unbinned; batches take problems of "
+                "fewer than 32 coil rows (2-D) or 4 (3-D)", p);
       st = TKBN_ERR_UNSUPPORTED;
     }
     if (st == TKBN_OK && !(grids_in && grids_in[p] && kdatas_out && kdatas_out[p] && kdatas_in && kdatas_in[p] &&
@@ -3180,8 +3499,12 @@ int tkbn_batch_create(const tkbn_interp_desc* descs, const tkbn_interp_desc* adj
     }
     BatchProb q{};
     q.g = make_geom<float>(d);
-    q.tf = make_tile_geom(d, false, true);
-    q.ta = make_tile_geom(da, b->det != 0);
+    q.sep_f = sep_eligible(d) ? 1 : 0;
+    q.sep_a = !b->det && coil_variant_eligible(da) ? 1 : 0;
+    q.tf = q.sep_f ? make_sep_gather_geom(d, &q.sf) : make_tile_geom(d, false, true);
+    q.ta = q.sep_a ? make_sep_spread_geom(da, &q.sa) : make_tile_geom(da, b->det != 0);
+    b->nsep_f += q.sep_f;
+    b->nsep_a += q.sep_a;
     q.grid_in = static_cast<const float2*>(grids_in[p]);
     q.kdata_out = static_cast<float2*>(kdatas_out[p]);
     q.kdata_in = static_cast<const float2*>(kdatas_in[p]);
@@ -3190,17 +3513,16 @@ int tkbn_batch_create(const tkbn_interp_desc* descs, const tkbn_interp_desc* adj
     const int64_t hdr = plan_cache_bytes(d);
     q.wf = reinterpret_cast<const int*>(static_cast<const char*>(fwd_workspaces[p]) + hdr);
     q.wa = reinterpret_cast<const int*>(static_cast<const char*>(adj_workspaces[p]) + hdr);
-    q.slot = static_cast<char*>(adj_workspaces[p]) + hdr + q.ta.plan_ints * 4;
+    q.slot = q.sep_a ? nullptr : static_cast<char*>(adj_workspaces[p]) + hdr + q.ta.plan_ints * 4;
     const int64_t nrows = d->batch * d->coils;
-    q.yf = ceil_div(nrows, q.tf.CC);
-    q.ya = ceil_div(nrows, q.ta.CC);
-    q.zoff = zoff;
+    if (q.sep_f) b->gat_rows = std::max(b->gat_rows, gat_rows(nrows));
+    if (q.sep_a) {
+      b->form = std::max(b->form, mm_form(nrows));
+      entries += sep_entries(da);
+      tiles += q.ta.NB;
+    }
+    b->rows.push_back(nrows);
     q.nom = (int64_t)d->ndim * d->klength;
-    zoff += (int64_t)q.ta.NB * q.ya;
-    b->lds_f = std::max(b->lds_f, (size_t)q.tf.CC * q.tf.rcells * sizeof(float2));
-    b->lds_a = std::max(b->lds_a, spread_lds_bytes(da, q.ta, b->det != 0));
-    b->bound_f += q.tf.maxwork * q.yf;
-    b->bound_a += q.ta.maxwork * q.ya;
     b->maxabs_blocks = std::max<int64_t>(b->maxabs_blocks, std::min<int64_t>(ceil_div(nrows * d->klength * 2, 4096), 64));
     b->probs.push_back(q);
     b->descs_f.push_back(*d);
@@ -3209,6 +3531,19 @@ int tkbn_batch_create(const tkbn_interp_desc* descs, const tkbn_interp_desc* adj
     b->descs_a.back().flags = 0;
     b->wsf.push_back(fwd_workspaces[p]);
     b->wsa.push_back(adj_workspaces[p]);
+  }
+  b->ks = mm_waves_per_item(entries, tiles, 1);
+  // row chunks per work item: one shape for all separable problems of a launch
+  for (int p = 0; p < nprob; ++p) {
+    BatchProb& q = b->probs[p];
+    q.yf = ceil_div(b->rows[p], q.sep_f ? b->gat_rows : q.tf.CC);
+    q.ya = ceil_div(b->rows[p], q.sep_a ? mm_rows(b->form) : q.ta.CC);
+    q.zoff = zoff;
+    zoff += (int64_t)q.ta.NB * q.ya;
+    if (!q.sep_f) b->lds_f = std::max(b->lds_f, (size_t)q.tf.CC * q.tf.rcells * sizeof(float2));
+    if (!q.sep_a) b->lds_a = std::max(b->lds_a, spread_lds_bytes(&b->descs_a[p], q.ta, b->det != 0));
+    b->bound_f += q.tf.maxwork * q.yf;
+    b->bound_a += q.ta.maxwork * q.ya;
   }
   b->zblocks = zoff;
   if (b->bound_f >= (1LL << 31) || b->bound_a >= (1LL << 31) || b->zblocks >= (1LL << 31)) {
@@ -3256,6 +3591,23 @@ int tkbn_batch_interp_fwd(const tkbn_batch* b, const void* table, void* workspac
   const dim3 grd((unsigned)b->bound_f);
 #define TKBN_BATCH_FWD(DD, JJ) \
   batch_fwd_kernel<DD, JJ><<<grd, dim3(fwd_tiled_threads<float, JJ>()), b->lds_f, s>>>(probs, b->nprob, off_f)
+  if (b->nsep_f > 0) {
+    switch (b->gat_rows) {
+#define TKBN_BATCH_GAT(R) \
+  batch_gather_sep_kernel<R><<<grd, dim3(GatShape<R>::kThreads), 0, s>>>(probs, b->nprob, off_f)
+      case 16: TKBN_BATCH_GAT(16); break;
+      case 8: TKBN_BATCH_GAT(8); break;
+      case 4: TKBN_BATCH_GAT(4); break;
+      case 2: TKBN_BATCH_GAT(2); break;
+      default: TKBN_BATCH_GAT(1); break;
+#undef TKBN_BATCH_GAT
+    }
+    TKBN_LAUNCH_CHECK("batch_gather_sep_kernel");
+  }
+  if (b->nsep_f == b->nprob) {
+    note_kernel("batch_fwd_kernel");
+    return TKBN_OK;
+  }
   if (b->jm == 6) {
     if (b->ndim == 1) TKBN_BATCH_FWD(1, 6);
     else if (b->ndim == 2) TKBN_BATCH_FWD(2, 6);
@@ -3290,10 +3642,27 @@ int tkbn_batch_interp_adj(const tkbn_batch* b, const void* table, void* workspac
     else batch_zero_hot_kernel<3><<<dim3((unsigned)b->zblocks), dim3(256), 0, s>>>(probs, b->nprob);
     TKBN_LAUNCH_CHECK("batch_zero_hot_kernel");
   }
-  batch_maxabs_kernel<<<dim3((unsigned)b->maxabs_blocks, (unsigned)b->nprob), dim3(256), 0, s>>>(probs);
-  TKBN_LAUNCH_CHECK("batch_maxabs_kernel");
+  if (b->nsep_a < b->nprob) {
+    batch_maxabs_kernel<<<dim3((unsigned)b->maxabs_blocks, (unsigned)b->nprob), dim3(256), 0, s>>>(probs);
+    TKBN_LAUNCH_CHECK("batch_maxabs_kernel");
+  }
   if (b->bound_a == 0) return TKBN_OK;
   const dim3 grd((unsigned)b->bound_a);
+  if (b->nsep_a > 0) {
+    const dim3 gs((unsigned)ceil_div(b->bound_a, kMmWaves / b->ks)), blk(64 * kMmWaves);
+    switch (b->form) {
+      case 1: batch_spread_sep_kernel<1><<<gs, blk, 0, s>>>(probs, b->nprob, off_a, b->ks); break;
+      case 2: batch_spread_sep_kernel<2><<<gs, blk, 0, s>>>(probs, b->nprob, off_a, b->ks); break;
+      case 4: batch_spread_sep_kernel<4><<<gs, blk, 0, s>>>(probs, b->nprob, off_a, b->ks); break;
+      case 8: batch_spread_sep_kernel<8><<<gs, blk, 0, s>>>(probs, b->nprob, off_a, b->ks); break;
+      default: batch_spread_sep_kernel<16><<<gs, blk, 0, s>>>(probs, b->nprob, off_a, b->ks); break;
+    }
+    TKBN_LAUNCH_CHECK("batch_spread_sep_kernel");
+  }
+  if (b->nsep_a == b->nprob) {
+    note_kernel("batch_spread_kernel<sep>");
+    return TKBN_OK;
+  }
 #define TKBN_BATCH_ADJ(FX, DD, JJ, FB) \
   batch_spread_kernel<FX, DD, JJ><<<grd, dim3(spread_tiles_threads(DD)), b->lds_a, s>>>(probs, b->nprob, off_a, FB)
 #define TKBN_BATCH_ADJ_PAIR(DD, JJ)      \
@@ -3373,7 +3742,21 @@ int tkbn_interp_adj_noalloc(const tkbn_interp_desc* desc, const void* kdata, con
   TKBN_REQUIRE(desc->flags == 0, TKBN_ERR_INVALID,
                "tkbn_interp_adj_noalloc takes no flags (its scratch may hold another call's plan)");
   if (desc->batch == 0 || desc->coils == 0) return TKBN_OK;
-  const int64_t need = tkbn_interp_adj_workspace_bytes(desc, mode);
+  // The scratch holds one path's plan at a time.  Fewer than 32 coil rows fall back to the
+  // sample-lane kernels, whose plan is smaller, where the separable plan does not fit.
+  const bool det = mode == TKBN_ADJ_DETERMINISTIC;
+  int64_t need = tkbn_interp_adj_workspace_bytes(desc, mode);
+  bool sep = true;
+  if (!det && coil_variant_eligible(desc)) {
+    SepGeom sg;
+    need = plan_cache_bytes(desc) + sep_workspace_bytes(desc, make_sep_spread_geom(desc, &sg));
+    if (need > kNoAllocScratchBytes && (desc->omega_batched || desc->batch * desc->coils < 32)) {
+      sep = false;
+      need = adj_lane_bytes(desc, det);
+    }
+  } else if (!det && desc->dtype == TKBN_F32 && desc->ndim == 2) {
+    need = adj_lane_bytes(desc, det);
+  }
   TKBN_REQUIRE(need >= 0 && need <= kNoAllocScratchBytes, TKBN_ERR_WORKSPACE,
                "tkbn_interp_adj_noalloc: this problem needs %lld bytes of workspace, more than the %lld-byte "
                "static scratch; use tkbn_interp_adj with a caller workspace",
@@ -3382,7 +3765,11 @@ int tkbn_interp_adj_noalloc(const tkbn_interp_desc* desc, const void* kdata, con
   void* ws = nullptr;
   st = noalloc_scratch(s, &ws);
   if (st != TKBN_OK) return st;
-  return tkbn_interp_adj(desc, kdata, omega, grid, mode, ws, kNoAllocScratchBytes, stream);
+  TKBN_REQUIRE(grid != nullptr, TKBN_ERR_INVALID, "NULL grid pointer");
+  TKBN_REQUIRE(desc->klength == 0 || (kdata && omega), TKBN_ERR_INVALID, "NULL data pointer");
+  TKBN_REQUIRE(desc->klength < (1LL << 31), TKBN_ERR_INVALID, "klength must be < 2^31");
+  if (desc->dtype == TKBN_F32) return interp_adj_t<float>(desc, det, kdata, omega, grid, ws, s, sep);
+  return interp_adj_t<double>(desc, det, kdata, omega, grid, ws, s);
 }
 
 int tkbn_profile_next_kernel(void* start_event, void* stop_event) {
@@ -3395,12 +3782,15 @@ int64_t tkbn_interp_adj_workspace_bytes(const tkbn_interp_desc* desc, int32_t mo
   if (validate_desc(desc) != TKBN_OK) return -1;
   if (mode != TKBN_ADJ_ATOMIC && mode != TKBN_ADJ_DETERMINISTIC) return -1;
   const bool det = mode == TKBN_ADJ_DETERMINISTIC;
-  const TileGeom tg = make_tile_geom(desc, det);
-  int64_t n = plan_cache_bytes(desc) + spread_workspace_bytes(desc, tg);
-  if (!det && coil_variant_eligible(desc)) {
+  int64_t n = adj_lane_bytes(desc, det);
+  // Room for the separable plan too, also where tuning fields ask for the sample-lane
+  // kernels: a caller that tunes one problem keeps one buffer.
+  tkbn_interp_desc plain = *desc;
+  for (int i = 0; i < 3; ++i) plain.tile[i] = 0;
+  plain.work_target = 0;
+  if (!det && coil_variant_eligible(&plain)) {
     SepGeom sg;
-    const int64_t nc = plan_cache_bytes(desc) + sep_workspace_bytes(make_sep_spread_geom(desc, &sg), false);
-    n = nc > n ? nc : n;
+    n += sep_workspace_bytes(desc, make_sep_spread_geom(desc, &sg));
   }
   if (reg3_eligible(desc)) {
     const int64_t nr = plan_cache_bytes(desc) + reg3_workspace_bytes(make_reg3_geom(desc, det));
