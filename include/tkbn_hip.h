@@ -288,6 +288,22 @@ TKBN_API int tkbn_fft_grid_adj(int32_t dtype, int32_t ndim, const int64_t* im_si
                                int64_t batch, int64_t coils, const void* grid, const void* smaps,
                                const void* scaling_coef, double scale, void* image, void* workspace,
                                int64_t workspace_bytes, void* stream);
+/*
+ * The same for grid sizes of any factors: primes up to 17 in place (sizes <= 2048), and a
+ * dimension with a larger one as a convolution (im_size + grid_size - 1 <= 1280).  The adjoint
+ * then takes smaps only where the last dimension is none, and scaling_coef NULL as 1.
+ */
+TKBN_API int tkbn_fft_any_supported(int32_t ndim, const int64_t* im_size, const int64_t* grid_size);
+TKBN_API int64_t tkbn_fft_any_workspace_bytes(int32_t ndim, const int64_t* im_size, const int64_t* grid_size,
+                                              int64_t batch, int64_t coils);
+TKBN_API int tkbn_fft_any_grid_fwd(int32_t dtype, int32_t ndim, const int64_t* im_size, const int64_t* grid_size,
+                                   int64_t batch, int64_t coils, int64_t image_coils, const void* image,
+                                   const void* smaps, const void* scaling_coef, double scale, void* grid,
+                                   void* workspace, int64_t workspace_bytes, void* stream);
+TKBN_API int tkbn_fft_any_grid_adj(int32_t dtype, int32_t ndim, const int64_t* im_size, const int64_t* grid_size,
+                                   int64_t batch, int64_t coils, const void* grid, const void* smaps,
+                                   const void* scaling_coef, double scale, void* image, void* workspace,
+                                   int64_t workspace_bytes, void* stream);
 
 /*
  * FFT filter on an oversampled grid (the Toeplitz-embedded normal operator), replacing

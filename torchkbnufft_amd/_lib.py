@@ -104,6 +104,18 @@ _SIGNATURES = {
         [_c_i32, _c_i32, ctypes.POINTER(_c_i64), ctypes.POINTER(_c_i64), _c_i64, _c_i64,
          _c_vp, _c_vp, _c_vp, _c_dbl, _c_vp, _c_vp, _c_i64, _c_vp],
     ),
+    "tkbn_fft_any_supported": (ctypes.c_int, [_c_i32, ctypes.POINTER(_c_i64), ctypes.POINTER(_c_i64)]),
+    "tkbn_fft_any_workspace_bytes": (_c_i64, [_c_i32, ctypes.POINTER(_c_i64), ctypes.POINTER(_c_i64), _c_i64, _c_i64]),
+    "tkbn_fft_any_grid_fwd": (
+        ctypes.c_int,
+        [_c_i32, _c_i32, ctypes.POINTER(_c_i64), ctypes.POINTER(_c_i64), _c_i64, _c_i64, _c_i64,
+         _c_vp, _c_vp, _c_vp, _c_dbl, _c_vp, _c_vp, _c_i64, _c_vp],
+    ),
+    "tkbn_fft_any_grid_adj": (
+        ctypes.c_int,
+        [_c_i32, _c_i32, ctypes.POINTER(_c_i64), ctypes.POINTER(_c_i64), _c_i64, _c_i64,
+         _c_vp, _c_vp, _c_vp, _c_dbl, _c_vp, _c_vp, _c_i64, _c_vp],
+    ),
     "tkbn_fft_filter": (
         ctypes.c_int,
         [_c_i32, _c_i32, ctypes.POINTER(_c_i64), ctypes.POINTER(_c_i64), _c_i64, _c_i64, _c_i64,

@@ -1,11 +1,12 @@
-"""Oversampled FFT stages: fused HIP scale/pad and crop/deapodise around torch.fft.
+"""Oversampled FFT stages: the fused HIP FFT, or fused scale/pad and crop/deapodise around torch.fft.
 
 ``fft_and_scale`` / ``ifft_and_scale`` keep the signatures of
 ``torchkbnufft/_nufft/fft.py:36-118``.  The element-wise work (scaling, zero-pad,
 crop, conjugate scaling, the SENSE coil expansion and coil combine of
-``modules/kbnufft.py:182-183,404-405``) is one HIP pass on each side; the FFT is
-``torch.fft`` (rocFFT) called unnormalised, with the ``"ortho"`` factor folded into
-the fused pass.
+``modules/kbnufft.py:182-183,404-405``) is part of the FFT's first and last pass
+(complex64, any grid size within the limits of ``tkbn_fft_any_supported``), or one HIP
+pass on each side of an unnormalised ``torch.fft`` (complex128, larger sizes); the
+``"ortho"`` factor is folded in.
 """
 from __future__ import annotations
 
@@ -89,6 +90,13 @@ def crop_deapod(grid: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, im_
             raise ValueError(f"smaps shape {tuple(smaps.shape)} does not match data ({B}, {C}) + {im}")
     sc = scaling_coef.to(device=grid.device, dtype=grid.dtype).contiguous()
     out = torch.empty((B, 1 if smaps is not None else C) + im, dtype=grid.dtype, device=grid.device)
+    _crop_deapod_into(grid, smaps, sc, im, scale, out)
+    return out
+
+
+def _crop_deapod_into(grid: Tensor, smaps: Optional[Tensor], sc: Tensor, im, scale: float, out: Tensor) -> None:
+    d, gs = len(im), tuple(grid.shape[2:])
+    B, C = grid.shape[0], grid.shape[1]
     with torch.cuda.device(grid.device):
         st = _lib.load().tkbn_crop_deapod(
             _lib.dtype_code(grid),
@@ -105,7 +113,6 @@ def crop_deapod(grid: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, im_
             _lib.stream_of(grid),
         )
     _lib.check(st, "tkbn_crop_deapod")
-    return out
 
 
 def fft_and_scale(image: Tensor, scaling_coef: Tensor, im_size: Tensor, grid_size: Tensor, norm: Optional[str] = None) -> Tensor:
@@ -115,7 +122,7 @@ def fft_and_scale(image: Tensor, scaling_coef: Tensor, im_size: Tensor, grid_siz
     gs = host_values(grid_size)
     im = host_values(im_size)
     scale = _norm_scale(norm, gs)
-    if fused_supported(image.dtype, im, gs):
+    if pipeline_supported(image.dtype, im, gs):
         return _run(GridForward, image, None, scaling_coef, im, gs, scale)
     grid = _run(ApodPad, image, None, scaling_coef, im, gs, scale)
     return torch.fft.fftn(grid, dim=tuple(range(-len(gs), 0)), norm="backward")
@@ -128,7 +135,7 @@ def ifft_and_scale(image: Tensor, scaling_coef: Tensor, im_size: Tensor, grid_si
     gs = host_values(grid_size)
     im = host_values(im_size)
     scale = _norm_scale(norm, gs)
-    if fused_supported(image.dtype, im, gs):
+    if pipeline_supported(image.dtype, im, gs):
         return _run(GridAdjoint, image, None, scaling_coef, im, scale)
     x = torch.fft.ifftn(image, dim=tuple(range(-len(gs), 0)), norm="forward")
     return _run(CropDeapod, x, None, scaling_coef, im, scale)
@@ -159,6 +166,33 @@ def fused_supported(dtype: torch.dtype, im_size, grid_size) -> bool:
     return ok
 
 
+def pipeline_supported(dtype: torch.dtype, im_size, grid_size) -> bool:
+    """The fused FFT, or the same passes with the other grid sizes as convolutions."""
+    if fused_supported(dtype, im_size, grid_size):
+        return True
+    if _FUSED_DISABLED or dtype != torch.complex64:
+        return False
+    key = (tuple(int(v) for v in im_size), tuple(int(v) for v in grid_size), "any")
+    ok = _FUSED_OK.get(key)
+    if ok is None:
+        ok = (
+            _lib.load().tkbn_fft_any_supported(len(key[0]), _lib.i64_array(key[0]), _lib.i64_array(key[1]))
+            == _lib.TKBN_OK
+        )
+        _FUSED_OK[key] = ok
+    return ok
+
+
+def _smooth(im, gs) -> bool:
+    """Every extent has compiled or planned butterflies (whatever set_fused_fft says)."""
+    key = (tuple(im), tuple(gs))
+    ok = _FUSED_OK.get(key)
+    if ok is None:
+        ok = _lib.load().tkbn_fft_supported(len(key[0]), _lib.i64_array(key[0]), _lib.i64_array(key[1])) == _lib.TKBN_OK
+        _FUSED_OK[key] = ok
+    return ok
+
+
 def _out_or_new(out: Optional[Tensor], shape: tuple, like: Tensor) -> Tensor:
     if out is None:
         return torch.empty(shape, dtype=like.dtype, device=like.device)
@@ -167,8 +201,9 @@ def _out_or_new(out: Optional[Tensor], shape: tuple, like: Tensor) -> Tensor:
     return out
 
 
-def _fft_workspace(dev, d, im, gs, B, C):
-    n = _lib.load().tkbn_fft_workspace_bytes(d, _lib.i64_array(im), _lib.i64_array(gs), B, C)
+def _fft_workspace(dev, d, im, gs, B, C, smooth=True):
+    lib = _lib.load()
+    n = (lib.tkbn_fft_workspace_bytes if smooth else lib.tkbn_fft_any_workspace_bytes)(d, _lib.i64_array(im), _lib.i64_array(gs), B, C)
     if n < 0:
         _lib.check(_lib.TKBN_ERR_INVALID, "tkbn_fft_workspace_bytes")
     return torch.empty(max(int(n), 1), dtype=torch.uint8, device=dev), int(n)
@@ -197,9 +232,11 @@ def fft_grid_fwd(image: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, i
             raise ValueError("image coil dimension must be 1 or match smaps")
     sc = scaling_coef.to(device=image.device, dtype=image.dtype).contiguous()
     grid = _out_or_new(out, (B, C) + gs, image)
-    ws, nws = _fft_workspace(image.device, d, im, gs, B, C)
+    smooth = _smooth(im, gs)
+    ws, nws = _fft_workspace(image.device, d, im, gs, B, C, smooth)
+    lib = _lib.load()
     with torch.cuda.device(image.device):
-        st = _lib.load().tkbn_fft_grid_fwd(
+        st = (lib.tkbn_fft_grid_fwd if smooth else lib.tkbn_fft_any_grid_fwd)(
             _lib.dtype_code(image), d, _lib.i64_array(im), _lib.i64_array(gs), B, C, image.shape[1],
             image.data_ptr(), smaps.data_ptr() if smaps is not None else None, sc.data_ptr(), float(scale),
             grid.data_ptr(), ws.data_ptr(), nws, _lib.stream_of(image),
@@ -225,15 +262,21 @@ def fft_grid_adj(grid: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, im
         if tuple(smaps.shape) != (B, C) + im:
             raise ValueError(f"smaps shape {tuple(smaps.shape)} does not match data ({B}, {C}) + {im}")
     sc = scaling_coef.to(device=grid.device, dtype=grid.dtype).contiguous()
+    smooth = _smooth(im, gs)
+    combine = smaps is not None and not smooth  # the convolution passes leave the coils apart
     out = _out_or_new(out, (B, 1 if smaps is not None else C) + im, grid)
-    ws, nws = _fft_workspace(grid.device, d, im, gs, B, C)
+    image = torch.empty((B, C) + im, dtype=grid.dtype, device=grid.device) if combine else out
+    ws, nws = _fft_workspace(grid.device, d, im, gs, B, C, smooth)
+    lib = _lib.load()
     with torch.cuda.device(grid.device):
-        st = _lib.load().tkbn_fft_grid_adj(
+        st = (lib.tkbn_fft_grid_adj if smooth else lib.tkbn_fft_any_grid_adj)(
             _lib.dtype_code(grid), d, _lib.i64_array(im), _lib.i64_array(gs), B, C, grid.data_ptr(),
-            smaps.data_ptr() if smaps is not None else None, sc.data_ptr(), float(scale), out.data_ptr(),
-            ws.data_ptr(), nws, _lib.stream_of(grid),
+            smaps.data_ptr() if smaps is not None and not combine else None, None if combine else sc.data_ptr(),
+            1.0 if combine else float(scale), image.data_ptr(), ws.data_ptr(), nws, _lib.stream_of(grid),
         )
     _lib.check(st, "tkbn_fft_grid_adj")
+    if combine:
+        _crop_deapod_into(image, smaps, sc, im, scale, out)
     return out
 
 

@@ -1,8 +1,7 @@
 // Oversampled FFT of the table NUFFT with the element-wise stages fused in (gfx950).
 //
 // Replaces fft_and_scale / ifft_and_scale (torchkbnufft/_nufft/fft.py:36-118) plus the
-// SENSE expansion and coil combine (modules/kbnufft.py:182-183, 404-405) for grid sizes
-// whose prime factors are 2, 3 and 5:
+// SENSE expansion and coil combine (modules/kbnufft.py:182-183, 404-405):
 //   forward : grid = FFT_K( pad_end( image * smaps * scaling_coef * scale ) )    (unnormalised)
 //   adjoint : image = sum_c crop( IFFT_K(grid) ) * conj(scaling_coef) * conj(smaps_c) * scale
 // as a sequence of one-dimensional passes over memory:
@@ -25,6 +24,9 @@
 // barriers at length 640) and twiddles evaluated by each group took 69 and 57, 92 and 92,
 // 148 us.  What is left over the copy's time is the butterflies' arithmetic (about 15
 // instructions per element and stage) that three groups per CU do not hide completely.
+// Grid sizes whose prime factors are 2, 3 and 5 have compiled or runtime plans of these
+// radices; the primes 7 to 17 add runtime butterflies of their own size, and a dimension with
+// a larger prime is transformed as a convolution (chirp kernels below).
 // Twiddles (double precision rounded to float) are put into LDS while the first stage's
 // loads are in flight.  Only the forward transform is coded: the inverse swaps real and
 // imaginary parts on the way in and out.
@@ -38,12 +40,12 @@ constexpr int kMaxStages = 6;
 // radices of a length
 // ---------------------------------------------------------------------------
 struct RadixList {
-  int n;  // stages; 0: a prime factor other than 2, 3, 5
+  int n;  // stages; 0: a prime factor above 17
   int r[kMaxStages];
 };
 
-constexpr int kNumRadices = 10;
-constexpr int kRadices[kNumRadices] = {16, 12, 10, 9, 8, 6, 5, 4, 3, 2};
+constexpr int kNumRadices = 14;
+constexpr int kRadices[kNumRadices] = {17, 16, 13, 12, 11, 10, 9, 8, 7, 6, 5, 4, 3, 2};
 
 // the shortest product of radices (in descending order) equal to K; among those of one
 // length, the one whose smallest radix is largest (fewest butterflies, so fewest threads)
@@ -258,7 +260,7 @@ __device__ __forceinline__ void dft(float2* x) {
     x[6] = csub(e[2], o2);
     x[3] = cadd(e[3], o3);
     x[7] = csub(e[3], o3);
-  } else if constexpr (R == 3 || R == 5) {
+  } else if constexpr (R == 3 || R == 5 || R == 7 || R == 11 || R == 13 || R == 17) {
     dft_prime<R>(x);
   } else if constexpr (R == 6) {
     dft_ab<2, 3>(x);
@@ -539,13 +541,19 @@ __device__ __forceinline__ void dit_stage(const Len& len, S s, const Map& map, i
   }
 }
 
+// (KC < 0: a runtime plan with primes above 5; their butterflies cost the other sizes'
+// kernels registers: 167 -> 215 in the first pass)
 #define TKBN_FOR_RADIX(r, CALL)                                                                   \
   switch (r) {                                                                                    \
+    case 17: if constexpr (KC < 0) { CALL(17); } break;                                           \
     case 16: CALL(16); break;                                                                     \
+    case 13: if constexpr (KC < 0) { CALL(13); } break;                                           \
     case 12: CALL(12); break;                                                                     \
+    case 11: if constexpr (KC < 0) { CALL(11); } break;                                           \
     case 10: CALL(10); break;                                                                     \
     case 9: CALL(9); break;                                                                       \
     case 8: CALL(8); break;                                                                       \
+    case 7: if constexpr (KC < 0) { CALL(7); } break;                                             \
     case 6: CALL(6); break;                                                                       \
     case 5: CALL(5); break;                                                                       \
     case 4: CALL(4); break;                                                                       \
@@ -604,7 +612,7 @@ __device__ __forceinline__ void dif_head_c(const FftPlan1D& pl, const Map& map, 
     dif_head_c<KC, HIN, S + 1>(pl, map, nl, buf, tw, tid, load, fill);
   }
 }
-template <class Map, class LoadF>
+template <int KC, class Map, class LoadF>
 __device__ __forceinline__ void dif_head_d(const FftPlan1D& pl, const Map& map, int nl, float2* buf,
                                            float2* tw, int tid, LoadF load, bool fill) {
   if (fill) fill_twiddles<0>(tw, pl);
@@ -638,7 +646,7 @@ __device__ __forceinline__ void dif_fft(const FftPlan1D& pl, const Map& map, int
     dif_stage<Len::L.r[Len::n - 1], false, true, false, HOUT, KC>(pl, Len{}, Int<Len::n - 1>{}, map, nl, buf, tw,
                                                                       tid, NoLoad{}, false, store);
   } else {
-    dif_head_d(pl, map, nl, buf, tw, tid, load, fill);
+    dif_head_d<KC>(pl, map, nl, buf, tw, tid, load, fill);
     const int s = pl.n - 1;
     const DynLen len(pl, s);
 #define TKBN_CALL(R) \
@@ -670,7 +678,7 @@ __device__ __forceinline__ void dif_dit(const FftPlan1D& pl, const Map& map, int
     dit_stage<Len::L.r[Len::n - 1], true, false, false>(Len{}, Int<Len::n - 1>{}, map, nl, buf, tw, tid, mid, drop);
     dit_tail_c<KC, HOUT, Len::n - 2>(map, nl, buf, tw, tid, store);
   } else {
-    dif_head_d(pl, map, nl, buf, tw, tid, load, fill);
+    dif_head_d<KC>(pl, map, nl, buf, tw, tid, load, fill);
     {
       const DynLen len(pl, pl.n - 1);
 #define TKBN_CALL(R) dit_stage<R, true, false, false>(len, pl.n - 1, map, nl, buf, tw, tid, mid, drop)
@@ -707,6 +715,7 @@ struct FftGeom {
 };
 struct FftPlans {
   FftPlan1D d[3];
+  int chirp_m[3];  // convolution length of a dimension whose extent has no plan, else 0
 };
 
 constexpr int kFftMaxThreads = 1024;
@@ -775,7 +784,7 @@ struct ImageLoad {
 
 // The runtime form of MODE 0 holds up to three operands of 16 values: 512 threads leave it
 // the registers.
-constexpr int last_max_threads(int mode, int kc) { return mode == 0 && kc == 0 ? 512 : kFftMaxThreads; }
+constexpr int last_max_threads(int mode, int kc) { return mode == 0 && kc <= 0 ? 512 : kFftMaxThreads; }
 // KC > 0: the last grid extent is KC and 2 N <= KC (compiled passes, halved first or last stage).
 template <int MODE, int KC>
 __global__ void __launch_bounds__((last_max_threads(MODE, KC)))
@@ -906,7 +915,7 @@ __global__ void __launch_bounds__(kFftMaxThreads)
   const float2* s = src + row * (int64_t)n_in * inner + col0;
   float2* o = dst + row * (int64_t)n_out * inner + col0;
   dif_fft<KC, !INV, INV>(
-      pl, LdsMap<true, KC != 0 ? cols_log2(KC) : -1>{lgc, 0}, ncol, buf, tw, threadIdx.x,
+      pl, LdsMap<true, (KC > 0 ? cols_log2(KC) : -1)>{lgc, 0}, ncol, buf, tw, threadIdx.x,
       ColLoad{s, inner, n_in, nc, swap},
       true,
       [&](int f, int t, float2 v, int) {
@@ -950,7 +959,7 @@ __global__ void __launch_bounds__(kFftMaxThreads)
   const int64_t K = KC > 0 ? KC : pl.K;
   const float2* kr = kern + (rows_per_kern > 0 ? row / rows_per_kern : 0) * K * inner + col0;
   dif_dit<KC, true, true>(
-      pl, LdsMap<true, KC != 0 ? cols_log2(KC) : -1>{lgc, 0}, ncol, buf, tw, threadIdx.x,
+      pl, LdsMap<true, (KC > 0 ? cols_log2(KC) : -1)>{lgc, 0}, ncol, buf, tw, threadIdx.x,
       ColLoad{d, inner, n, nc, false},
       true,
       KernelMul{kr, inner, nc},
@@ -960,8 +969,196 @@ __global__ void __launch_bounds__(kFftMaxThreads)
 }
 
 // ---------------------------------------------------------------------------
+// A length K with a prime factor above 17, as a convolution (Bluestein, "A linear filtering approach to the
+// computation of discrete Fourier transform", 1970): with c[n] = exp(-i pi n^2 / K),
+//   X[k] = c[k] sum_n (x[n] c[n]) conj(c[k - n]),
+// a circular convolution of length M >= n_in + n_out - 1, M one of the compiled lengths.  A
+// group transforms its lines to length M, multiplies by the spectrum H of conj(c) and
+// transforms back, all in LDS (dif_dit); the zero padding, the crop and the apodisation
+// cost no pass of their own.  Bound as the passes above by LDS and memory together; the two
+// transforms of 1.3 to 2 K values take about three times the LDS work of a smooth length.
+// 39 images, 217 x 181 -> 434 x 362 (2 * 7 * 31 and 2 * 181; M = 768 and 576), forward and
+// adjoint: row passes 28 and 24 us, column passes 42 and 43 us, chirps 7 us a call, against
+// 219 us each way for the pad or crop kernel, rocFFT's own convolutions of the unpruned grid
+// and its transposes.
+// c and H are written by one small kernel of the same call (chirp_prep_kernel), evaluated in
+// double and rounded once.
+// ---------------------------------------------------------------------------
+constexpr int kMaxChirpM = 1280;  // chirp_prep_kernel's LDS
+
+struct ChirpDim {
+  int K, M, n_in, n_out;
+  float2 *c, *h;
+};
+struct ChirpDims {
+  ChirpDim d[3];
+};
+
+// blockIdx.y: dimension.  A block sums 32 values of H, 32 threads each.
+__global__ void __launch_bounds__(1024) chirp_prep_kernel(const ChirpDims dims) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  __shared__ double2 part[32][33];
+  const ChirpDim q = blockIdx.y == 0 ? dims.d[0] : blockIdx.y == 1 ? dims.d[1] : dims.d[2];
+  const int f0 = blockIdx.x * 32;
+  if (f0 >= q.M) return;
+  double2* const w = reinterpret_cast<double2*>(smem);  // exp(-2 pi i p / M)
+  double2* const h = w + q.M;                           // conj(c) around the circle
+  const auto chirp = [&](int n) {  // exp(i pi n^2 / K)
+    double s, c;
+    sincospi((double)((int64_t)n * n % (2 * q.K)) / (double)q.K, &s, &c);
+    return make_double2(c, s);
+  };
+  for (int p = threadIdx.x; p < q.M; p += blockDim.x) {
+    double s, c;
+    sincospi(2. * (double)p / (double)q.M, &s, &c);
+    w[p] = make_double2(c, -s);
+    h[p] = p < q.n_out ? chirp(p) : p > q.M - q.n_in ? chirp(q.M - p) : make_double2(0., 0.);
+  }
+  if (threadIdx.x < 32 && f0 + (int)threadIdx.x < q.K) {
+    const double2 e = chirp(f0 + threadIdx.x);
+    q.c[f0 + threadIdx.x] = make_float2((float)e.x, (float)-e.y);
+  }
+  __syncthreads();
+  const int o = threadIdx.x & 31, r = threadIdx.x >> 5;
+  const int f = f0 + o < q.M ? f0 + o : q.M - 1;
+  int at = f * r % q.M;
+  const int step = f * 32 % q.M;
+  double2 sum = make_double2(0., 0.);
+  for (int p = r; p < q.M; p += 32) {
+    const double2 a = h[p], b = w[at];
+    sum.x += a.x * b.x - a.y * b.y;
+    sum.y += a.x * b.y + a.y * b.x;
+    at += step;
+    if (at >= q.M) at -= q.M;
+  }
+  part[r][o] = sum;
+  __syncthreads();
+  if (r == 0 && f0 + o < q.M) {
+    for (int k = 1; k < 32; ++k) {
+      sum.x += part[k][o].x;
+      sum.y += part[k][o].y;
+    }
+    q.h[f] = make_float2((float)(sum.x / q.M), (float)(sum.y / q.M));
+  }
+}
+
+// a source times the chirp
+template <class Load>
+struct ChirpLoad {
+  Load l;
+  const float2* c;
+  int n;
+  struct Raw {
+    typename Load::Raw v;
+    float2 c;
+  };
+  __device__ __forceinline__ Raw read(int k, int t) const {
+    Raw r;
+    r.v = l.read(k, t);
+    r.c = c[k < n ? k : 0];
+    return r;
+  }
+  __device__ __forceinline__ float2 value(const Raw& r, int k, int t) const { return cmul(l.value(r.v, k, t), r.c); }
+};
+// line t of consecutive lines of n values, real and imaginary exchanged, zeros past the end
+struct PaddedLineLoad {
+  const float2* s;
+  int n;
+  using Raw = float2;
+  __device__ __forceinline__ Raw read(int k, int t) const { return s[(int64_t)t * n + (k < n ? k : 0)]; }
+  __device__ __forceinline__ float2 value(Raw v, int k, int) const { return k < n ? cswap(v) : make_float2(0.f, 0.f); }
+};
+// times the spectrum, real and imaginary exchanged for the way back
+struct SpectrumMul {
+  const float2* h;
+  __device__ __forceinline__ float2 read(int f, int) const { return h[f]; }
+  __device__ __forceinline__ float2 value(float2 m, float2 v) const { return cswap(cmul(v, m)); }
+};
+
+// KC > 0: M = KC, of which the first half takes all inputs (forward) or outputs (inverse)
+constexpr int chirp_max_threads(bool inv) { return inv ? kFftMaxThreads : 512; }
+template <bool INV, int KC>
+__global__ void __launch_bounds__((chirp_max_threads(INV)))
+    chirp_last_kernel(const FftGeom g, const FftPlan1D pl, const ChirpDim cd, const float2* __restrict__ src,
+                      const float2* __restrict__ smaps, const float2* __restrict__ scaling, float2* __restrict__ dst,
+                      int lpg) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int D = g.ndim;
+  const int M = KC > 0 ? KC : pl.K, N = g.N[D - 1], K = cd.K;
+  const LdsMap<false> map{0, KC > 0 ? M + StaticLen<KC>::L.r[0] : M + pl.r[0]};
+  float2* tw = reinterpret_cast<float2*>(smem);
+  float2* buf = tw + pl.ntw;
+  const float2* const c = cd.c;
+  int64_t Q = 1;
+  for (int d = 0; d < D - 1; ++d) Q *= g.N[d];
+  const int64_t line0 = (int64_t)blockIdx.x * lpg;
+  const int64_t nlines = g.B * g.C * Q;
+  const int nl = (int)(line0 + lpg <= nlines ? lpg : nlines - line0);
+  if constexpr (!INV) {
+    dif_dit<KC, true, false>(
+        pl, map, nl, buf, tw, threadIdx.x,
+        ChirpLoad<ImageLoad>{ImageLoad{g, src, smaps, scaling, line0, Q, Q * N, N}, c, N}, true, SpectrumMul{cd.h},
+        [&](int k, int t, float2 v) {
+          if (k < K) dst[(line0 + t) * K + k] = cmul(cswap(v), c[k]);
+        });
+  } else {
+    dif_dit<KC, false, true>(
+        pl, map, nl, buf, tw, threadIdx.x, ChirpLoad<PaddedLineLoad>{PaddedLineLoad{src + line0 * K, K}, c, K}, true,
+        SpectrumMul{cd.h}, [&](int k, int t, float2 v) {
+          if (k < N) {
+            v = cswap(cmul(cswap(v), c[k]));
+            if (scaling) {
+              const uint32_t line = (uint32_t)(line0 + t);
+              const int64_t q = line - fdiv(line, g.fQ) * (uint32_t)Q;
+              v = cmul_conj(v, scaling[q * N + k]);
+            }
+            v.x *= g.scale;
+            v.y *= g.scale;
+            dst[(line0 + t) * N + k] = v;
+          }
+        });
+  }
+}
+
+template <bool INV, int KC>
+__global__ void __launch_bounds__(kFftMaxThreads)
+    chirp_mid_kernel(const FftPlan1D pl, const ChirpDim cd, int64_t rows, int64_t inner, int lgc,
+                     const float2* __restrict__ src, float2* __restrict__ dst) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  float2* tw = reinterpret_cast<float2*>(smem);
+  float2* buf = tw + pl.ntw;
+  const float2* const c = cd.c;
+  const int lg = KC > 0 ? cols_log2(KC) : lgc;
+  const int ncol = 1 << lg;
+  const int64_t item = xcd_contiguous_item();
+  const int64_t chunks = (inner + ncol - 1) >> lg;
+  const int64_t row = item / chunks;
+  const int64_t col0 = (item - row * chunks) << lg;
+  if (row >= rows) return;
+  const int nc = (int)(col0 + ncol <= inner ? ncol : inner - col0);
+  const float2* s = src + row * (int64_t)cd.n_in * inner + col0;
+  float2* o = dst + row * (int64_t)cd.n_out * inner + col0;
+  const int n_out = cd.n_out;
+  dif_dit<KC, !INV, INV>(
+      pl, LdsMap<true, (KC > 0 ? cols_log2(KC) : -1)>{lgc, 0}, ncol, buf, tw, threadIdx.x,
+      ChirpLoad<ColLoad>{ColLoad{s, inner, cd.n_in, nc, INV}, c, cd.n_in}, true, SpectrumMul{cd.h},
+      [&](int k, int t, float2 v) {
+        if (k < n_out && t < nc) {
+          v = cmul(cswap(v), c[k]);
+          o[(int64_t)k * inner + t] = INV ? cswap(v) : v;
+        }
+      });
+}
+
+// ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
+static bool smooth5(int64_t n) {
+  for (int p : {2, 3, 5})
+    while (n % p == 0) n /= p;
+  return n == 1;
+}
+
 static bool factorize(int K, FftPlan1D* pl) {
   const RadixList L = radix_list(K);
   if (L.n == 0) return false;
@@ -1002,7 +1199,20 @@ static int fft_lines(const FftPlan1D& pl, int64_t total) {
 }
 constexpr int kMaxK = 2048;
 
-static int check_fft(int32_t ndim, const int64_t* im, const int64_t* gs, FftGeom* g, FftPlans* plans) {
+// Lengths of the convolutions: all but the last two are compiled.
+#define TKBN_CHIRP_COMPILED_SIZES(X) X(192) X(256) X(320) X(384) X(480) X(576) X(640) X(768) X(1024)
+static int chirp_length(int need) {
+#define TKBN_CHIRP_FIT(M) \
+  if (need <= M) return M;
+  TKBN_CHIRP_COMPILED_SIZES(TKBN_CHIRP_FIT)
+#undef TKBN_CHIRP_FIT
+  return need <= 1152 ? 1152 : kMaxChirpM;
+}
+
+// `any`: extents may hold the primes 7 to 17 too (butterflies of those sizes in the runtime
+// plan: a convolution was up to 1.6 times further from 64-bit values, 63^2 -> 126^2 adjoint
+// 2.41e-7 against 1.51e-7), and any larger one (the convolution)
+static int check_fft(int32_t ndim, const int64_t* im, const int64_t* gs, FftGeom* g, FftPlans* plans, bool any) {
   TKBN_REQUIRE(ndim >= 1 && ndim <= 3, TKBN_ERR_UNSUPPORTED, "ndim %d not in 1..3", ndim);
   TKBN_REQUIRE(im && gs, TKBN_ERR_INVALID, "NULL size array");
   g->ndim = ndim;
@@ -1012,8 +1222,15 @@ static int check_fft(int32_t ndim, const int64_t* im, const int64_t* gs, FftGeom
   }
   for (int d = 0; d < ndim; ++d) {
     TKBN_REQUIRE(im[d] >= 1 && gs[d] >= im[d], TKBN_ERR_INVALID, "dim %d: need 1 <= im_size <= grid_size", d);
-    TKBN_REQUIRE(gs[d] <= kMaxK && factorize((int)gs[d], &plans->d[d]), TKBN_ERR_UNSUPPORTED,
+    plans->chirp_m[d] = 0;
+    TKBN_REQUIRE(any || (gs[d] <= kMaxK && smooth5(gs[d])), TKBN_ERR_UNSUPPORTED,
                  "grid size %lld is not a product of 2, 3, 5 up to %d", (long long)gs[d], kMaxK);
+    if (!(gs[d] <= kMaxK && factorize((int)gs[d], &plans->d[d]))) {
+      TKBN_REQUIRE(im[d] + gs[d] - 1 <= kMaxChirpM, TKBN_ERR_UNSUPPORTED,
+                   "grid size %lld needs a convolution of more than %d values", (long long)gs[d], kMaxChirpM);
+      plans->chirp_m[d] = chirp_length((int)(im[d] + gs[d] - 1));
+      TKBN_REQUIRE(factorize(plans->chirp_m[d], &plans->d[d]), TKBN_ERR_UNSUPPORTED, "no convolution length");
+    }
     g->N[d] = (int)im[d];
     g->K[d] = (int)gs[d];
   }
@@ -1057,7 +1274,7 @@ static int launch_last(const FftGeom& g, const FftPlan1D& pl, const float2* src,
     lpg = fft_lines(pl, g.B * g.C * Q);
     groups = ceil_div(g.B * g.C * Q, lpg);
   }
-  const int kc = 2 * g.N[D - 1] <= pl.K ? pl.K : 0;  // compiled, if in the list below
+  const int kc = !smooth5(pl.K) ? -1 : 2 * g.N[D - 1] <= pl.K ? pl.K : 0;  // compiled, if in the list below
   unsigned threads = fft_threads(pl, lpg, MODE == 1 ? g.N[D - 1] : 0);
   const size_t lds = (size_t)fft_lds_bytes(pl.K, lpg);
   const dim3 grid((unsigned)groups), block(threads);
@@ -1068,6 +1285,10 @@ static int launch_last(const FftGeom& g, const FftPlan1D& pl, const float2* src,
     break;
     TKBN_FFT_COMPILED_SIZES(TKBN_LAST)
 #undef TKBN_LAST
+    case -1:
+      threads = threads < (unsigned)last_max_threads(MODE, -1) ? threads : (unsigned)last_max_threads(MODE, -1);
+      fft_last_kernel<MODE, -1><<<grid, dim3(threads), lds, s>>>(g, pl, src, smaps, scaling, dst, lpg);
+      break;
     default:
       threads = threads < (unsigned)last_max_threads(MODE, 0) ? threads : (unsigned)last_max_threads(MODE, 0);
       fft_last_kernel<MODE, 0><<<grid, dim3(threads), lds, s>>>(g, pl, src, smaps, scaling, dst, lpg);
@@ -1083,7 +1304,7 @@ static int launch_mid(bool inv, const FftPlan1D& pl, int64_t rows, int n_in, int
   TKBN_REQUIRE(groups < (1LL << 31), TKBN_ERR_INVALID, "too many FFT columns");
   const size_t lds = (size_t)fft_lds_bytes(pl.K, 1 << lgc);
   const dim3 grid((unsigned)groups), block(fft_threads(pl, 1 << lgc, 0));
-  switch (2 * (inv ? n_out : n_in) <= pl.K ? pl.K : 0) {
+  switch (!smooth5(pl.K) ? -1 : 2 * (inv ? n_out : n_in) <= pl.K ? pl.K : 0) {
 #define TKBN_MID(KV)                                                                                            \
   case KV:                                                                                                      \
     if (inv)                                                                                                    \
@@ -1093,6 +1314,9 @@ static int launch_mid(bool inv, const FftPlan1D& pl, int64_t rows, int n_in, int
     break;
     TKBN_FFT_COMPILED_SIZES(TKBN_MID)
 #undef TKBN_MID
+    case -1:
+      fft_mid_kernel<false, -1><<<grid, block, lds, s>>>(pl, rows, n_in, n_out, inner, lgc, inv ? 1 : 0, src, dst);
+      break;
     default:
       fft_mid_kernel<false, 0><<<grid, block, lds, s>>>(pl, rows, n_in, n_out, inner, lgc, inv ? 1 : 0, src, dst);
   }
@@ -1121,6 +1345,73 @@ static int launch_filter(const FftPlan1D& pl, int64_t rows, int n, int64_t inner
   return TKBN_OK;
 }
 
+// Lines of the last dimension: as many as fft_lines says of their convolutions.
+template <bool INV>
+static int launch_chirp_last(const FftGeom& g, const FftPlan1D& pl, const ChirpDim& cd, const float2* src,
+                             const float2* smaps, const float2* scaling, float2* dst, hipStream_t s) {
+  int64_t Q = 1;
+  for (int d = 0; d < g.ndim - 1; ++d) Q *= g.N[d];
+  const int lpg = fft_lines(pl, g.B * g.C * Q);
+  unsigned threads = fft_threads(pl, lpg, 0);
+  threads = threads < (unsigned)chirp_max_threads(INV) ? threads : (unsigned)chirp_max_threads(INV);
+  const size_t lds = (size_t)fft_lds_bytes(pl.K, lpg);
+  const dim3 grid((unsigned)ceil_div(g.B * g.C * Q, lpg)), block(threads);
+  switch (cd.M) {
+#define TKBN_CHIRP(MV)                                                                                       \
+  case MV: chirp_last_kernel<INV, MV><<<grid, block, lds, s>>>(g, pl, cd, src, smaps, scaling, dst, lpg); break;
+    TKBN_CHIRP_COMPILED_SIZES(TKBN_CHIRP)
+#undef TKBN_CHIRP
+    default: chirp_last_kernel<INV, 0><<<grid, block, lds, s>>>(g, pl, cd, src, smaps, scaling, dst, lpg);
+  }
+  TKBN_LAUNCH_CHECK("chirp_last_kernel");
+  return TKBN_OK;
+}
+
+template <bool INV>
+static int launch_chirp_mid(const FftPlan1D& pl, const ChirpDim& cd, int64_t rows, int64_t inner, const float2* src,
+                            float2* dst, hipStream_t s) {
+  const int lgc = cols_log2(pl.K);
+  const int64_t groups = ceil_div(rows * ceil_div(inner, 1 << lgc), 8) * 8;  // see xcd_contiguous_item
+  TKBN_REQUIRE(groups < (1LL << 31), TKBN_ERR_INVALID, "too many FFT columns");
+  const size_t lds = (size_t)fft_lds_bytes(pl.K, 1 << lgc);
+  const dim3 grid((unsigned)groups), block(fft_threads(pl, 1 << lgc, 0));
+  switch (cd.M) {
+#define TKBN_CHIRP(MV) \
+  case MV: chirp_mid_kernel<INV, MV><<<grid, block, lds, s>>>(pl, cd, rows, inner, lgc, src, dst); break;
+    TKBN_CHIRP_COMPILED_SIZES(TKBN_CHIRP)
+#undef TKBN_CHIRP
+    default: chirp_mid_kernel<INV, 0><<<grid, block, lds, s>>>(pl, cd, rows, inner, lgc, src, dst);
+  }
+  TKBN_LAUNCH_CHECK("chirp_mid_kernel");
+  return TKBN_OK;
+}
+
+// elements of the chirps and spectra
+static int64_t chirp_elements(const FftGeom& g, const FftPlans& plans) {
+  int64_t n = 0;
+  for (int d = 0; d < g.ndim; ++d)
+    if (plans.chirp_m[d]) n += g.K[d] + plans.chirp_m[d];
+  return n;
+}
+// lays them out at `p` and fills them
+static int launch_chirp_prep(const FftGeom& g, const FftPlans& plans, bool inv, float2* p, ChirpDim (&cd)[3],
+                             hipStream_t s) {
+  ChirpDims dims{};
+  int n = 0, mmax = 0;
+  for (int d = 0; d < g.ndim; ++d) {
+    const int M = plans.chirp_m[d];
+    if (!M) continue;
+    cd[d] = ChirpDim{g.K[d], M, inv ? g.K[d] : g.N[d], inv ? g.N[d] : g.K[d], p, p + g.K[d]};
+    p += g.K[d] + M;
+    dims.d[n++] = cd[d];
+    mmax = M > mmax ? M : mmax;
+  }
+  if (n == 0) return TKBN_OK;
+  chirp_prep_kernel<<<dim3((unsigned)ceil_div(mmax, 32), (unsigned)n), dim3(1024), (size_t)mmax * 32, s>>>(dims);
+  TKBN_LAUNCH_CHECK("chirp_prep_kernel");
+  return TKBN_OK;
+}
+
 // elements of the intermediate after the last-dim pass (forward) / before it (adjoint),
 // and after/before each middle pass; ws holds two ping-pong buffers
 static void ws_sizes(const FftGeom& g, int64_t* a, int64_t* b) {
@@ -1142,38 +1433,32 @@ static void ws_sizes(const FftGeom& g, int64_t* a, int64_t* b) {
   *b = idx > 1 ? sz[1] : 0;
 }
 
-}  // namespace tkbn
-
-using namespace tkbn;
-
-extern "C" {
-
-int tkbn_fft_supported(int32_t ndim, const int64_t* im_size, const int64_t* grid_size) {
+static int fft_supported(int32_t ndim, const int64_t* im_size, const int64_t* grid_size, bool any) {
   FftGeom g;
   FftPlans plans;
-  return check_fft(ndim, im_size, grid_size, &g, &plans);
+  return check_fft(ndim, im_size, grid_size, &g, &plans, any);
 }
 
-int64_t tkbn_fft_workspace_bytes(int32_t ndim, const int64_t* im_size, const int64_t* grid_size, int64_t batch,
-                                 int64_t coils) {
+static int64_t fft_workspace_bytes(int32_t ndim, const int64_t* im_size, const int64_t* grid_size, int64_t batch,
+                                   int64_t coils, bool any) {
   FftGeom g;
   FftPlans plans;
-  if (check_fft(ndim, im_size, grid_size, &g, &plans) != TKBN_OK) return -1;
+  if (check_fft(ndim, im_size, grid_size, &g, &plans, any) != TKBN_OK) return -1;
   g.B = batch;
   g.C = coils;
   int64_t a, b;
   ws_sizes(g, &a, &b);
-  return (a + b) * 8 + 256;
+  return (a + b + chirp_elements(g, plans)) * 8 + 256;
 }
 
-int tkbn_fft_grid_fwd(int32_t dtype, int32_t ndim, const int64_t* im_size, const int64_t* grid_size, int64_t batch,
+static int fft_grid_fwd(bool any, int32_t dtype, int32_t ndim, const int64_t* im_size, const int64_t* grid_size, int64_t batch,
                       int64_t coils, int64_t image_coils, const void* image, const void* smaps,
                       const void* scaling_coef, double scale, void* grid, void* workspace, int64_t workspace_bytes,
                       void* stream) {
   FftGeom g;
   FftPlans plans;
   TKBN_REQUIRE(dtype == TKBN_F32, TKBN_ERR_UNSUPPORTED, "fused FFT is complex64 only");
-  int st = check_fft(ndim, im_size, grid_size, &g, &plans);
+  int st = check_fft(ndim, im_size, grid_size, &g, &plans, any);
   if (st != TKBN_OK) return st;
   TKBN_REQUIRE(batch >= 0 && coils >= 0, TKBN_ERR_INVALID, "negative batch/coils");
   TKBN_REQUIRE(image_coils == 1 || image_coils == coils, TKBN_ERR_INVALID, "image_coils must be 1 or coils");
@@ -1189,15 +1474,22 @@ int tkbn_fft_grid_fwd(int32_t dtype, int32_t ndim, const int64_t* im_size, const
   if (st != TKBN_OK) return st;
   int64_t wa, wb;
   ws_sizes(g, &wa, &wb);
-  TKBN_REQUIRE(workspace_bytes >= (wa + wb) * 8 && (wa + wb == 0 || workspace), TKBN_ERR_WORKSPACE,
-               "workspace of %lld bytes needed", (long long)((wa + wb) * 8));
+  const int64_t need = (wa + wb + chirp_elements(g, plans)) * 8;
+  TKBN_REQUIRE(workspace_bytes >= need && (need == 0 || workspace), TKBN_ERR_WORKSPACE,
+               "workspace of %lld bytes needed", (long long)need);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int D = ndim;
   float2* bufa = static_cast<float2*>(workspace);
   float2* bufb = bufa + wa;
+  ChirpDim cd[3];
+  st = launch_chirp_prep(g, plans, false, bufb + wb, cd, s);
+  if (st != TKBN_OK) return st;
   // pass 1: last dimension with fused apodisation / SENSE / zero-pad
-  st = launch_last<0>(g, plans.d[D - 1], static_cast<const float2*>(image), static_cast<const float2*>(smaps),
-                      static_cast<const float2*>(scaling_coef), D == 1 ? static_cast<float2*>(grid) : bufa, s);
+  const float2 *im = static_cast<const float2*>(image), *sm = static_cast<const float2*>(smaps),
+               *sc = static_cast<const float2*>(scaling_coef);
+  float2* first = D == 1 ? static_cast<float2*>(grid) : bufa;
+  st = plans.chirp_m[D - 1] ? launch_chirp_last<false>(g, plans.d[D - 1], cd[D - 1], im, sm, sc, first, s)
+                            : launch_last<0>(g, plans.d[D - 1], im, sm, sc, first, s);
   if (st != TKBN_OK) return st;
   // remaining dimensions, innermost first
   int e[3];
@@ -1209,7 +1501,8 @@ int tkbn_fft_grid_fwd(int32_t dtype, int32_t ndim, const int64_t* im_size, const
     for (int k = 0; k < d; ++k) outer *= e[k];
     for (int k = d + 1; k < D; ++k) inner *= e[k];
     float2* out = d == 0 ? static_cast<float2*>(grid) : (cur == bufa ? bufb : bufa);
-    st = launch_mid(false, plans.d[d], outer, g.N[d], g.K[d], inner, cur, out, s);
+    st = plans.chirp_m[d] ? launch_chirp_mid<false>(plans.d[d], cd[d], outer, inner, cur, out, s)
+                          : launch_mid(false, plans.d[d], outer, g.N[d], g.K[d], inner, cur, out, s);
     if (st != TKBN_OK) return st;
     e[d] = g.K[d];
     cur = out;
@@ -1217,17 +1510,17 @@ int tkbn_fft_grid_fwd(int32_t dtype, int32_t ndim, const int64_t* im_size, const
   return TKBN_OK;
 }
 
-int tkbn_fft_grid_adj(int32_t dtype, int32_t ndim, const int64_t* im_size, const int64_t* grid_size, int64_t batch,
+static int fft_grid_adj(bool any, int32_t dtype, int32_t ndim, const int64_t* im_size, const int64_t* grid_size, int64_t batch,
                       int64_t coils, const void* grid, const void* smaps, const void* scaling_coef, double scale,
                       void* image, void* workspace, int64_t workspace_bytes, void* stream) {
   FftGeom g;
   FftPlans plans;
   TKBN_REQUIRE(dtype == TKBN_F32, TKBN_ERR_UNSUPPORTED, "fused FFT is complex64 only");
-  int st = check_fft(ndim, im_size, grid_size, &g, &plans);
+  int st = check_fft(ndim, im_size, grid_size, &g, &plans, any);
   if (st != TKBN_OK) return st;
   TKBN_REQUIRE(batch >= 0 && coils >= 0, TKBN_ERR_INVALID, "negative batch/coils");
   if (batch == 0 || coils == 0) return TKBN_OK;
-  TKBN_REQUIRE(grid && scaling_coef && image, TKBN_ERR_INVALID, "NULL data pointer");
+  TKBN_REQUIRE(grid && (any || scaling_coef) && image, TKBN_ERR_INVALID, "NULL data pointer");
   g.B = batch;
   g.C = coils;
   g.image_coils = (int)coils;
@@ -1237,12 +1530,18 @@ int tkbn_fft_grid_adj(int32_t dtype, int32_t ndim, const int64_t* im_size, const
   if (st != TKBN_OK) return st;
   int64_t wa, wb;
   ws_sizes(g, &wa, &wb);
-  TKBN_REQUIRE(workspace_bytes >= (wa + wb) * 8 && (wa + wb == 0 || workspace), TKBN_ERR_WORKSPACE,
-               "workspace of %lld bytes needed", (long long)((wa + wb) * 8));
+  const int64_t need = (wa + wb + chirp_elements(g, plans)) * 8;
+  TKBN_REQUIRE(workspace_bytes >= need && (need == 0 || workspace), TKBN_ERR_WORKSPACE,
+               "workspace of %lld bytes needed", (long long)need);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int D = ndim;
   float2* bufa = static_cast<float2*>(workspace);
   float2* bufb = bufa + wa;
+  TKBN_REQUIRE(!(smaps && plans.chirp_m[D - 1]), TKBN_ERR_UNSUPPORTED,
+               "coil maps need a last grid size without prime factors above 17");
+  ChirpDim cd[3];
+  st = launch_chirp_prep(g, plans, true, bufb + wb, cd, s);
+  if (st != TKBN_OK) return st;
   // outer dimensions first (inverse, cropping), mirror of the forward sequence
   int e[3];
   for (int d = 0; d < D; ++d) e[d] = g.K[d];
@@ -1255,7 +1554,8 @@ int tkbn_fft_grid_adj(int32_t dtype, int32_t ndim, const int64_t* im_size, const
     // choose the buffer so that the last middle pass lands in bufa
     const int remaining = (D - 2) - d;  // passes after this one
     float2* out = (remaining % 2 == 0) ? bufa : bufb;
-    st = launch_mid(true, plans.d[d], outer, g.K[d], g.N[d], inner, cur, out, s);
+    st = plans.chirp_m[d] ? launch_chirp_mid<true>(plans.d[d], cd[d], outer, inner, cur, out, s)
+                          : launch_mid(true, plans.d[d], outer, g.K[d], g.N[d], inner, cur, out, s);
     if (st != TKBN_OK) return st;
     e[d] = g.N[d];
     cur = out;
@@ -1263,7 +1563,57 @@ int tkbn_fft_grid_adj(int32_t dtype, int32_t ndim, const int64_t* im_size, const
   if (smaps)
     return launch_last<1>(g, plans.d[D - 1], cur, static_cast<const float2*>(smaps), static_cast<const float2*>(scaling_coef),
                           static_cast<float2*>(image), s);
+  if (plans.chirp_m[D - 1])
+    return launch_chirp_last<true>(g, plans.d[D - 1], cd[D - 1], cur, nullptr, static_cast<const float2*>(scaling_coef),
+                                   static_cast<float2*>(image), s);
   return launch_last<2>(g, plans.d[D - 1], cur, nullptr, static_cast<const float2*>(scaling_coef), static_cast<float2*>(image), s);
+}
+
+}  // namespace tkbn
+
+using namespace tkbn;
+
+extern "C" {
+
+int tkbn_fft_supported(int32_t ndim, const int64_t* im_size, const int64_t* grid_size) {
+  return fft_supported(ndim, im_size, grid_size, false);
+}
+int tkbn_fft_any_supported(int32_t ndim, const int64_t* im_size, const int64_t* grid_size) {
+  return fft_supported(ndim, im_size, grid_size, true);
+}
+int64_t tkbn_fft_workspace_bytes(int32_t ndim, const int64_t* im_size, const int64_t* grid_size, int64_t batch,
+                                 int64_t coils) {
+  return fft_workspace_bytes(ndim, im_size, grid_size, batch, coils, false);
+}
+int64_t tkbn_fft_any_workspace_bytes(int32_t ndim, const int64_t* im_size, const int64_t* grid_size, int64_t batch,
+                                     int64_t coils) {
+  return fft_workspace_bytes(ndim, im_size, grid_size, batch, coils, true);
+}
+int tkbn_fft_grid_fwd(int32_t dtype, int32_t ndim, const int64_t* im_size, const int64_t* grid_size, int64_t batch,
+                      int64_t coils, int64_t image_coils, const void* image, const void* smaps,
+                      const void* scaling_coef, double scale, void* grid, void* workspace, int64_t workspace_bytes,
+                      void* stream) {
+  return fft_grid_fwd(false, dtype, ndim, im_size, grid_size, batch, coils, image_coils, image, smaps, scaling_coef, scale,
+                      grid, workspace, workspace_bytes, stream);
+}
+int tkbn_fft_grid_adj(int32_t dtype, int32_t ndim, const int64_t* im_size, const int64_t* grid_size, int64_t batch,
+                      int64_t coils, const void* grid, const void* smaps, const void* scaling_coef, double scale,
+                      void* image, void* workspace, int64_t workspace_bytes, void* stream) {
+  return fft_grid_adj(false, dtype, ndim, im_size, grid_size, batch, coils, grid, smaps, scaling_coef, scale, image,
+                      workspace, workspace_bytes, stream);
+}
+int tkbn_fft_any_grid_fwd(int32_t dtype, int32_t ndim, const int64_t* im_size, const int64_t* grid_size, int64_t batch,
+                      int64_t coils, int64_t image_coils, const void* image, const void* smaps,
+                      const void* scaling_coef, double scale, void* grid, void* workspace, int64_t workspace_bytes,
+                      void* stream) {
+  return fft_grid_fwd(true, dtype, ndim, im_size, grid_size, batch, coils, image_coils, image, smaps, scaling_coef, scale,
+                      grid, workspace, workspace_bytes, stream);
+}
+int tkbn_fft_any_grid_adj(int32_t dtype, int32_t ndim, const int64_t* im_size, const int64_t* grid_size, int64_t batch,
+                      int64_t coils, const void* grid, const void* smaps, const void* scaling_coef, double scale,
+                      void* image, void* workspace, int64_t workspace_bytes, void* stream) {
+  return fft_grid_adj(true, dtype, ndim, im_size, grid_size, batch, coils, grid, smaps, scaling_coef, scale, image,
+                      workspace, workspace_bytes, stream);
 }
 
 int tkbn_fft_filter(int32_t dtype, int32_t ndim, const int64_t* im_size, const int64_t* grid_size, int64_t batch,
@@ -1273,7 +1623,7 @@ int tkbn_fft_filter(int32_t dtype, int32_t ndim, const int64_t* im_size, const i
   FftGeom g;
   FftPlans plans;
   TKBN_REQUIRE(dtype == TKBN_F32, TKBN_ERR_UNSUPPORTED, "fused FFT is complex64 only");
-  int st = check_fft(ndim, im_size, grid_size, &g, &plans);
+  int st = check_fft(ndim, im_size, grid_size, &g, &plans, false);
   if (st != TKBN_OK) return st;
   TKBN_REQUIRE(ndim >= 2, TKBN_ERR_UNSUPPORTED, "the fused FFT filter needs at least two dimensions");
   TKBN_REQUIRE(batch >= 0 && coils >= 0, TKBN_ERR_INVALID, "negative batch/coils");

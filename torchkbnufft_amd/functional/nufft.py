@@ -9,14 +9,14 @@ from torch import Tensor
 from .._autograd._apply import run as _run
 from .._autograd.fft import ApodPad, CropDeapod, GridAdjoint, GridForward
 from .._nufft._host import host_values
-from .._nufft.fft import _norm_scale, fused_supported
+from .._nufft.fft import _norm_scale, pipeline_supported
 from .interp import kb_spmat_interp, kb_spmat_interp_adjoint, kb_table_interp, kb_table_interp_adjoint
 
 
 def _to_grid(image, smaps, scaling_coef, im_size, grid_size, norm):
     gs = host_values(grid_size)
     im = host_values(im_size)
-    if fused_supported(image.dtype, im, gs):
+    if pipeline_supported(image.dtype, im, gs):
         return _run(GridForward, image, smaps, scaling_coef, im, gs, _norm_scale(norm, gs))
     grid = _run(ApodPad, image, smaps, scaling_coef, im, gs, _norm_scale(norm, gs))
     return torch.fft.fftn(grid, dim=tuple(range(-len(gs), 0)), norm="backward")
@@ -25,7 +25,7 @@ def _to_grid(image, smaps, scaling_coef, im_size, grid_size, norm):
 def _from_grid(grid, smaps, scaling_coef, im_size, grid_size, norm):
     gs = host_values(grid_size)
     im = host_values(im_size)
-    if fused_supported(grid.dtype, im, gs):
+    if pipeline_supported(grid.dtype, im, gs):
         return _run(GridAdjoint, grid, smaps, scaling_coef, im, _norm_scale(norm, gs))
     grid = torch.fft.ifftn(grid, dim=tuple(range(-len(gs), 0)), norm="forward")
     return _run(CropDeapod, grid, smaps, scaling_coef, im, _norm_scale(norm, gs))
