@@ -78,8 +78,12 @@ constexpr int kLdsBudget = 60 * 1024;
 // 4.4 -> 5.4-6.0 ms with 512-1024).
 // (complex128 and numpoints above 6 keep 256: at 1024 threads their registers spill.)
 constexpr int spread_tiles_threads(int) { return 256; }
-template <typename T, int JM>
-constexpr int fwd_tiled_threads() { return sizeof(T) == 4 && JM <= 6 ? 1024 : 256; }
+// (The 3-D gather's registers leave a CU six waves per SIMD: one group of 1024 threads, which
+// then waits for its own 60 KB of staging, or three of 512, of which LDS holds two, one
+// gathering while the other stages.  320^3, 8 rows, 1.6 M radial samples: 256 threads 2.95 ms,
+// 512 2.47 ms, 1024 2.59 ms.)
+template <typename T, int JM, int D>
+constexpr int fwd_tiled_threads() { return sizeof(T) == 4 && JM <= 6 ? (D == 3 ? 512 : 1024) : 256; }
 
 template <typename T>
 __device__ __forceinline__ int64_t sample_base_wrapped(const Geom<T>& g, int d, T omega) {
@@ -906,7 +910,7 @@ __device__ __forceinline__ void fwd_tiled_item(const Geom<T>& g, const TileGeom&
 }
 
 template <typename T, int D, int JM>
-__global__ void __launch_bounds__((fwd_tiled_threads<T, JM>()))
+__global__ void __launch_bounds__((fwd_tiled_threads<T, JM, D>()))
     interp_fwd_tiled_kernel(const Geom<T> g, const TileGeom tg, const cplx<T>* __restrict__ grid,
                             const T* __restrict__ omega, const int* __restrict__ ws, cplx<T>* __restrict__ kdata) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -3120,7 +3124,7 @@ int fwd_tiled_launch(const Geom<T>& g, const TileGeom& tg, const void* grid, con
   }
   const size_t lds = (size_t)tg.CC * tg.rcells * sizeof(cplx<T>);
   interp_fwd_tiled_kernel<T, D, JM>
-      <<<dim3((unsigned)tg.maxwork, (unsigned)ceil_div(nrows, tg.CC), (unsigned)zdim), dim3(fwd_tiled_threads<T, JM>()),
+      <<<dim3((unsigned)tg.maxwork, (unsigned)ceil_div(nrows, tg.CC), (unsigned)zdim), dim3(fwd_tiled_threads<T, JM, D>()),
          lds, s>>>(g, tg, static_cast<const cplx<T>*>(grid), static_cast<const T*>(omega), ws,
                    static_cast<cplx<T>*>(kdata));
   TKBN_LAUNCH_CHECK("interp_fwd_tiled_kernel");
@@ -3292,7 +3296,7 @@ __device__ __forceinline__ int batch_find(const int* off, int nprob, int item) {
 }
 
 template <int D, int JM>
-__global__ void __launch_bounds__((fwd_tiled_threads<float, JM>()))
+__global__ void __launch_bounds__((fwd_tiled_threads<float, JM, D>()))
     batch_fwd_kernel(const BatchProb* __restrict__ probs, int nprob, const int* __restrict__ off) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   const int item = blockIdx.x;
@@ -3590,7 +3594,7 @@ int tkbn_batch_interp_fwd(const tkbn_batch* b, const void* table, void* workspac
   if (b->bound_f == 0) return TKBN_OK;
   const dim3 grd((unsigned)b->bound_f);
 #define TKBN_BATCH_FWD(DD, JJ) \
-  batch_fwd_kernel<DD, JJ><<<grd, dim3(fwd_tiled_threads<float, JJ>()), b->lds_f, s>>>(probs, b->nprob, off_f)
+  batch_fwd_kernel<DD, JJ><<<grd, dim3(fwd_tiled_threads<float, JJ, DD>()), b->lds_f, s>>>(probs, b->nprob, off_f)
   if (b->nsep_f > 0) {
     switch (b->gat_rows) {
 #define TKBN_BATCH_GAT(R) \
