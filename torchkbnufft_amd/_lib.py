@@ -6,6 +6,7 @@ fallback: if the library is missing every operator raises.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 import threading
@@ -187,6 +188,16 @@ def check(status: int, what: str) -> None:
 def i64_array(values) -> ctypes.Array:
     vals = [int(v) for v in values]
     return (_c_i64 * max(len(vals), 1))(*vals)
+
+
+_HERE = contextlib.nullcontext()
+
+
+def on_device(t: torch.Tensor):
+    """Context in which ``t``'s device is the current one (switching costs the host about
+    2 us each way, several times per module call; usually it is the current one already)."""
+    device = t.device
+    return _HERE if device.index == torch.cuda.current_device() else torch.cuda.device(device)
 
 
 def stream_of(t: torch.Tensor) -> int:

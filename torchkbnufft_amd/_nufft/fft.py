@@ -53,7 +53,7 @@ def apod_pad(image: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, im_si
     if sc.numel() != math.prod(im):
         raise ValueError("scaling_coef does not match im_size")
     grid = torch.empty((B, C) + gs, dtype=image.dtype, device=image.device)
-    with torch.cuda.device(image.device):
+    with _lib.on_device(image):
         st = _lib.load().tkbn_apod_pad(
             _lib.dtype_code(image),
             d,
@@ -97,7 +97,7 @@ def crop_deapod(grid: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, im_
 def _crop_deapod_into(grid: Tensor, smaps: Optional[Tensor], sc: Tensor, im, scale: float, out: Tensor) -> None:
     d, gs = len(im), tuple(grid.shape[2:])
     B, C = grid.shape[0], grid.shape[1]
-    with torch.cuda.device(grid.device):
+    with _lib.on_device(grid):
         st = _lib.load().tkbn_crop_deapod(
             _lib.dtype_code(grid),
             d,
@@ -235,7 +235,7 @@ def fft_grid_fwd(image: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, i
     smooth = _smooth(im, gs)
     ws, nws = _fft_workspace(image.device, d, im, gs, B, C, smooth)
     lib = _lib.load()
-    with torch.cuda.device(image.device):
+    with _lib.on_device(image):
         st = (lib.tkbn_fft_grid_fwd if smooth else lib.tkbn_fft_any_grid_fwd)(
             _lib.dtype_code(image), d, _lib.i64_array(im), _lib.i64_array(gs), B, C, image.shape[1],
             image.data_ptr(), smaps.data_ptr() if smaps is not None else None, sc.data_ptr(), float(scale),
@@ -268,7 +268,7 @@ def fft_grid_adj(grid: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, im
     image = torch.empty((B, C) + im, dtype=grid.dtype, device=grid.device) if combine else out
     ws, nws = _fft_workspace(grid.device, d, im, gs, B, C, smooth)
     lib = _lib.load()
-    with torch.cuda.device(grid.device):
+    with _lib.on_device(grid):
         st = (lib.tkbn_fft_grid_adj if smooth else lib.tkbn_fft_any_grid_adj)(
             _lib.dtype_code(grid), d, _lib.i64_array(im), _lib.i64_array(gs), B, C, grid.data_ptr(),
             smaps.data_ptr() if smaps is not None and not combine else None, None if combine else sc.data_ptr(),
@@ -318,7 +318,7 @@ def fft_filter_fused(image: Tensor, smaps: Optional[Tensor], kernel: Tensor, ker
         raise ValueError(f"kernel of shape {tuple(kernel.shape)} does not match batch {B} and grid {gs}")
     out = torch.empty((B, 1 if smaps is not None else C) + im, dtype=image.dtype, device=image.device)
     ws, nws = _fft_workspace(image.device, d, im, gs, B, C)
-    with torch.cuda.device(image.device):
+    with _lib.on_device(image):
         st = _lib.load().tkbn_fft_filter(
             _lib.dtype_code(image), d, _lib.i64_array(im), _lib.i64_array(gs), B, C, image.shape[1],
             image.data_ptr(), smaps.data_ptr() if smaps is not None else None, kernel.data_ptr(),

@@ -221,7 +221,7 @@ def table_interp(
                 desc.flags = plan.flags()
             else:
                 ws = _plan_workspace("fwd", key_omega, image, nws)
-    with torch.cuda.device(image.device):
+    with _lib.on_device(image):
         st = lib.tkbn_interp_fwd(
             ctypes.byref(desc), image.data_ptr(), omega.data_ptr(), kdata.data_ptr(),
             ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, _lib.stream_of(image),
@@ -277,7 +277,7 @@ def table_interp_adjoint(
         desc.flags = plan.flags()
     else:
         ws = _plan_workspace("adj", key_omega, data, int(ws_bytes))
-    with torch.cuda.device(data.device):
+    with _lib.on_device(data):
         st = lib.tkbn_interp_adj(
             ctypes.byref(desc),
             data.data_ptr(),
@@ -318,7 +318,7 @@ def table_interp_domega(
     B, C = grid.shape[0], grid.shape[1]
     desc = make_desc(grid, om, tables, n_shift, numpoints, table_oversamp, tuple(grid.shape[2:]), B, C)
     out = torch.empty(om.shape, dtype=om.dtype, device=om.device)
-    with torch.cuda.device(grid.device):
+    with _lib.on_device(grid):
         st = _lib.load().tkbn_interp_domega(
             ctypes.byref(desc), grid.data_ptr(), grad_kdata.data_ptr(), om.data_ptr(), out.data_ptr(),
             _lib.stream_of(grid),
