@@ -2231,8 +2231,8 @@ static TileGeom make_coil_tile_geom(const tkbn_interp_desc* d) {
 // they are the only 2-D path (their tuning fields are ignored); below, a caller's tile or
 // work target asks for the sample-lane kernels, whose fields they are, and so does a
 // problem whose separable plan (about 80 bytes a sample) would pass 1 GiB.  Below 32 rows,
-// sample-lane against separable: spread 31 -> 18 us, gather 25 -> 13 us (one row, 512^2 grid,
-// 206 000 samples), spread + gather 255 -> 108 us (8 trajectories x 8 rows, 384^2).
+// sample-lane against separable: spread 31 -> 18 us, gather 25 -> 17 us (one row, 512^2 grid,
+// 206 000 samples); call pair 371 -> 207 us (8 trajectories x 8 rows, 384^2).
 static bool sep_eligible(const tkbn_interp_desc* d) {
   if (d->dtype != TKBN_F32 || d->ndim != 2) return false;
   if (d->numpoints[0] > 6 || d->numpoints[1] > 6) return false;
