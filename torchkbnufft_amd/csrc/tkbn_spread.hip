@@ -2180,7 +2180,7 @@ static int64_t rows_of(const tkbn_interp_desc* d) { return d->omega_batched ? d-
 // Form of the spread (see spread_sep_item): the outer form up to four rows (two products per
 // row and four entries; the rows form takes about eight per eight rows), 16 rows at once
 // where there are more than eight (the weights of four entries then serve twice the rows).
-static int mm_form(int64_t nrows) { return nrows > 8 ? 16 : nrows > 4 ? 8 : nrows > 2 ? 4 : (int)nrows; }
+static int mm_form(int64_t nrows) { return nrows > 8 ? 16 : nrows > 4 ? 8 : nrows > 2 ? 4 : nrows > 1 ? 2 : 1; }
 
 // (sample, tile) entries of all trajectories, about: (21/16)^2 a sample
 static int64_t sep_entries(const tkbn_interp_desc* d) { return plans_of(d) * (d->klength * 7 / 4); }
