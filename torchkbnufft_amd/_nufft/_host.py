@@ -52,6 +52,12 @@ def require_gpu(*tensors: Tensor) -> torch.device:
     return dev
 
 
+def plain(t: Tensor) -> Tensor:
+    """``t`` contiguous, with a lazy conjugate or negative carried out: the kernels read the
+    memory as it lies, and ``contiguous()`` keeps those bits."""
+    return t.resolve_conj().resolve_neg().contiguous()
+
+
 def real_dtype_of(t: Tensor) -> torch.dtype:
     return {torch.complex64: torch.float32, torch.complex128: torch.float64}[t.dtype]
 

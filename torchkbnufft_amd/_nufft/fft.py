@@ -19,7 +19,7 @@ from torch import Tensor
 
 from .. import _lib
 from .._autograd._apply import run as _run
-from ._host import host_values, require_gpu
+from ._host import host_values, plain, require_gpu
 
 
 def _norm_scale(norm: Optional[str], grid_size) -> float:
@@ -33,7 +33,7 @@ def _norm_scale(norm: Optional[str], grid_size) -> float:
 def apod_pad(image: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, im_size, grid_size, scale: float) -> Tensor:
     """grid[b, c] = pad_end(image[b, c or 0] * smaps[b, c] * scaling_coef) * scale."""
     require_gpu(image, smaps, scaling_coef)
-    image = image.contiguous()
+    image = plain(image)
     im = tuple(int(v) for v in im_size)
     gs = tuple(int(v) for v in grid_size)
     d = len(im)
@@ -42,14 +42,14 @@ def apod_pad(image: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, im_si
     if tuple(image.shape[2:]) != im:
         raise ValueError(f"image spatial shape {tuple(image.shape[2:])} != im_size {im}")
     if smaps is not None:
-        smaps = smaps.to(image.dtype).contiguous()
+        smaps = plain(smaps.to(image.dtype))
         if tuple(smaps.shape) != (B, C) + im and not (smaps.shape[0] == 1 and tuple(smaps.shape[1:]) == (C,) + im):
             raise ValueError(f"smaps shape {tuple(smaps.shape)} does not match image {tuple(image.shape)}")
         if smaps.shape[0] != B:
             smaps = smaps.expand(B, *smaps.shape[1:]).contiguous()
         if image.shape[1] not in (1, C):
             raise ValueError("image coil dimension must be 1 or match smaps")
-    sc = scaling_coef.to(device=image.device, dtype=image.dtype).contiguous()
+    sc = plain(scaling_coef.to(device=image.device, dtype=image.dtype))
     if sc.numel() != math.prod(im):
         raise ValueError("scaling_coef does not match im_size")
     grid = torch.empty((B, C) + gs, dtype=image.dtype, device=image.device)
@@ -77,18 +77,18 @@ def crop_deapod(grid: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, im_
     """image[b, c] = crop(grid[b, c]) * conj(scaling_coef) * scale; with smaps summed
     over coils against conj(smaps) into image[b, 0]."""
     require_gpu(grid, smaps, scaling_coef)
-    grid = grid.contiguous()
+    grid = plain(grid)
     im = tuple(int(v) for v in im_size)
     d = len(im)
     gs = tuple(grid.shape[2:])
     B, C = grid.shape[0], grid.shape[1]
     if smaps is not None:
-        smaps = smaps.to(grid.dtype).contiguous()
+        smaps = plain(smaps.to(grid.dtype))
         if smaps.shape[0] != B:
             smaps = smaps.expand(B, *smaps.shape[1:]).contiguous()
         if tuple(smaps.shape) != (B, C) + im:
             raise ValueError(f"smaps shape {tuple(smaps.shape)} does not match data ({B}, {C}) + {im}")
-    sc = scaling_coef.to(device=grid.device, dtype=grid.dtype).contiguous()
+    sc = plain(scaling_coef.to(device=grid.device, dtype=grid.dtype))
     out = torch.empty((B, 1 if smaps is not None else C) + im, dtype=grid.dtype, device=grid.device)
     _crop_deapod_into(grid, smaps, sc, im, scale, out)
     return out
@@ -213,7 +213,7 @@ def fft_grid_fwd(image: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, i
                  out: Optional[Tensor] = None) -> Tensor:
     """FFT(pad_end(image * smaps * scaling_coef)) * scale in one fused HIP pipeline."""
     require_gpu(image, smaps, scaling_coef)
-    image = image.contiguous()
+    image = plain(image)
     im = tuple(int(v) for v in im_size)
     gs = tuple(int(v) for v in grid_size)
     d = len(im)
@@ -225,12 +225,12 @@ def fft_grid_fwd(image: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, i
         smaps = smaps.to(image.dtype)
         if smaps.shape[0] != B:
             smaps = smaps.expand(B, *smaps.shape[1:])
-        smaps = smaps.contiguous()
+        smaps = plain(smaps)
         if tuple(smaps.shape) != (B, C) + im:
             raise ValueError(f"smaps shape {tuple(smaps.shape)} does not match image {tuple(image.shape)}")
         if image.shape[1] not in (1, C):
             raise ValueError("image coil dimension must be 1 or match smaps")
-    sc = scaling_coef.to(device=image.device, dtype=image.dtype).contiguous()
+    sc = plain(scaling_coef.to(device=image.device, dtype=image.dtype))
     grid = _out_or_new(out, (B, C) + gs, image)
     smooth = _smooth(im, gs)
     ws, nws = _fft_workspace(image.device, d, im, gs, B, C, smooth)
@@ -249,7 +249,7 @@ def fft_grid_adj(grid: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, im
                  out: Optional[Tensor] = None) -> Tensor:
     """sum_c crop(IFFT(grid)) * conj(scaling_coef) * conj(smaps_c) * scale (per coil without smaps)."""
     require_gpu(grid, smaps, scaling_coef)
-    grid = grid.contiguous()
+    grid = plain(grid)
     im = tuple(int(v) for v in im_size)
     gs = tuple(grid.shape[2:])
     d = len(im)
@@ -258,10 +258,10 @@ def fft_grid_adj(grid: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, im
         smaps = smaps.to(grid.dtype)
         if smaps.shape[0] != B:
             smaps = smaps.expand(B, *smaps.shape[1:])
-        smaps = smaps.contiguous()
+        smaps = plain(smaps)
         if tuple(smaps.shape) != (B, C) + im:
             raise ValueError(f"smaps shape {tuple(smaps.shape)} does not match data ({B}, {C}) + {im}")
-    sc = scaling_coef.to(device=grid.device, dtype=grid.dtype).contiguous()
+    sc = plain(scaling_coef.to(device=grid.device, dtype=grid.dtype))
     smooth = _smooth(im, gs)
     combine = smaps is not None and not smooth  # the convolution passes leave the coils apart
     out = _out_or_new(out, (B, 1 if smaps is not None else C) + im, grid)
@@ -300,7 +300,7 @@ def fft_filter_fused(image: Tensor, smaps: Optional[Tensor], kernel: Tensor, ker
     """One tkbn_fft_filter call: image (B, 1|C, *N) [, smaps (B|1, C, *N)], kernel
     (*K) or (B, *K) with kernel_batched; returns (B, 1|C, *N)."""
     require_gpu(image, smaps, kernel)
-    image = image.contiguous()
+    image = plain(image)
     d = image.ndim - 2
     im = tuple(int(v) for v in image.shape[2:])
     gs = tuple(int(v) for v in kernel.shape[-d:])
@@ -310,10 +310,10 @@ def fft_filter_fused(image: Tensor, smaps: Optional[Tensor], kernel: Tensor, ker
         smaps = smaps.to(image.dtype)
         if smaps.shape[0] != B:
             smaps = smaps.expand(B, *smaps.shape[1:])
-        smaps = smaps.contiguous()
+        smaps = plain(smaps)
         if tuple(smaps.shape) != (B, C) + im:
             raise ValueError(f"smaps shape {tuple(smaps.shape)} does not match image {tuple(image.shape)}")
-    kernel = kernel.to(image.dtype).contiguous()
+    kernel = plain(kernel.to(image.dtype))
     if kernel.numel() != (B if kernel_batched else 1) * math.prod(gs):
         raise ValueError(f"kernel of shape {tuple(kernel.shape)} does not match batch {B} and grid {gs}")
     out = torch.empty((B, 1 if smaps is not None else C) + im, dtype=image.dtype, device=image.device)

@@ -15,7 +15,7 @@ import torch
 from torch import Tensor
 
 from .. import _lib
-from ._host import host_values, real_dtype_of, require_gpu
+from ._host import host_values, plain, real_dtype_of, require_gpu
 
 # adjoint mode used when the caller does not ask for one
 _DEFAULT_ADJ_MODE = _lib.TKBN_ADJ_ATOMIC
@@ -172,12 +172,12 @@ def _check_out(out: Optional[Tensor], shape: tuple, like: Tensor) -> Tensor:
 
 
 def _prep_tables(tables: List[Tensor], like: Tensor) -> List[Tensor]:
-    return [t.to(device=like.device, dtype=like.dtype).contiguous() for t in tables]
+    return [plain(t.to(device=like.device, dtype=like.dtype)) for t in tables]
 
 
 def _prep_omega(omega: Tensor, like: Tensor) -> Tensor:
     # the trajectory is evaluated in the data's real precision (tm, rint, floor)
-    return omega.to(device=like.device, dtype=real_dtype_of(like)).contiguous()
+    return plain(omega.to(device=like.device, dtype=real_dtype_of(like)))
 
 
 def table_interp(
@@ -201,7 +201,7 @@ def table_interp(
     omega = _check_omega(omega, image.shape[0], "image")
     require_gpu(image, omega)
     key_omega = omega
-    image = image.contiguous()
+    image = plain(image)
     tables = _prep_tables(tables, image)
     omega = _prep_omega(omega, image)
     grid_size = tuple(image.shape[2:])
@@ -252,7 +252,7 @@ def table_interp_adjoint(
     omega = _check_omega(omega, data.shape[0], "data")
     require_gpu(data, omega)
     key_omega = omega
-    data = data.contiguous()
+    data = plain(data)
     tables = _prep_tables(tables, data)
     omega = _prep_omega(omega, data)
     gs = tuple(int(v) for v in host_values(grid_size))
@@ -311,8 +311,8 @@ def table_interp_domega(
     orig = omega
     om = _check_omega(omega, grid.shape[0], "image")
     require_gpu(grid, grad_kdata, om)
-    grid = grid.contiguous()
-    grad_kdata = grad_kdata.to(grid.dtype).contiguous()
+    grid = plain(grid)
+    grad_kdata = plain(grad_kdata.to(grid.dtype))
     tables = _prep_tables(tables, grid)
     om = _prep_omega(om, grid)
     B, C = grid.shape[0], grid.shape[1]

@@ -30,7 +30,7 @@ from scipy import special
 from torch import Tensor
 
 from .. import _lib
-from ._host import host_values, require_gpu
+from ._host import host_values, plain, require_gpu
 from .utils import validate_args
 
 _BLOCK_ROWS = 8  # rows per block of the sparse format (the library's tkbn_spmv_block_rows)
@@ -182,7 +182,7 @@ class SpmvPlan:
 
     def apply(self, x: Tensor) -> Tensor:
         """y (batch, nrows) = A x for x (batch, ncols), complex, on the plan's device."""
-        x = x.contiguous()
+        x = plain(x)
         batch = x.shape[0]
         y = torch.empty((batch, self.nrows), dtype=x.dtype, device=x.device)
         if batch == 0 or self.nrows == 0:
