@@ -1547,7 +1547,7 @@ __global__ void __launch_bounds__(GatShape<ROWS>::kThreads)
 // On the matrix cores: in the rotated frame every tap of an entry adds s * w0[i] * w1[j]
 // with real w0, w1 (s = kdata * F), so a tile's sum over its entries is a matrix product
 // with the entries as the inner dimension.  A wave takes four entries of a 16 x 16 tile per
-// 16x16x4 float32 MFMA; their weights and data pass through its own part of LDS, without
+// 16x16x4 MFMA; their weights and data pass through its own part of LDS, without
 // work-group barriers.  A tile (or a piece of its entries) belongs to one wave, or, where
 // tiles are dense, to the four waves of a group, which split its entries and add their sums
 // through LDS at the end: a tile's entries are a serial chain, and cutting it into more
@@ -1577,23 +1577,37 @@ constexpr int mm_waves(int G) { return G >= 8 ? 2 : G > 2 ? 3 : 4; }
 // floats per staged entry's data (two components a row; +2 spreads the banks)
 constexpr int mm_spitch(int G) { return 2 * G + 2; }
 
-// Dense tiles add hundreds of entries to a cell, and one float32 chain over them was the
-// spread's largest error (8 rows, 256^2: image off by 1.8e-7; 64-bit integer sums: 1.6e-7).
-// So each batch's 32 entries have a chain of their own, and the batches are added up outside
-// the matrix cores: in double for one or two rows, in float32 for more (1.6e-7 again).  16
-// rows leave no registers for it; with 12 rows one chain is as good as the integer sums
-// (1.1e-7 both).
-__host__ __device__ constexpr bool mm_two_level(int G) { return G <= 8; }
-template <bool Double>
+// Sums.  Chunks of up to 8 rows: in double, on the float64 MFMA (half the float32 rate), the
+// weights' products too, so that a cell is rounded once however many entries it meets, as with
+// the 64-bit integer sums of the sample-lane kernel.  Against 64-bit sums of random data, 900
+// samples in one tile: 6.0e-8, the integer sums 6.8e-8; float32 chains of 32 entries added up
+// in double 8.4e-8, one float32 chain 1.6e-7 (and 4e-7 on a cell of one-sign data, now 6e-8).
+// 256^2, 402 x 512 radial, adjoint interpolation of 1 / 8 / 12 rows: 29 / 64 / 107 us, 25 /
+// 53 / 70 with float32 sums, 44 / 163 / 223 with the integer sums.  Chunks of 16 rows, which
+// only problems of 32 rows on one trajectory and more take, stay in float32, as their sums
+// have always been.
+template <int G>
 struct MmSum {
-  typedef f32x4 vec;
-  typedef float one;
-};
-template <>
-struct MmSum<true> {
   typedef f64x4 vec;
   typedef double one;
 };
+template <>
+struct MmSum<16> {
+  typedef f32x4 vec;
+  typedef float one;
+};
+__device__ __forceinline__ f32x4 mm_mfma(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f64x4 mm_mfma(double a, double b, f64x4 c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+// Row of the first operand that lane n16 brings, so that register v of lane group k4 holds row
+// 4 k4 + v of the product (the float32 form's own order; the float64 one holds row 4 v + k4)
+template <int G>
+__device__ __forceinline__ int mm_arow(int n16) {
+  return sizeof(typename MmSum<G>::one) == 4 ? n16 : 4 * (n16 & 3) + (n16 >> 2);
+}
 
 template <int G>
 struct __attribute__((aligned(16))) MmLds {  // one wave's staging
@@ -1666,18 +1680,12 @@ __device__ __forceinline__ void spread_sep_item(const Geom<float>& g, const Tile
   const double2 pc = reinterpret_cast<const double2*>(plan + sg.o_ptab[1])[min(o1 + n16, g.K[1] - 1)];
 
   constexpr int kAcc = kGroups > 0 ? kGroups * kRegT0 : 2 * kRows;
-  f32x4 acc[kAcc];
+  typedef typename MmSum<G>::vec Sum;
+  typedef typename MmSum<G>::one Sum1;
+  const int arow = mm_arow<G>(n16);
+  Sum sum[kAcc];
 #pragma unroll
-  for (int c = 0; c < kAcc; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // Sums of the batches' sums
-  typedef typename MmSum<(G <= 2)>::vec Sum;
-  typedef typename MmSum<(G <= 2)>::one Sum1;
-  constexpr bool kTwo = mm_two_level(G);
-  Sum tot[kTwo ? kAcc : 1];
-  if constexpr (kTwo) {
-#pragma unroll
-    for (int c = 0; c < kAcc; ++c) tot[c] = Sum{0, 0, 0, 0};
-  }
+  for (int c = 0; c < kAcc; ++c) sum[c] = Sum{0, 0, 0, 0};
 
   // Staging: lane (entry e, half h) holds the sample's header, its weights along dimension h
   // and its data for the half's rows.  The sample indices are loaded two batches ahead, the
@@ -1703,7 +1711,7 @@ __device__ __forceinline__ void spread_sep_item(const Geom<float>& g, const Tile
   };
   int nexc = 0;  // entries left to the atomic pass
   // operands of entries 4 k .. 4 k + 3: rows form: the tile's 16 row weights, outer form: the
-  // weight of row n16; the weight of column n16; the data
+  // weight of row arow; the weight of column n16; the data
   struct Operands {
     f32x4 w0[kGroups > 0 ? 4 : 1];
     float w1, a[kGroups > 0 ? kGroups : 2 * kRows];
@@ -1714,11 +1722,11 @@ __device__ __forceinline__ void spread_sep_item(const Geom<float>& g, const Tile
     o.w1 = lds.w1[en * kMmWPitch + n16];
     if constexpr (kGroups > 0) {
 #pragma unroll
-      for (int u = 0; u < kGroups; ++u) o.a[u] = lds.s[en * kSP + 16 * u + n16];
+      for (int u = 0; u < kGroups; ++u) o.a[u] = lds.s[en * kSP + 16 * u + arow];
 #pragma unroll
       for (int q = 0; q < 4; ++q) o.w0[q] = *reinterpret_cast<const f32x4*>(&lds.w0[en * kMmWPitch + 4 * q]);
     } else {
-      o.w0[0][0] = lds.w0[en * kMmWPitch + n16];
+      o.w0[0][0] = lds.w0[en * kMmWPitch + arow];
 #pragma unroll
       for (int c = 0; c < kRows; ++c) {
         const float2 sv = *reinterpret_cast<const float2*>(&lds.s[en * kSP + 2 * c]);
@@ -1796,35 +1804,22 @@ __device__ __forceinline__ void spread_sep_item(const Geom<float>& g, const Tile
 #pragma unroll
         for (int r = 0; r < kRegT0; ++r) {
           if ((mk >> r) & 1u) {
-            const float w = op.w0[r / 4][r % 4] * op.w1;
+            const Sum1 w = (Sum1)op.w0[r / 4][r % 4] * (Sum1)op.w1;
 #pragma unroll
-            for (int u = 0; u < kGroups; ++u)
-              acc[u * kRegT0 + r] = __builtin_amdgcn_mfma_f32_16x16x4f32(op.a[u], w, acc[u * kRegT0 + r], 0, 0, 0);
+            for (int u = 0; u < kGroups; ++u) sum[u * kRegT0 + r] = mm_mfma((Sum1)op.a[u], w, sum[u * kRegT0 + r]);
           }
         }
       } else if (mk != 0) {
 #pragma unroll
         for (int c = 0; c < kRows; ++c) {
-          acc[2 * c] = __builtin_amdgcn_mfma_f32_16x16x4f32(op.w0[0][0] * op.a[2 * c], op.w1, acc[2 * c], 0, 0, 0);
-          acc[2 * c + 1] =
-              __builtin_amdgcn_mfma_f32_16x16x4f32(op.w0[0][0] * op.a[2 * c + 1], op.w1, acc[2 * c + 1], 0, 0, 0);
+          sum[2 * c] = mm_mfma((Sum1)op.w0[0][0] * (Sum1)op.a[2 * c], (Sum1)op.w1, sum[2 * c]);
+          sum[2 * c + 1] = mm_mfma((Sum1)op.w0[0][0] * (Sum1)op.a[2 * c + 1], (Sum1)op.w1, sum[2 * c + 1]);
         }
       }
       op = nxt;
     }
     wave_lds_sync();  // the next batch overwrites the staging
-    if constexpr (kTwo) {
-#pragma unroll
-      for (int c = 0; c < kAcc; ++c) {
-        tot[c] += __builtin_convertvector(acc[c], Sum);
-        acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-    }
   }
-  Sum(&sum)[kAcc] = [&]() -> Sum(&)[kAcc] {
-    if constexpr (kTwo) return tot;
-    else return acc;
-  }();
 
   const int exc = lane < kMmExc ? lds.exc[lane] : 0;  // (the staging is reused)
 
@@ -2178,9 +2173,14 @@ int spread_launch(const Geom<T>& g, const TileGeom& tg, bool det, const void* kd
 static int64_t plans_of(const tkbn_interp_desc* d) { return d->omega_batched ? d->batch : 1; }
 static int64_t rows_of(const tkbn_interp_desc* d) { return d->omega_batched ? d->coils : d->batch * d->coils; }
 // Form of the spread (see spread_sep_item): the outer form up to four rows (two products per
-// row and four entries; the rows form takes about eight per eight rows), 16 rows at once
-// where there are more than eight (the weights of four entries then serve twice the rows).
-static int mm_form(int64_t nrows) { return nrows > 8 ? 16 : nrows > 4 ? 8 : nrows > 2 ? 4 : nrows > 1 ? 2 : 1; }
+// row and four entries; the rows form takes about eight per eight rows), else 8 rows at once;
+// 16, in float32 (the weights of four entries then serve twice the rows), from 32 rows on one
+// trajectory on, whose sums have always been float32.
+static bool sep_many_rows(const tkbn_interp_desc* d) { return !d->omega_batched && d->batch * d->coils >= 32; }
+static int mm_form(const tkbn_interp_desc* d) {
+  const int64_t nrows = rows_of(d);
+  return sep_many_rows(d) ? 16 : nrows > 4 ? 8 : nrows > 2 ? 4 : nrows > 1 ? 2 : 1;
+}
 
 // (sample, tile) entries of all trajectories, about: (21/16)^2 a sample
 static int64_t sep_entries(const tkbn_interp_desc* d) { return plans_of(d) * (d->klength * 7 / 4); }
@@ -2209,7 +2209,7 @@ static TileGeom make_coil_tile_geom(const tkbn_interp_desc* d) {
   // chains end with the rest, within 128 (one coil, 256^2, 402 x 512 radial: 16.6 us, 21.1
   // with 384) and 1024 (64 rows, 320^2 radial: 216 us at 896, 250 at 512, 277 at 384).
   {
-    const int64_t chunks = ceil_div(rows_of(d), mm_rows(mm_form(rows_of(d))));
+    const int64_t chunks = ceil_div(rows_of(d), mm_rows(mm_form(d)));
     const int64_t per_simd = sep_entries(d) * chunks / 1024;
     const int64_t half = ceil_div(per_simd / 2, kMmBatch) * kMmBatch;
     const int ks = mm_waves_per_item(sep_entries(d), (int64_t)tg.NB * plans_of(d), chunks);
@@ -2236,7 +2236,7 @@ static TileGeom make_coil_tile_geom(const tkbn_interp_desc* d) {
 static bool sep_eligible(const tkbn_interp_desc* d) {
   if (d->dtype != TKBN_F32 || d->ndim != 2) return false;
   if (d->numpoints[0] > 6 || d->numpoints[1] > 6) return false;
-  if (!d->omega_batched && d->batch * d->coils >= 32) return true;
+  if (sep_many_rows(d)) return true;
   if (d->tile[0] > 0 || d->tile[1] > 0 || d->work_target > 0) return false;
   return (d->omega_batched ? d->batch : 1) * d->klength * 80 <= (1LL << 30);
 }
@@ -2313,7 +2313,7 @@ static TileGeom make_sep_spread_geom(const tkbn_interp_desc* d, SepGeom* sg) {
   // 16 rows a chunk: a record per entry is read in order (16 coils x 4, 320^2 radial: 225 us;
   // through the sample index: 245); fewer rows, where the plan weighs more against the data,
   // a record per sample (one row, 205 824 samples: 16 instead of 56 MB, 17.8 us both)
-  tg.rec_entry = mm_form(rows_of(d)) == 16;
+  tg.rec_entry = mm_form(d) == 16;
   tg.T[2] = 2 * tg.target + tg.rec_entry;  // part of the plan's key
   *sg = sep_phase_of(d);
   int64_t o = 0;
@@ -2435,7 +2435,7 @@ static int spread_sep_launch(const tkbn_interp_desc* d, const void* kdata, const
   const int st = sep_plan_launch(d, static_cast<float2*>(grid), g, tg, sg, om, ws, wsi, s);
   if (st != TKBN_OK) return st;
   const int64_t nrows = rows_of(d), np = plans_of(d);
-  const int form = mm_form(nrows);
+  const int form = mm_form(d);
   const int nchunk = (int)ceil_div(nrows, mm_rows(form));
   const int ks = mm_waves_per_item(sep_entries(d), tg.NB * plans_of(d), nchunk);
   const int64_t groups = ceil_div(tg.maxwork * nchunk, kMmWaves / ks);
@@ -3521,7 +3521,7 @@ int tkbn_batch_create(const tkbn_interp_desc* descs, const tkbn_interp_desc* adj
     const int64_t nrows = d->batch * d->coils;
     if (q.sep_f) b->gat_rows = std::max(b->gat_rows, gat_rows(nrows));
     if (q.sep_a) {
-      b->form = std::max(b->form, mm_form(nrows));
+      b->form = std::max(b->form, mm_form(da));
       entries += sep_entries(da);
       tiles += q.ta.NB;
     }
@@ -3658,8 +3658,7 @@ int tkbn_batch_interp_adj(const tkbn_batch* b, const void* table, void* workspac
       case 1: batch_spread_sep_kernel<1><<<gs, blk, 0, s>>>(probs, b->nprob, off_a, b->ks); break;
       case 2: batch_spread_sep_kernel<2><<<gs, blk, 0, s>>>(probs, b->nprob, off_a, b->ks); break;
       case 4: batch_spread_sep_kernel<4><<<gs, blk, 0, s>>>(probs, b->nprob, off_a, b->ks); break;
-      case 8: batch_spread_sep_kernel<8><<<gs, blk, 0, s>>>(probs, b->nprob, off_a, b->ks); break;
-      default: batch_spread_sep_kernel<16><<<gs, blk, 0, s>>>(probs, b->nprob, off_a, b->ks); break;
+      default: batch_spread_sep_kernel<8><<<gs, blk, 0, s>>>(probs, b->nprob, off_a, b->ks); break;
     }
     TKBN_LAUNCH_CHECK("batch_spread_sep_kernel");
   }
