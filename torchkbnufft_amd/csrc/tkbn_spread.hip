@@ -2204,16 +2204,21 @@ static TileGeom make_coil_tile_geom(const tkbn_interp_desc* d) {
   tg.bstride[1] = 1;
   tg.bstride[0] = tg.nb[1];
   tg.NB = tg.nb[0] * tg.nb[1];
-  // Entries per piece and wave.  A wave's entries are a serial chain, and pieces add with
-  // atomics: half of what a SIMD gets if the entries of all chunks spread evenly, so that the
-  // chains end with the rest, within 128 (one coil, 256^2, 402 x 512 radial: 16.6 us, 21.1
-  // with 384) and 1024 (64 rows, 320^2 radial: 216 us at 896, 250 at 512, 277 at 384).
+  // Entries per piece: a multiple of the mean tile's, so that few tiles are cut (pieces add
+  // with atomics) and none is a long serial chain.  The rows have no say in it (a plan serves
+  // calls of any number of rows, see sep_many_rows), nor has the number of waves that a launch
+  // gives a piece, so it holds for both.  Adjoint interpolation of 8 rows, us, pieces of 128 /
+  // 256 / 512 / 768 / 1024 / 2048: 256^2, 206 k radial samples (352 entries a tile) 153 / 88 /
+  // 69 / 65 / 64 / 84; 96^2, 12 k (140) 20 / 21 / 28 / 35 / 42 / 44; 512^2, 307 k (131) 142 /
+  // 91 / 92 / 116 / 142 / 239.  64 rows, 320^2, 256 k (280), 512 / 704 / 896 / 1024: 255 / 230 /
+  // 218 / 214; 32 rows, 96^2, 512 / 704 / 1024: 33 / 38 / 47; float32 chains of more than 768
+  // entries would be further from 64-bit sums than they have been (one-sign data, 1000 entries
+  // in a tile: 4.8e-7 at 1024, 3.1e-7 at 768).
   {
-    const int64_t chunks = ceil_div(rows_of(d), mm_rows(mm_form(d)));
-    const int64_t per_simd = sep_entries(d) * chunks / 1024;
-    const int64_t half = ceil_div(per_simd / 2, kMmBatch) * kMmBatch;
-    const int ks = mm_waves_per_item(sep_entries(d), (int64_t)tg.NB * plans_of(d), chunks);
-    tg.target = ks * (int)(half < 128 ? 128 : half > 1024 ? 1024 : half);
+    const int64_t mean = sep_entries(d) / ((int64_t)tg.NB * std::max<int64_t>(plans_of(d), 1));
+    const bool many = sep_many_rows(d);
+    const int64_t t = ceil_div(many ? 4 * mean : mean * 5 / 2, kMmBatch) * kMmBatch;
+    tg.target = (int)std::min<int64_t>(std::max<int64_t>(t, many ? 512 : 256), many ? 768 : 1024);
   }
   // tiles a footprint can meet per dimension: 2, or 3 when the last tile is shorter
   // than J - 1 (the footprint then crosses it into the first tile)
