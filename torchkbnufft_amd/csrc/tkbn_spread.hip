@@ -2235,20 +2235,29 @@ static TileGeom make_coil_tile_geom(const tkbn_interp_desc* d) {
 // The separable kernels take complex64, 2-D, J <= 6.  From 32 coil rows on one trajectory
 // they are the only 2-D path (their tuning fields are ignored); below, a caller's tile or
 // work target asks for the sample-lane kernels, whose fields they are, and so does a
-// problem whose separable plan (about 80 bytes a sample) would pass 1 GiB.  Below 32 rows,
+// problem one of whose separable workspaces (72 bytes a sample in the forward, 88 to 108 in
+// the adjoint, tables and tile lists beside) would pass 1 GiB.  Below 32 rows,
 // sample-lane against separable: spread 31 -> 18 us, gather 25 -> 17 us (one row, 512^2 grid,
 // 206 000 samples); call pair 371 -> 207 us (8 trajectories x 8 rows, 384^2).
+constexpr int64_t kSepMaxBytes = 1LL << 30;
+static int64_t sep_fwd_bytes(const tkbn_interp_desc* d);
+static int64_t sep_adj_bytes(const tkbn_interp_desc* d);
+
+// (the spread needs grids of at least tile + J - 1 cells per dimension)
+static bool sep_spread_grid(const tkbn_interp_desc* d) {
+  return d->grid_size[0] >= kRegT0 + 5 && d->grid_size[1] >= kRegT1 + 5;
+}
+static bool sep_form(const tkbn_interp_desc* d) {
+  return d->dtype == TKBN_F32 && d->ndim == 2 && d->numpoints[0] <= 6 && d->numpoints[1] <= 6;
+}
 static bool sep_eligible(const tkbn_interp_desc* d) {
-  if (d->dtype != TKBN_F32 || d->ndim != 2) return false;
-  if (d->numpoints[0] > 6 || d->numpoints[1] > 6) return false;
+  if (!sep_form(d)) return false;
   if (sep_many_rows(d)) return true;
   if (d->tile[0] > 0 || d->tile[1] > 0 || d->work_target > 0) return false;
-  return (d->omega_batched ? d->batch : 1) * d->klength * 80 <= (1LL << 30);
+  return std::max(sep_fwd_bytes(d), sep_spread_grid(d) ? sep_adj_bytes(d) : 0) <= kSepMaxBytes;
 }
-// and the spread grids of at least tile + J - 1 cells per dimension
-static bool coil_variant_eligible(const tkbn_interp_desc* d) {
-  return sep_eligible(d) && d->grid_size[0] >= kRegT0 + 5 && d->grid_size[1] >= kRegT1 + 5;
-}
+static bool coil_variant_eligible(const tkbn_interp_desc* d) { return sep_eligible(d) && sep_spread_grid(d); }
+
 // One-shot timing hook: events the caller asked to have recorded around the next
 // main interpolation kernel (tkbn_profile_next_kernel).
 struct ProfileHook {
@@ -2337,7 +2346,11 @@ static TileGeom make_sep_spread_geom(const tkbn_interp_desc* d, SepGeom* sg) {
 }
 
 static int64_t sep_workspace_bytes(const tkbn_interp_desc* d, const TileGeom& tg) {
-  return plans_of(d) * tg.plan_stride * 4;
+  return plan_cache_bytes(d) + plans_of(d) * tg.plan_stride * 4;
+}
+static int64_t sep_adj_bytes(const tkbn_interp_desc* d) {
+  SepGeom sg;
+  return sep_workspace_bytes(d, make_sep_spread_geom(d, &sg));
 }
 
 // The plan kernels of the separable gather (grid = nullptr) or spread, one plan per
@@ -3207,11 +3220,13 @@ static TileGeom make_gather_geom(const tkbn_interp_desc* d) {
   return tg;
 }
 
+static int64_t sep_fwd_bytes(const tkbn_interp_desc* d) {
+  SepGeom sg;
+  return sep_workspace_bytes(d, make_sep_gather_geom(d, &sg));
+}
+
 int64_t interp_fwd_workspace_bytes(const tkbn_interp_desc* d) {
-  if (sep_eligible(d)) {
-    SepGeom sg;
-    return plan_cache_bytes(d) + sep_workspace_bytes(d, make_sep_gather_geom(d, &sg));
-  }
+  if (sep_eligible(d)) return sep_fwd_bytes(d);
   const TileGeom tg = make_tile_geom(d, false, true);
   const size_t lds = (size_t)tg.CC * tg.rcells * (d->dtype == TKBN_F32 ? 8 : 16);
   if (lds > (size_t)kLdsBudget) return 0;  // region too large for LDS: plain kernel
@@ -3756,8 +3771,7 @@ int tkbn_interp_adj_noalloc(const tkbn_interp_desc* desc, const void* kdata, con
   int64_t need = tkbn_interp_adj_workspace_bytes(desc, mode);
   bool sep = true;
   if (!det && coil_variant_eligible(desc)) {
-    SepGeom sg;
-    need = plan_cache_bytes(desc) + sep_workspace_bytes(desc, make_sep_spread_geom(desc, &sg));
+    need = sep_adj_bytes(desc);
     if (need > kNoAllocScratchBytes && (desc->omega_batched || desc->batch * desc->coils < 32)) {
       sep = false;
       need = adj_lane_bytes(desc, det);
@@ -3791,15 +3805,12 @@ int64_t tkbn_interp_adj_workspace_bytes(const tkbn_interp_desc* desc, int32_t mo
   if (mode != TKBN_ADJ_ATOMIC && mode != TKBN_ADJ_DETERMINISTIC) return -1;
   const bool det = mode == TKBN_ADJ_DETERMINISTIC;
   int64_t n = adj_lane_bytes(desc, det);
-  // Room for the separable plan too, also where tuning fields ask for the sample-lane
-  // kernels: a caller that tunes one problem keeps one buffer.
+  // Room for either path's plan, also where tuning fields ask for the sample-lane kernels: a
+  // caller that tunes one problem keeps one buffer (it holds one plan at a time).
   tkbn_interp_desc plain = *desc;
   for (int i = 0; i < 3; ++i) plain.tile[i] = 0;
   plain.work_target = 0;
-  if (!det && coil_variant_eligible(&plain)) {
-    SepGeom sg;
-    n += sep_workspace_bytes(desc, make_sep_spread_geom(desc, &sg));
-  }
+  if (!det && coil_variant_eligible(&plain)) n = std::max(n, sep_adj_bytes(desc));
   if (reg3_eligible(desc)) {
     const int64_t nr = plan_cache_bytes(desc) + reg3_workspace_bytes(make_reg3_geom(desc, det));
     n = nr > n ? nr : n;
