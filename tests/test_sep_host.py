@@ -82,3 +82,12 @@ def test_workspace_holds_the_larger_plan_not_both():
     d = _desc(1, 4, 200000, (512, 512))
     lane = 24 * 200000
     assert _bytes(d) < 88 * 200000 + lane
+
+
+def test_frames_share_tables_and_phases():
+    """Per trajectory a plan holds its samples and tile lists only: the real tables (12290
+    floats here) and cell phases are one per workspace."""
+    one, many = _desc(1, 1, 128, (128, 128), batched=True), _desc(1001, 1, 128, (128, 128), batched=True)
+    for way, per_sample in (("fwd", 72), ("adj", 88)):
+        per_frame = (_bytes(many, way) - _bytes(one, way)) / 1000
+        assert per_frame < 128 * per_sample + 4 * 10 * (64 + 4)

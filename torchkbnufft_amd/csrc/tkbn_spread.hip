@@ -937,9 +937,12 @@ __global__ void __launch_bounds__((fwd_tiled_threads<T, JM, D>()))
 // ---------------------------------------------------------------------------
 struct SepGeom {
   int L[2];            // table oversampling
-  int64_t o_rtab[2];   // int offsets of the real tables in the plan
-  int64_t o_ptab[2];   // int offsets of the cell phases P_d(k), k < K_d (double2) in the plan
-  int64_t o_nm1;       // int offset of N_d - 1 (2 ints), found from the tables by the plan
+  // int offsets of what the trajectories of a call share (behind their plans):
+  int64_t o_rtab[2];   // the real tables
+  int64_t o_ptab[2];   // the cell phases P_d(k), k < K_d (double2)
+  int64_t o_nm1;       // N_d - 1 (2 ints), found from the tables
+  int64_t o_flag;      // set where a table is not of the form
+  int64_t end;         // ints of the plans and this in all
 };
 
 // N - 1 of the table's phase, read off its first entry past the centre:
@@ -1050,14 +1053,16 @@ __device__ __forceinline__ float2 sep_factor(float theta, double turns) {
   return make_float2((float)c, (float)s);
 }
 
-// Real tables R_d[i] = Re(t_d[i] exp(i pi (N-1)(i - J L / 2) / (L K))) into the plan;
-// flags the plan when any imaginary part is not negligible (the table does not have
+// Real tables R_d[i] = Re(t_d[i] exp(i pi (N-1)(i - J L / 2) / (L K))) and cell phases, once
+// for all trajectories (the blocks of the first one; 12 000 values in double for the usual
+// tables); sets the flag when any imaginary part is not negligible (the table does not have
 // the form, or N is unknown for a complex table).  Grid-stride over both tables.
-__device__ __forceinline__ void sep_table_prep(const Geom<float>& g, const SepGeom& sg, int* plan, int* flag) {
+__device__ __forceinline__ void sep_table_prep(const Geom<float>& g, const SepGeom& sg, int* tabs) {
+  if (blockIdx.y != 0) return;
   const int nm1[2] = {sep_nm1_estimate(g, 0), sep_nm1_estimate(g, 1)};
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    plan[sg.o_nm1] = nm1[0];
-    plan[sg.o_nm1 + 1] = nm1[1];
+    tabs[sg.o_nm1] = nm1[0];
+    tabs[sg.o_nm1 + 1] = nm1[1];
   }
   const int64_t n0 = g.tmax[0] + 1, n1 = g.tmax[1] + 1;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n0 + n1;
@@ -1068,23 +1073,25 @@ __device__ __forceinline__ void sep_table_prep(const Geom<float>& g, const SepGe
     const double2 p = pi_phase_d((int64_t)nm1[d] * (m - g.center[d]), (int64_t)sg.L[d] * g.K[d]);
     const float re = (float)((double)t.x * p.x - (double)t.y * p.y);
     const float im = (float)((double)t.x * p.y + (double)t.y * p.x);
-    reinterpret_cast<float*>(plan + sg.o_rtab[d])[m] = re;
-    if (!(fabsf(im) <= 0x1p-19f * (fabsf(t.x) + fabsf(t.y)))) atomicOr(flag, 1);
+    reinterpret_cast<float*>(tabs + sg.o_rtab[d])[m] = re;
+    if (!(fabsf(im) <= 0x1p-19f * (fabsf(t.x) + fabsf(t.y)))) atomicOr(tabs + sg.o_flag, 1);
   }
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < (int64_t)g.K[0] + g.K[1];
        i += (int64_t)gridDim.x * blockDim.x) {
     const int d = i < g.K[0] ? 0 : 1;
     const int k = (int)(d == 0 ? i : i - g.K[0]);
-    reinterpret_cast<double2*>(plan + sg.o_ptab[d])[k] = pi_phase_d((int64_t)nm1[d] * k, g.K[d]);
+    reinterpret_cast<double2*>(tabs + sg.o_ptab[d])[k] = pi_phase_d((int64_t)nm1[d] * k, g.K[d]);
   }
 }
 
 // ---- plans -------------------------------------------------------------------------
 __device__ __forceinline__ void sep_gat_record(const Geom<float>& g, const TileGeom& tg, const SepGeom& sg,
-                                               const float* __restrict__ omega, int* __restrict__ ws, int m, int key,
+                                               const float* __restrict__ omega, int* __restrict__ plan,
+                                               const int* __restrict__ tabs, int m, int key,
                                                const int (&l)[2], int pos);
 __device__ __forceinline__ void sep_spr_scatter_item(const Geom<float>& g, const TileGeom& tg, const SepGeom& sg,
-                                                     const float* __restrict__ omega, int* __restrict__ ws, int m);
+                                                     const float* __restrict__ omega, int* __restrict__ plan,
+                                                     const int* __restrict__ tabs, int m);
 
 // Scan of per-tile counts into tile starts and the work list, longest work first: tiles
 // above `target` entries, cut into pieces of `target`, then the others by size class (above
@@ -1149,7 +1156,7 @@ __device__ __forceinline__ void sep_scan_if_last(const TileGeom& tg, int* __rest
   __shared__ bool last;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if (threadIdx.x == 0) last = atomicAdd(plan + tg.o_count + tg.NB + 1, 1) == (int)gridDim.x - 1;
+  if (threadIdx.x == 0) last = atomicAdd(plan + tg.o_count + tg.NB, 1) == (int)gridDim.x - 1;
   __syncthreads();
   if (!last) return;
   __threadfence();
@@ -1157,15 +1164,15 @@ __device__ __forceinline__ void sep_scan_if_last(const TileGeom& tg, int* __rest
 }
 
 // Forward: each sample once, in the 16 x 16 tile of its base cell (trajectory order
-// within a tile as far as the building atomics keep it); count[NB] is the table flag.
+// within a tile as far as the building atomics keep it); count[NB] counts finished blocks.
 // blockIdx.y: the trajectory (one plan each).
 __global__ void __launch_bounds__(256)
     sep_gat_count_kernel(const Geom<float> g, const TileGeom tg, const SepGeom sg, const float* __restrict__ omega,
                          int* __restrict__ ws, const CacheHdr* cache) {
   if (cache_hit(cache)) return;  // cached plan reused
+  sep_table_prep(g, sg, ws);
   omega += (int64_t)blockIdx.y * 2 * g.M;
   ws += (int64_t)blockIdx.y * tg.plan_stride;
-  sep_table_prep(g, sg, ws, ws + tg.o_count + tg.NB);
   for (int m0 = blockIdx.x * blockDim.x; m0 < g.M; m0 += gridDim.x * blockDim.x) {
     const int m = m0 + threadIdx.x;
     const bool live = m < g.M;
@@ -1181,31 +1188,32 @@ __global__ void __launch_bounds__(256)
                            int* __restrict__ ws, const CacheHdr* cache) {
   if (cache_hit(cache)) return;  // cached plan reused
   omega += (int64_t)blockIdx.y * 2 * g.M;
-  ws += (int64_t)blockIdx.y * tg.plan_stride;
+  int* const plan = ws + (int64_t)blockIdx.y * tg.plan_stride;
   for (int m0 = blockIdx.x * blockDim.x; m0 < g.M; m0 += gridDim.x * blockDim.x) {
     const int m = m0 + threadIdx.x;
     const bool live = m < g.M;
     int l[2] = {0, 0};
     const int key = live ? gat_base_tile(g, tg, omega, m, l) : 0;
-    const int pos = wave_aggregated_inc(ws + tg.o_cursor, key, live);
-    if (live) sep_gat_record(g, tg, sg, omega, ws, m, key, l, pos);
+    const int pos = wave_aggregated_inc(plan + tg.o_cursor, key, live);
+    if (live) sep_gat_record(g, tg, sg, omega, plan, ws, m, key, l, pos);
   }
 }
 
 // the forward record of sample m (tile `key`, base cell l inside it) at plan position pos
 __device__ __forceinline__ void sep_gat_record(const Geom<float>& g, const TileGeom& tg, const SepGeom& sg,
-                                               const float* __restrict__ omega, int* __restrict__ ws, int m, int key,
+                                               const float* __restrict__ omega, int* __restrict__ plan,
+                                               const int* __restrict__ tabs, int m, int key,
                                                const int (&l)[2], int pos) {
-  const bool tab_ok = ws[tg.o_count + tg.NB] == 0;
-  const int nm10 = ws[sg.o_nm1], nm11 = ws[sg.o_nm1 + 1];
+  const bool tab_ok = tabs[sg.o_flag] == 0;
+  const int nm10 = tabs[sg.o_nm1], nm11 = tabs[sg.o_nm1 + 1];
   const float om0 = omega[m], om1 = omega[g.M + m];
   const SepTaps a = sep_taps(g, 0, om0), b = sep_taps(g, 1, om1);
   const float theta = sample_theta<float, 2>(g, omega, m);
   double turns = 0.;
   SepRec rec;
   const bool exc = !(tab_ok && a.regular && b.regular);
-  const float* R0 = reinterpret_cast<const float*>(ws + sg.o_rtab[0]);
-  const float* R1 = reinterpret_cast<const float*>(ws + sg.o_rtab[1]);
+  const float* R0 = reinterpret_cast<const float*>(tabs + sg.o_rtab[0]);
+  const float* R1 = reinterpret_cast<const float*>(tabs + sg.o_rtab[1]);
 #pragma unroll
   for (int j = 0; j < 6; ++j) {
     rec.w0[j] = (!exc && j < g.J[0]) ? R0[a.ti0 - j * sg.L[0]] : 0.f;
@@ -1220,19 +1228,19 @@ __device__ __forceinline__ void sep_gat_record(const Geom<float>& g, const TileG
   rec.me = m | (exc ? (int)0x80000000u : 0);
   rec.rc = (l[0] + 8) | ((l[1] + 8) << 8);
   rec.F = sep_factor(theta, turns);
-  reinterpret_cast<SepRec*>(reinterpret_cast<char*>(ws) + tg.o_rec_bytes)[pos] = rec;
+  reinterpret_cast<SepRec*>(reinterpret_cast<char*>(plan) + tg.o_rec_bytes)[pos] = rec;
 }
 
-// Adjoint: one entry per (sample, 16 x 16 tile its footprint meets); count[NB] is the
-// table flag.  The sample index (with the exception flag) goes to perm, the record to
-// the same position.
+// Adjoint: one entry per (sample, 16 x 16 tile its footprint meets), count[NB] as above.  The
+// sample index goes to perm; the record, with the exception flag, to the same position or (not
+// rec_entry) to the sample's.
 __global__ void __launch_bounds__(256)
     sep_spr_count_kernel(const Geom<float> g, const TileGeom tg, const SepGeom sg, const float* __restrict__ omega,
                          int* __restrict__ ws, const CacheHdr* cache) {
   if (cache_hit(cache)) return;  // cached plan reused
+  sep_table_prep(g, sg, ws);
   omega += (int64_t)blockIdx.y * 2 * g.M;
   ws += (int64_t)blockIdx.y * tg.plan_stride;
-  sep_table_prep(g, sg, ws, ws + tg.o_count + tg.NB);
   for (int m0 = blockIdx.x * blockDim.x; m0 < g.M; m0 += gridDim.x * blockDim.x) {
     const int m = m0 + threadIdx.x;
     const bool live = m < g.M;
@@ -1268,15 +1276,16 @@ __global__ void __launch_bounds__(256)
   }
   if (cache_hit(cache)) return;  // cached plan reused
   omega += (int64_t)blockIdx.y * 2 * g.M;
-  ws += (int64_t)blockIdx.y * tg.plan_stride;
+  int* const plan = ws + (int64_t)blockIdx.y * tg.plan_stride;
   for (int m0 = blockIdx.x * blockDim.x; m0 < g.M; m0 += nscatter * blockDim.x)
-    sep_spr_scatter_item(g, tg, sg, omega, ws, m0 + threadIdx.x);
+    sep_spr_scatter_item(g, tg, sg, omega, plan, ws, m0 + threadIdx.x);
 }
 
 // the adjoint's record and entries of sample m (m >= M: a dead lane that still takes part in the
 // wave-aggregated cursor increments)
 __device__ __forceinline__ void sep_spr_scatter_item(const Geom<float>& g, const TileGeom& tg, const SepGeom& sg,
-                                                     const float* __restrict__ omega, int* __restrict__ ws, int m) {
+                                                     const float* __restrict__ omega, int* __restrict__ plan,
+                                                     const int* __restrict__ tabs, int m) {
   const bool live = m < g.M;
   int tl[2][3], off[2][3], n[2];
   coil_sample_tiles(g, tg, omega, m, live, tl, off, n);
@@ -1287,13 +1296,12 @@ __device__ __forceinline__ void sep_spr_scatter_item(const Geom<float>& g, const
     a = sep_taps(g, 0, omega[m]);
     b = sep_taps(g, 1, omega[g.M + m]);
     theta = sample_theta<float, 2>(g, omega, m);
-    regular = ws[tg.o_count + tg.NB] == 0 && a.regular && b.regular;
+    regular = tabs[sg.o_flag] == 0 && a.regular && b.regular;
   }
-  const float* R0 = reinterpret_cast<const float*>(ws + sg.o_rtab[0]);
-  const float* R1 = reinterpret_cast<const float*>(ws + sg.o_rtab[1]);
-  const int nm10 = ws[sg.o_nm1], nm11 = ws[sg.o_nm1 + 1];
-  int* plan = ws;
-  SepRec* recs = reinterpret_cast<SepRec*>(reinterpret_cast<char*>(ws) + tg.o_rec_bytes);
+  const float* R0 = reinterpret_cast<const float*>(tabs + sg.o_rtab[0]);
+  const float* R1 = reinterpret_cast<const float*>(tabs + sg.o_rtab[1]);
+  const int nm10 = tabs[sg.o_nm1], nm11 = tabs[sg.o_nm1 + 1];
+  SepRec* recs = reinterpret_cast<SepRec*>(reinterpret_cast<char*>(plan) + tg.o_rec_bytes);
   const int c0 = live ? (int)sample_base_wrapped<float>(g, 0, omega[m]) : 0;
   const int c1 = live ? (int)sample_base_wrapped<float>(g, 1, omega[g.M + m]) : 0;
   SepRec rec;
@@ -1396,13 +1404,13 @@ __device__ __forceinline__ float2 sep_gat_complex(const Geom<float>& g, float om
 }
 
 // One work item: tile piece wi, chunk of ROWS coil rows; `plan`, `omega` and rows
-// [rowbase, rowbase + nrows) belong to one trajectory.  `region`: kGatCells * kPitch cells,
+// [rowbase, rowbase + nrows) belong to one trajectory, `tabs` to all.  `region`: kGatCells * kPitch cells,
 // `ph`: the phases P_0 of the region's rows and P_1 of its columns.
 template <int JF, int ROWS>
 __device__ __forceinline__ void gather_sep_item(const Geom<float>& g, const TileGeom& tg, const SepGeom& sg,
                                                 const float2* __restrict__ grid, const float* __restrict__ omega,
-                                                const int* plan, float2* kdata, int64_t rowbase, int64_t nrows,
-                                                int64_t wi, int chunk, float2* region, float2* ph) {
+                                                const int* plan, const int* tabs, float2* kdata, int64_t rowbase,
+                                                int64_t nrows, int64_t wi, int chunk, float2* region, float2* ph) {
   constexpr int kPitch = GatShape<ROWS>::kPitch, kThreads = GatShape<ROWS>::kThreads;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -1423,8 +1431,8 @@ __device__ __forceinline__ void gather_sep_item(const Geom<float>& g, const Tile
   float2* const p1 = ph + kGatR0;
   const auto phases = [&](int i) {  // i-th of the kGatR0 + kGatR1 phases
     const int d = i < kGatR0 ? 0 : 1;
-    const int nm1 = plan[sg.o_nm1 + d];
-    const double2* P = reinterpret_cast<const double2*>(plan + sg.o_ptab[d]);
+    const int nm1 = tabs[sg.o_nm1 + d];
+    const double2* P = reinterpret_cast<const double2*>(tabs + sg.o_ptab[d]);
     ph[i] = sep_cell_phase(P, g.K[d], nm1, d == 0 ? o0 + i : o1 + i - kGatR0);
   };
 
@@ -1538,7 +1546,7 @@ __global__ void __launch_bounds__(GatShape<ROWS>::kThreads)
   const int64_t b = blockIdx.y;  // trajectory
   const int64_t item = xcd_work_item(blockIdx.x, kXcdTiles * nchunk);
   const int64_t wi = item / nchunk;
-  gather_sep_item<JF, ROWS>(g, tg, sg, grid, omega + b * 2 * g.M, ws + b * tg.plan_stride, kdata,
+  gather_sep_item<JF, ROWS>(g, tg, sg, grid, omega + b * 2 * g.M, ws + b * tg.plan_stride, ws, kdata,
                             g.batched ? b * g.C : 0, g.batched ? g.C : g.B * g.C, wi, (int)(item - wi * nchunk), region,
                             ph);
 }
@@ -1636,12 +1644,13 @@ __device__ __forceinline__ float2 cmul_once(float2 a, float2 b) {
 
 // One work item: tile piece wi, chunk of coil rows, for one wave (ks = 1) or the whole group
 // (ks = kMmWaves, this wave its part `part`); `plan`, `omega` and rows [rowbase, rowbase +
-// nrows) belong to one trajectory.
+// nrows) belong to one trajectory, `tabs` to all.
 template <int G>
 __device__ __forceinline__ void spread_sep_item(const Geom<float>& g, const TileGeom& tg, const SepGeom& sg,
                                                 const float2* __restrict__ kdata, const float* __restrict__ omega,
-                                                const int* __restrict__ plan, float2* __restrict__ grid,
-                                                int64_t rowbase, int64_t nrows, int64_t wi, int chunk, int ks, int part,
+                                                const int* __restrict__ plan, const int* __restrict__ tabs,
+                                                float2* __restrict__ grid, int64_t rowbase, int64_t nrows, int64_t wi,
+                                                int chunk, int ks, int part,
                                                 MmLds<G>* group_lds, MmLds<G>& lds) {
   constexpr int kRows = mm_rows(G), kSP = mm_spitch(G);
   constexpr int kGroups = G >= 8 ? G / 8 : 0;  // rows form: 8 coil rows each
@@ -1669,15 +1678,15 @@ __device__ __forceinline__ void spread_sep_item(const Geom<float>& g, const Tile
   }
   const SepRec* recs = reinterpret_cast<const SepRec*>(reinterpret_cast<const char*>(plan) + tg.o_rec_bytes);
   const int* perm = plan + tg.o_perm + cstart;
-  const int odd0 = plan[sg.o_nm1] & 1, odd1 = plan[sg.o_nm1 + 1] & 1;
+  const int odd0 = tabs[sg.o_nm1] & 1, odd1 = tabs[sg.o_nm1 + 1] & 1;
   // a footprint's first cell relative to the tile, below 0 where it starts before the tile
   // or past the grid's end
   const auto rel = [](int cell, int o, int T, int K) { return cell - o < T ? cell - o : cell - o - K; };
   const int J0 = g.J[0];
 
   // phases of the tile's rows (lane n16: row n16) and of this lane's column, for the flush
-  const double2 pr16 = reinterpret_cast<const double2*>(plan + sg.o_ptab[0])[min(o0 + n16, g.K[0] - 1)];
-  const double2 pc = reinterpret_cast<const double2*>(plan + sg.o_ptab[1])[min(o1 + n16, g.K[1] - 1)];
+  const double2 pr16 = reinterpret_cast<const double2*>(tabs + sg.o_ptab[0])[min(o0 + n16, g.K[0] - 1)];
+  const double2 pc = reinterpret_cast<const double2*>(tabs + sg.o_ptab[1])[min(o1 + n16, g.K[1] - 1)];
 
   constexpr int kAcc = kGroups > 0 ? kGroups * kRegT0 : 2 * kRows;
   typedef typename MmSum<G>::vec Sum;
@@ -1944,7 +1953,7 @@ __global__ void __launch_bounds__(64 * kMmWaves) __attribute__((amdgpu_waves_per
   const int64_t b = blockIdx.y;  // trajectory
   const int64_t item = ks == 1 ? (int64_t)blockIdx.x * kMmWaves + wave : (int64_t)blockIdx.x;
   const int64_t wi = item / nchunk;
-  spread_sep_item<G>(g, tg, sg, kdata, omega + b * 2 * g.M, ws + b * tg.plan_stride, grid, g.batched ? b * g.C : 0,
+  spread_sep_item<G>(g, tg, sg, kdata, omega + b * 2 * g.M, ws + b * tg.plan_stride, ws, grid, g.batched ? b * g.C : 0,
                      g.batched ? g.C : g.B * g.C, wi, (int)(item - wi * nchunk), ks, wave, lds, lds[wave]);
 }
 
@@ -2279,11 +2288,17 @@ static TileGeom make_gather_geom(const tkbn_interp_desc* d);
 constexpr int kPlanSepGather = 6;
 constexpr int kPlanSepSpread = 7;
 
-// N - 1 and the real tables after the plan's int arrays; records 64-byte aligned after them
+// Records 64-byte aligned after a plan's int arrays; after all trajectories' plans what they
+// share: N - 1, the flag, cell phases and real tables.
 static void sep_finish_layout(TileGeom& tg, SepGeom& sg, int64_t o, const tkbn_interp_desc* d) {
+  o = (o + 15) & ~15LL;
+  tg.plan_ints = o;
+  tg.o_rec_bytes = o * 4;
+  tg.plan_stride = o + (tg.rec_entry ? tg.maxent : d->klength) * (int64_t)(sizeof(SepRec) / 4);
+  o = plans_of(d) * tg.plan_stride;
   sg.o_nm1 = o;
-  o += 2;
-  o = (o + 3) & ~3LL;
+  sg.o_flag = o + 2;
+  o += 4;
   for (int i = 0; i < 2; ++i) {
     sg.o_ptab[i] = o;
     o += 4 * d->grid_size[i];
@@ -2292,10 +2307,7 @@ static void sep_finish_layout(TileGeom& tg, SepGeom& sg, int64_t o, const tkbn_i
     sg.o_rtab[i] = o;
     o += d->numpoints[i] * d->table_oversamp[i] + 1;
   }
-  o = (o + 15) & ~15LL;
-  tg.plan_ints = o;
-  tg.o_rec_bytes = o * 4;
-  tg.plan_stride = o + (tg.rec_entry ? tg.maxent : d->klength) * (int64_t)(sizeof(SepRec) / 4);
+  sg.end = o;
 }
 
 static SepGeom sep_phase_of(const tkbn_interp_desc* d) {
@@ -2310,7 +2322,7 @@ static TileGeom make_sep_gather_geom(const tkbn_interp_desc* d, SepGeom* sg) {
   int64_t o = 0;
   tg.o_key = o;
   tg.o_perm = o;  // unused: the records carry the sample index
-  tg.o_count = o; o += tg.NB + 2;  // + the table flag, finished count blocks
+  tg.o_count = o; o += tg.NB + 1;  // + finished count blocks
   tg.o_start = o; o += tg.NB + 1;
   tg.o_cursor = o; o += tg.NB;
   tg.o_wstart = o; o += tg.NB + 1;
@@ -2333,7 +2345,7 @@ static TileGeom make_sep_spread_geom(const tkbn_interp_desc* d, SepGeom* sg) {
   int64_t o = 0;
   tg.o_key = o;
   tg.o_perm = o; o += tg.maxent;
-  tg.o_count = o; o += tg.NB + 2;  // + the table flag, finished count blocks
+  tg.o_count = o; o += tg.NB + 1;  // + finished count blocks
   tg.o_start = o; o += tg.NB + 1;
   tg.o_cursor = o; o += tg.NB;
   tg.o_wstart = o; o += tg.NB + 1;
@@ -2345,12 +2357,10 @@ static TileGeom make_sep_spread_geom(const tkbn_interp_desc* d, SepGeom* sg) {
   return tg;
 }
 
-static int64_t sep_workspace_bytes(const tkbn_interp_desc* d, const TileGeom& tg) {
-  return plan_cache_bytes(d) + plans_of(d) * tg.plan_stride * 4;
-}
 static int64_t sep_adj_bytes(const tkbn_interp_desc* d) {
   SepGeom sg;
-  return sep_workspace_bytes(d, make_sep_spread_geom(d, &sg));
+  make_sep_spread_geom(d, &sg);
+  return plan_cache_bytes(d) + sg.end * 4;
 }
 
 // The plan kernels of the separable gather (grid = nullptr) or spread, one plan per
@@ -2375,9 +2385,11 @@ static int sep_plan_launch(const tkbn_interp_desc* d, float2* grid, const Geom<f
   } else {
     CacheZero z;
     z.p = wsi + tg.o_count;
-    z.n = tg.NB + 2;
+    z.n = tg.NB + 1;
     z.stride = tg.plan_stride;
     z.copies = np;
+    z.p2 = wsi + sg.o_flag;
+    z.n2 = 1;
     const int st = plan_cache_begin(d, kind, tg.T, om, ws, s, &cache, z);
     if (st != TKBN_OK) return st;
     if (spread)
@@ -3222,7 +3234,8 @@ static TileGeom make_gather_geom(const tkbn_interp_desc* d) {
 
 static int64_t sep_fwd_bytes(const tkbn_interp_desc* d) {
   SepGeom sg;
-  return sep_workspace_bytes(d, make_sep_gather_geom(d, &sg));
+  make_sep_gather_geom(d, &sg);
+  return plan_cache_bytes(d) + sg.end * 4;
 }
 
 int64_t interp_fwd_workspace_bytes(const tkbn_interp_desc* d) {
@@ -3410,9 +3423,11 @@ __global__ void __launch_bounds__(GatShape<ROWS>::kThreads)
   const int64_t wi = li / q.yf;
   const int yc = (int)(li - wi * q.yf);
   if (q.g.J[0] == 6 && q.g.J[1] == 6)
-    gather_sep_item<6, ROWS>(q.g, q.tf, q.sf, q.grid_in, q.omega, q.wf, q.kdata_out, 0, q.g.B * q.g.C, wi, yc, region, ph);
+    gather_sep_item<6, ROWS>(q.g, q.tf, q.sf, q.grid_in, q.omega, q.wf, q.wf, q.kdata_out, 0, q.g.B * q.g.C, wi, yc, region,
+                             ph);
   else
-    gather_sep_item<0, ROWS>(q.g, q.tf, q.sf, q.grid_in, q.omega, q.wf, q.kdata_out, 0, q.g.B * q.g.C, wi, yc, region, ph);
+    gather_sep_item<0, ROWS>(q.g, q.tf, q.sf, q.grid_in, q.omega, q.wf, q.wf, q.kdata_out, 0, q.g.B * q.g.C, wi, yc, region,
+                             ph);
 }
 
 template <int G>
@@ -3427,8 +3442,8 @@ __global__ void __launch_bounds__(64 * kMmWaves) __attribute__((amdgpu_waves_per
   if (!q.sep_a) return;
   const int li = item - off[p];
   const int64_t wi = li / q.ya;
-  spread_sep_item<G>(q.g, q.ta, q.sa, q.kdata_in, q.omega, q.wa, q.grid_out, 0, q.g.B * q.g.C, wi, (int)(li - wi * q.ya),
-                     ks, wave, lds, lds[wave]);
+  spread_sep_item<G>(q.g, q.ta, q.sa, q.kdata_in, q.omega, q.wa, q.wa, q.grid_out, 0, q.g.B * q.g.C, wi,
+                     (int)(li - wi * q.ya), ks, wave, lds, lds[wave]);
 }
 
 }  // namespace tkbn
