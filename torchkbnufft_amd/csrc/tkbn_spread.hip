@@ -57,10 +57,10 @@ struct TileGeom {
   int64_t o_key, o_perm, o_count, o_start, o_cursor, o_wstart, o_work, o_nwork, plan_ints;
   int64_t o_maxabs_bytes;  // byte offset of the max|kdata| slot (8 bytes)
   FastDiv fT[3], fl[3], fR[3], ftc, frc;  // dividers by T, lstride, R, tcells, rcells
-  int64_t nkeys;           // multi-coil plan: (tile, footprint column) keys
-  int64_t o_hot, o_cold;   // multi-coil plan: scans of split / unsplit tiles
-  int64_t o_rec_bytes;     // multi-coil plan: byte offset of the entry records
-  int64_t plan_stride;     // multi-coil plan: ints from one trajectory's plan to the next
+  FastDiv ftarget;         // separable plan: divider by target
+  int64_t o_rec_bytes;     // separable plan: byte offset of the records
+  int64_t plan_stride;     // separable plan: ints from one trajectory's plan to the next
+  int64_t o_hot;                             // 3-D register-tile plan: list of split tiles
   int64_t o_meta, o_tmp, o_sort, o_scratch;  // 3-D register-tile plan: counts, scan scratch, sort
   int64_t o_sw, o_sb;                        // 3-D register-tile plan: per-sample tap weights, bases
   int64_t pool_off_bytes, pool_slots;        // 3-D register-tile plan: piece partials
@@ -1098,52 +1098,124 @@ __device__ __forceinline__ void sep_spr_scatter_item(const Geom<float>& g, const
 // 1/2, 1/4, 1/8 of the target, the rest), so that no long tile starts late (16 coils x 4,
 // 320^2 radial: the spread's waves were 1.2 per SIMD on average with the tiles in grid
 // order, 2 fit).  Empty tiles get no item when `skip_empty`.
+// One block does it, so it is bound by its own chain of loads and barriers: one pass adds the
+// classes up, one scans entries, pieces and classes together, 2048 tiles a round, the next
+// round's counts loaded ahead (16384 tiles, 4000 samples: the count kernel with its scan 65 us,
+// 368 with a block scan each of entries, pieces and four classes; 1024 tiles, 206 k samples: 39
+// and 62 us).
 constexpr int kSepClasses = 4;
-__device__ __forceinline__ void sep_plan_scan(const TileGeom& tg, int* __restrict__ plan, bool skip_empty, int* sbuf) {
-  const int target = tg.target;
+constexpr int kScanTiles = 8;  // tiles of a thread per round
+struct SepSums {
+  int ent, pieces;
+  unsigned long long cls;  // classes 1 .. 4, 16 bits each (a round has at most 2048 tiles)
+};
+__device__ __forceinline__ SepSums sep_add(SepSums a, SepSums b) {
+  return SepSums{a.ent + b.ent, a.pieces + b.pieces, a.cls + b.cls};
+}
+struct SepScanLds {
+  SepSums wave[4];
+  int total[kSepClasses + 1];
+};
+__device__ __forceinline__ void sep_plan_scan(const TileGeom& tg, int* __restrict__ plan, bool skip_empty,
+                                              SepScanLds& lds) {
+  const int target = tg.target, NB = tg.NB;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;  // 256 threads
   const int* count = plan + tg.o_count;
   int* start = plan + tg.o_start;
   int* cursor = plan + tg.o_cursor;
   int* wstart = plan + tg.o_wstart;
   int* work = plan + tg.o_work;
-  int* hot = plan + tg.o_hot;
-  int* rank = plan + tg.o_cold;
-  const int NB = tg.NB;
   const auto size_class = [&](int v) {  // 0: split; kSepClasses + 1: no item
     if (v > target) return 0;
     if (v == 0 && skip_empty) return kSepClasses + 1;
     return 2 * v > target ? 1 : 4 * v > target ? 2 : 8 * v > target ? 3 : 4;
   };
-  block_exclusive_scan(count, start, NB, sbuf);
-  for (int t = threadIdx.x; t < NB; t += blockDim.x) {
-    cursor[t] = start[t];
-    const int v = count[t];
-    work[t] = v > target ? (v + target - 1) / target : 0;
+  const auto sums_of = [&](int v) {
+    const int c = size_class(v);
+    return SepSums{v, c == 0 ? (int)fdiv(v + target - 1, tg.ftarget) : 0, c >= 1 && c <= kSepClasses ? 1ull << (16 * (c - 1)) : 0ull};
+  };
+  if (tid <= kSepClasses) lds.total[tid] = 0;
+  __syncthreads();
+  int mine[kSepClasses + 1] = {0, 0, 0, 0, 0};
+  for (int t0 = tid; t0 < NB; t0 += kScanTiles * 256) {
+    int v[kScanTiles];
+    SepSums a{0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < kScanTiles; ++i) v[i] = count[min(t0 + i * 256, NB - 1)];
+#pragma unroll
+    for (int i = 0; i < kScanTiles; ++i)
+      if (t0 + i * 256 < NB) a = sep_add(a, sums_of(v[i]));
+    mine[0] += a.pieces;
+#pragma unroll
+    for (int c = 0; c < kSepClasses; ++c) mine[c + 1] += (int)((a.cls >> (16 * c)) & 0xffff);
+  }
+#pragma unroll
+  for (int c = 0; c <= kSepClasses; ++c) {
+    for (int off = 32; off > 0; off >>= 1) mine[c] += __shfl_down(mine[c], off, 64);
+    if (lane == 0 && mine[c] != 0) atomicAdd(&lds.total[c], mine[c]);
   }
   __syncthreads();
-  block_exclusive_scan(work, hot, NB, sbuf);
-  int nwork = hot[NB];
-  __syncthreads();  // `work` and `cursor` are the scans' scratch below
-  for (int t = threadIdx.x; t < NB; t += blockDim.x)
-    if (size_class(count[t]) == 0) wstart[t] = hot[t];
-  for (int c = 1; c <= kSepClasses; ++c) {
-    for (int t = threadIdx.x; t < NB; t += blockDim.x) work[t] = size_class(count[t]) == c ? 1 : 0;
-    __syncthreads();
-    block_exclusive_scan(work, rank, NB, sbuf);
-    for (int t = threadIdx.x; t < NB; t += blockDim.x)
-      if (size_class(count[t]) == c) wstart[t] = nwork + rank[t];
-    nwork += rank[NB];
-    __syncthreads();
-  }
+  // next item of each class, entries so far
+  int next[kSepClasses + 1], ent = 0;
+  next[0] = 0;
+#pragma unroll
+  for (int c = 1; c <= kSepClasses; ++c) next[c] = next[c - 1] + lds.total[c - 1];
   const int cap = (int)tg.maxwork;
-  for (int t = threadIdx.x; t < NB; t += blockDim.x) {
-    const int c = size_class(count[t]);
-    if (c > kSepClasses) continue;
-    const int items = c == 0 ? hot[t + 1] - hot[t] : 1;
-    const int a = wstart[t], e = min(a + items, cap);
-    for (int w = a; w < e; ++w) work[w] = t;
+  if (tid == 0) plan[tg.o_nwork] = min(next[kSepClasses] + lds.total[kSepClasses], cap);
+
+  int ahead[kScanTiles];  // the next round's counts
+#pragma unroll
+  for (int i = 0; i < kScanTiles; ++i) ahead[i] = count[min(kScanTiles * tid + i, NB - 1)];
+  for (int t0 = 0; t0 < NB; t0 += kScanTiles * 256) {
+    const int t = t0 + kScanTiles * tid;
+    int v[kScanTiles];
+    SepSums sum{0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < kScanTiles; ++i) {
+      v[i] = ahead[i];
+      ahead[i] = count[min(t + kScanTiles * 256 + i, NB - 1)];
+    }
+#pragma unroll
+    for (int i = 0; i < kScanTiles; ++i)
+      if (t + i < NB) sum = sep_add(sum, sums_of(v[i]));
+    SepSums incl = sum;
+    for (int off = 1; off < 64; off <<= 1) {
+      const SepSums o{__shfl_up(incl.ent, off, 64), __shfl_up(incl.pieces, off, 64), __shfl_up(incl.cls, off, 64)};
+      if (lane >= off) incl = sep_add(incl, o);
+    }
+    if (lane == 63) lds.wave[wave] = incl;
+    __syncthreads();
+    SepSums run{incl.ent - sum.ent, incl.pieces - sum.pieces, incl.cls - sum.cls}, all{0, 0, 0};
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      if (w < wave) run = sep_add(run, lds.wave[w]);
+      all = sep_add(all, lds.wave[w]);
+    }
+    __syncthreads();  // the next round overwrites the waves' sums
+#pragma unroll
+    for (int i = 0; i < kScanTiles; ++i) {
+      if (t + i < NB) {
+        const int c = size_class(v[i]);
+        const SepSums one = sums_of(v[i]);
+        start[t + i] = cursor[t + i] = ent + run.ent;
+        int at = 0;  // (a select each: an indexed register array would go through memory)
+#pragma unroll
+        for (int k = 0; k <= kSepClasses; ++k)
+          if (c == k) at = next[k] + (k == 0 ? run.pieces : (int)((run.cls >> (16 * (k - 1))) & 0xffff));
+        if (c <= kSepClasses) {
+          wstart[t + i] = at;
+          const int e = min(at + (c == 0 ? one.pieces : 1), cap);
+          for (int w = at; w < e; ++w) work[w] = t + i;
+        }
+        run = sep_add(run, one);
+      }
+    }
+    ent += all.ent;
+    next[0] += all.pieces;
+#pragma unroll
+    for (int k = 1; k <= kSepClasses; ++k) next[k] += (int)((all.cls >> (16 * (k - 1))) & 0xffff);
   }
-  if (threadIdx.x == 0) plan[tg.o_nwork] = min(nwork, cap);
+  if (tid == 0) start[NB] = ent;
 }
 
 // The count kernels' end: the last block of a trajectory to finish scans its counts (its
@@ -1152,7 +1224,7 @@ __device__ __forceinline__ void sep_plan_scan(const TileGeom& tg, int* __restric
 // off; nothing else is read here (a release fence by every block wrote the L2 back 800
 // times: 69 instead of 62 us for 206 000 new samples).
 __device__ __forceinline__ void sep_scan_if_last(const TileGeom& tg, int* __restrict__ plan, bool skip_empty) {
-  __shared__ int sbuf[256];
+  __shared__ SepScanLds lds;
   __shared__ bool last;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
@@ -1160,7 +1232,7 @@ __device__ __forceinline__ void sep_scan_if_last(const TileGeom& tg, int* __rest
   __syncthreads();
   if (!last) return;
   __threadfence();
-  sep_plan_scan(tg, plan, skip_empty, sbuf);
+  sep_plan_scan(tg, plan, skip_empty, lds);
 }
 
 // Forward: each sample once, in the 16 x 16 tile of its base cell (trajectory order
@@ -2238,6 +2310,7 @@ static TileGeom make_coil_tile_geom(const tkbn_interp_desc* d) {
   }
   tg.maxent = per_sample * d->klength;
   tg.maxwork = tg.NB + tg.maxent / tg.target + 1;  // sum of ceil(V / target)
+  tg.ftarget = make_fastdiv((uint32_t)tg.target);
   return tg;
 }
 
@@ -2328,8 +2401,6 @@ static TileGeom make_sep_gather_geom(const tkbn_interp_desc* d, SepGeom* sg) {
   tg.o_wstart = o; o += tg.NB + 1;
   tg.o_work = o; o += (tg.maxwork > tg.NB ? tg.maxwork : tg.NB);
   tg.o_nwork = o; o += 1;
-  tg.o_hot = o; o += tg.NB + 1;
-  tg.o_cold = o; o += tg.NB + 1;
   sep_finish_layout(tg, *sg, o, d);
   return tg;
 }
@@ -2351,8 +2422,6 @@ static TileGeom make_sep_spread_geom(const tkbn_interp_desc* d, SepGeom* sg) {
   tg.o_wstart = o; o += tg.NB + 1;
   tg.o_work = o; o += (tg.maxwork > tg.NB ? tg.maxwork : tg.NB);
   tg.o_nwork = o; o += 1;
-  tg.o_hot = o; o += tg.NB + 1;
-  tg.o_cold = o; o += tg.NB + 1;
   sep_finish_layout(tg, *sg, o, d);
   return tg;
 }
@@ -3215,20 +3284,7 @@ static TileGeom make_gather_geom(const tkbn_interp_desc* d) {
   const int64_t M = d->klength;
   tg.maxent = M;
   tg.maxwork = tg.NB + M / tg.target + 1;
-  int64_t o = 0;
-  tg.o_key = o;
-  tg.o_perm = o; o += tg.maxent;
-  tg.o_count = o; o += tg.NB;
-  tg.o_start = o; o += tg.NB + 1;
-  tg.o_cursor = o; o += tg.NB;
-  tg.o_wstart = o; o += tg.NB + 1;
-  tg.o_work = o; o += (tg.maxwork > tg.NB ? tg.maxwork : tg.NB);
-  tg.o_nwork = o; o += 1;
-  tg.o_hot = o; o += tg.NB + 1;
-  tg.o_cold = o; o += tg.NB + 1;
-  o = (o + 3) & ~3LL;
-  tg.plan_ints = o;
-  tg.o_rec_bytes = o * 4;
+  tg.ftarget = make_fastdiv((uint32_t)tg.target);
   return tg;
 }
 
