@@ -8,8 +8,9 @@ iterations of ATen gathers and ``index_add_`` calls.
 from __future__ import annotations
 
 import ctypes
+import threading
 from collections import OrderedDict
-from typing import List, Optional, Sequence
+from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
 from torch import Tensor
@@ -34,11 +35,35 @@ _WORKSPACES_MAX = 256  # entries
 _WORKSPACES_MAX_BYTES = 8 << 30
 
 
+# torch's allocator asks the device for every tensor above 10 MiB it has no free block for, at
+# 25 to 450 us each, and a trajectory whose plans take 16 MiB needs two: the first pair on
+# one more trajectory of 206 000 samples took 390 to 440 us, 260 with memory at hand.  So
+# workspaces of that size are cut from blocks of four.  A block is given back when none of
+# its workspaces is held any more (the newest one of each device and stream: by
+# clear_plan_cache).
+_BLOCK_BYTES = (10 << 20, 64 << 20)
+_BLOCK_COUNT = 4
+_BLOCKS: Dict[tuple, Tuple[Tensor, int]] = {}
+_BLOCKS_LOCK = threading.Lock()
+
+
+def _new_workspace(like: Tensor, nbytes: int) -> Tensor:
+    if not _BLOCK_BYTES[0] < nbytes <= _BLOCK_BYTES[1] or torch.cuda.is_current_stream_capturing():
+        return torch.empty(nbytes, dtype=torch.uint8, device=like.device)
+    key, size = (like.device, _lib.stream_of(like)), -(-nbytes // 512) * 512
+    with _BLOCKS_LOCK:
+        block, used = _BLOCKS.get(key, (None, 0))
+        if block is None or used + size > block.numel():
+            block, used = torch.empty(_BLOCK_COUNT * size, dtype=torch.uint8, device=like.device), 0
+        _BLOCKS[key] = (block, used + size)
+    return block[used : used + nbytes]
+
+
 def _plan_workspace(kind: str, omega: Tensor, like: Tensor, nbytes: int) -> Tensor:
     key = (kind, like.device, _lib.stream_of(like), omega.data_ptr(), tuple(omega.shape), omega.dtype)
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(max(nbytes, _lib.PLAN_CACHE_HEADER_BYTES), dtype=torch.uint8, device=like.device)
+        ws = _new_workspace(like, max(nbytes, _lib.PLAN_CACHE_HEADER_BYTES))
         ws[: _lib.PLAN_CACHE_HEADER_BYTES].zero_()  # a zero header never matches: first call builds
         _WORKSPACES[key] = ws
         while len(_WORKSPACES) > 1 and (
@@ -53,6 +78,8 @@ def _plan_workspace(kind: str, omega: Tensor, like: Tensor, nbytes: int) -> Tens
 def clear_plan_cache() -> None:
     """Release the workspaces that hold cached trajectory plans."""
     _WORKSPACES.clear()
+    with _BLOCKS_LOCK:
+        _BLOCKS.clear()
 
 
 def set_binned_forward_threshold(work: int) -> None:
