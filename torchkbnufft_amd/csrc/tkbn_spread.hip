@@ -2268,8 +2268,9 @@ static int64_t sep_entries(const tkbn_interp_desc* d) { return plans_of(d) * (d-
 // Waves that share a tile's entries: the whole group where the tiles x chunks alone do not
 // fill the chip (4096 waves) and hold at least a batch of entries each (39 rows, 434 x 362:
 // 142 -> 77 us, 12 rows, 512^2: 75 -> 51 us; 64 rows, 640^2, the other way: 216 -> 273 us).
-static int mm_waves_per_item(int64_t entries, int64_t tiles, int64_t chunks) {
-  return tiles * chunks < 4096 && entries >= kMmBatch * tiles ? kMmWaves : 1;
+// `items`: tiles x chunks.  A launch's own choice: the pieces of a plan do not depend on it.
+static int mm_waves_per_item(int64_t entries, int64_t tiles, int64_t items) {
+  return items < 4096 && entries >= kMmBatch * tiles ? kMmWaves : 1;
 }
 
 static TileGeom make_coil_tile_geom(const tkbn_interp_desc* d) {
@@ -2536,7 +2537,7 @@ static int spread_sep_launch(const tkbn_interp_desc* d, const void* kdata, const
   const int64_t nrows = rows_of(d), np = plans_of(d);
   const int form = mm_form(d);
   const int nchunk = (int)ceil_div(nrows, mm_rows(form));
-  const int ks = mm_waves_per_item(sep_entries(d), tg.NB * plans_of(d), nchunk);
+  const int ks = mm_waves_per_item(sep_entries(d), tg.NB * np, tg.NB * np * nchunk);
   const int64_t groups = ceil_div(tg.maxwork * nchunk, kMmWaves / ks);
   TKBN_REQUIRE(groups < (1LL << 31), TKBN_ERR_UNSUPPORTED, "too many coil rows x work items for one launch");
   const dim3 grd((unsigned)groups, (unsigned)np), blk(64 * kMmWaves);
@@ -3560,7 +3561,7 @@ int tkbn_batch_create(const tkbn_interp_desc* descs, const tkbn_interp_desc* adj
   b->det = mode == TKBN_ADJ_DETERMINISTIC ? 1 : 0;
   b->ndim = descs[0].ndim;
   b->jm = max_numpoints(&descs[0]) <= 6 ? 6 : 16;
-  int64_t zoff = 0, entries = 0, tiles = 0;
+  int64_t zoff = 0, entries = 0, tiles = 0, items = 0;
   for (int p = 0; p < nprob; ++p) {
     const tkbn_interp_desc* d = &descs[p];
     const tkbn_interp_desc* da = adj_descs ? &adj_descs[p] : d;
@@ -3627,12 +3628,12 @@ int tkbn_batch_create(const tkbn_interp_desc* descs, const tkbn_interp_desc* adj
     b->wsf.push_back(fwd_workspaces[p]);
     b->wsa.push_back(adj_workspaces[p]);
   }
-  b->ks = mm_waves_per_item(entries, tiles, 1);
   // row chunks per work item: one shape for all separable problems of a launch
   for (int p = 0; p < nprob; ++p) {
     BatchProb& q = b->probs[p];
     q.yf = ceil_div(b->rows[p], q.sep_f ? b->gat_rows : q.tf.CC);
     q.ya = ceil_div(b->rows[p], q.sep_a ? mm_rows(b->form) : q.ta.CC);
+    if (q.sep_a) items += q.ta.NB * q.ya;
     q.zoff = zoff;
     zoff += (int64_t)q.ta.NB * q.ya;
     if (!q.sep_f) b->lds_f = std::max(b->lds_f, (size_t)q.tf.CC * q.tf.rcells * sizeof(float2));
@@ -3641,6 +3642,7 @@ int tkbn_batch_create(const tkbn_interp_desc* descs, const tkbn_interp_desc* adj
     b->bound_a += q.ta.maxwork * q.ya;
   }
   b->zblocks = zoff;
+  b->ks = mm_waves_per_item(entries, tiles, items);  // of all problems: together they fill the chip
   if (b->bound_f >= (1LL << 31) || b->bound_a >= (1LL << 31) || b->zblocks >= (1LL << 31)) {
     set_error("tkbn_batch_create: too many work items for one launch");
     delete b;
