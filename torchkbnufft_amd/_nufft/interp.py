@@ -38,47 +38,70 @@ _WORKSPACES_MAX_BYTES = 8 << 30
 # torch's allocator asks the device for every tensor above 10 MiB it has no free block for, at
 # 25 to 450 us each, and a trajectory whose plans take 16 MiB needs two: the first pair on
 # one more trajectory of 206 000 samples took 390 to 440 us, 260 with memory at hand.  So
-# workspaces of that size are cut from blocks of four.  A block is given back when none of
-# its workspaces is held any more (the newest one of each device and stream: by
-# clear_plan_cache).
+# workspaces of that size are cut from blocks of four.  A block counts whole against the limit
+# while any of its workspaces is held and is given back with the last one; the block being cut
+# is kept beside them, one per device and stream, of the last few streams.
 _BLOCK_BYTES = (10 << 20, 64 << 20)
 _BLOCK_COUNT = 4
-_BLOCKS: Dict[tuple, Tuple[Tensor, int]] = {}
-_BLOCKS_LOCK = threading.Lock()
+_BLOCKS: "OrderedDict[tuple, Tuple[Tensor, int]]" = OrderedDict()
+_BLOCKS_MAX = 4
+_LOCK = threading.Lock()
+_HELD: Dict[int, List[int]] = {}  # memory of _WORKSPACES: address -> [workspaces, bytes]
 
 
 def _new_workspace(like: Tensor, nbytes: int) -> Tensor:
     if not _BLOCK_BYTES[0] < nbytes <= _BLOCK_BYTES[1] or torch.cuda.is_current_stream_capturing():
         return torch.empty(nbytes, dtype=torch.uint8, device=like.device)
     key, size = (like.device, _lib.stream_of(like)), -(-nbytes // 512) * 512
-    with _BLOCKS_LOCK:
-        block, used = _BLOCKS.get(key, (None, 0))
-        if block is None or used + size > block.numel():
+    block, used = _BLOCKS.pop(key, (None, 0))
+    if block is None or used + size > block.numel():
+        try:
             block, used = torch.empty(_BLOCK_COUNT * size, dtype=torch.uint8, device=like.device), 0
-        _BLOCKS[key] = (block, used + size)
+        except torch.cuda.OutOfMemoryError:
+            return torch.empty(nbytes, dtype=torch.uint8, device=like.device)
+    _BLOCKS[key] = (block, used + size)
+    while len(_BLOCKS) > _BLOCKS_MAX:
+        _BLOCKS.popitem(last=False)
     return block[used : used + nbytes]
+
+
+def _hold(ws: Tensor) -> None:
+    memory = ws.untyped_storage()
+    _HELD.setdefault(memory.data_ptr(), [0, memory.nbytes()])[0] += 1
+
+
+def _drop(ws: Tensor) -> None:
+    at = ws.untyped_storage().data_ptr()
+    _HELD[at][0] -= 1
+    if _HELD[at][0] == 0:
+        del _HELD[at]
 
 
 def _plan_workspace(kind: str, omega: Tensor, like: Tensor, nbytes: int) -> Tensor:
     key = (kind, like.device, _lib.stream_of(like), omega.data_ptr(), tuple(omega.shape), omega.dtype)
-    ws = _WORKSPACES.get(key)
-    if ws is None or ws.numel() < nbytes:
+    with _LOCK:
+        ws = _WORKSPACES.get(key)
+        if ws is not None and ws.numel() >= nbytes:
+            _WORKSPACES.move_to_end(key)
+            return ws
+        if ws is not None:
+            _drop(_WORKSPACES.pop(key))
         ws = _new_workspace(like, max(nbytes, _lib.PLAN_CACHE_HEADER_BYTES))
         ws[: _lib.PLAN_CACHE_HEADER_BYTES].zero_()  # a zero header never matches: first call builds
+        _hold(ws)
         _WORKSPACES[key] = ws
         while len(_WORKSPACES) > 1 and (
-            len(_WORKSPACES) > _WORKSPACES_MAX or sum(w.numel() for w in _WORKSPACES.values()) > _WORKSPACES_MAX_BYTES
+            len(_WORKSPACES) > _WORKSPACES_MAX or sum(n for _, n in _HELD.values()) > _WORKSPACES_MAX_BYTES
         ):
-            _WORKSPACES.popitem(last=False)
-    else:
-        _WORKSPACES.move_to_end(key)
+            _drop(_WORKSPACES.popitem(last=False)[1])
     return ws
 
 
 def clear_plan_cache() -> None:
     """Release the workspaces that hold cached trajectory plans."""
-    _WORKSPACES.clear()
-    with _BLOCKS_LOCK:
+    with _LOCK:
+        _WORKSPACES.clear()
+        _HELD.clear()
         _BLOCKS.clear()
 
 
