@@ -193,6 +193,18 @@ def _smooth(im, gs) -> bool:
     return ok
 
 
+def _combines(im, gs) -> bool:
+    """The adjoint's last pass can sum the coils: where the last dimension is no convolution (a
+    line's workspace then holds no chirp, as that of one value)."""
+    key = (int(im[-1]), int(gs[-1]), "combine")
+    ok = _FUSED_OK.get(key)
+    if ok is None:
+        size = _lib.load().tkbn_fft_any_workspace_bytes
+        ok = size(1, _lib.i64_array(key[:1]), _lib.i64_array(key[1:2]), 1, 1) == size(1, _lib.i64_array([1]), _lib.i64_array([1]), 1, 1)
+        _FUSED_OK[key] = ok
+    return ok
+
+
 def _out_or_new(out: Optional[Tensor], shape: tuple, like: Tensor) -> Tensor:
     if out is None:
         return torch.empty(shape, dtype=like.dtype, device=like.device)
@@ -263,7 +275,7 @@ def fft_grid_adj(grid: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, im
             raise ValueError(f"smaps shape {tuple(smaps.shape)} does not match data ({B}, {C}) + {im}")
     sc = plain(scaling_coef.to(device=grid.device, dtype=grid.dtype))
     smooth = _smooth(im, gs)
-    combine = smaps is not None and not smooth  # the convolution passes leave the coils apart
+    combine = smaps is not None and not _combines(im, gs)  # a convolution leaves the coils apart
     out = _out_or_new(out, (B, 1 if smaps is not None else C) + im, grid)
     image = torch.empty((B, C) + im, dtype=grid.dtype, device=grid.device) if combine else out
     ws, nws = _fft_workspace(grid.device, d, im, gs, B, C, smooth)
