@@ -158,6 +158,13 @@ __device__ __forceinline__ float2 mul_root(float2 a) {
 template <int R>
 __device__ __forceinline__ void dft(float2* x);
 
+// the multiple of A below A * B that is 1 modulo B
+constexpr int unit_multiple(int A, int B) {
+  int m = A;
+  while (m % B != 1) m += A;
+  return m;
+}
+
 // R = A * B: A-point DFTs over the inputs n2 + B n1, roots, B-point DFTs
 template <int A, int B, int N2, int K1>
 __device__ __forceinline__ void mul_roots_row(float2 (&y)[A]) {
@@ -188,6 +195,32 @@ __device__ __forceinline__ void dft_ab(float2* x) {
     dft<B>(z);
 #pragma unroll
     for (int k2 = 0; k2 < B; ++k2) x[k1 + A * k2] = z[k2];
+  }
+}
+
+// R = A * B without a common factor: A-point and B-point DFTs with no roots between them (Good,
+// "The interaction algorithm and practical Fourier analysis", 1958): input B n1 + A n2, output
+// congruent to k1 modulo A and to k2 modulo B.  The roots that dft_ab multiplies by cost
+// roundings beside their work: 1000 = 10 * 10 * 10 was 5 to 14 % further from 64-bit values
+// than passes of radices 8 and below, 216 = 6 * 6 * 6 7 to 12 %.
+template <int A, int B>
+__device__ __forceinline__ void dft_coprime(float2* x) {
+  constexpr int R = A * B, E1 = unit_multiple(B, A), E2 = unit_multiple(A, B);
+  float2 y[B][A];
+#pragma unroll
+  for (int n2 = 0; n2 < B; ++n2) {
+#pragma unroll
+    for (int n1 = 0; n1 < A; ++n1) y[n2][n1] = x[(B * n1 + A * n2) % R];
+    dft<A>(y[n2]);
+  }
+#pragma unroll
+  for (int k1 = 0; k1 < A; ++k1) {
+    float2 z[B];
+#pragma unroll
+    for (int n2 = 0; n2 < B; ++n2) z[n2] = y[n2][k1];
+    dft<B>(z);
+#pragma unroll
+    for (int k2 = 0; k2 < B; ++k2) x[(E1 * k1 + E2 * k2) % R] = z[k2];
   }
 }
 
@@ -263,13 +296,13 @@ __device__ __forceinline__ void dft(float2* x) {
   } else if constexpr (R == 3 || R == 5 || R == 7 || R == 11 || R == 13 || R == 17) {
     dft_prime<R>(x);
   } else if constexpr (R == 6) {
-    dft_ab<2, 3>(x);
+    dft_coprime<2, 3>(x);
   } else if constexpr (R == 9) {
     dft_ab<3, 3>(x);
   } else if constexpr (R == 10) {
-    dft_ab<2, 5>(x);
+    dft_coprime<2, 5>(x);
   } else if constexpr (R == 12) {
-    dft_ab<4, 3>(x);
+    dft_coprime<4, 3>(x);
   } else if constexpr (R == 16) {
     dft_ab<4, 4>(x);
   } else {
