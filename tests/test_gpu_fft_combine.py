@@ -1,5 +1,6 @@
 """Adjoint FFT with coil maps on grids that are not products of 2, 3, 5: the last pass sums the
-coils itself wherever the last dimension is no convolution, whatever the others are.
+coils itself wherever the last dimension is no convolution and is short enough, whatever the
+others are.
 
 Tolerance: per dimension at most a convolution's rms error, (2 log2(M) + 6) * 2^-24 * 0.6 =
 9.3e-7 for M <= 1280 (a planned dimension has less than half); two dimensions, the maps' product
@@ -15,16 +16,22 @@ DEV = "cuda:0"
 TOL = 2e-6
 
 # (image, grid, coils, combined by the last pass): last dimensions of primes 7 to 17, one lone
-# radix, a smooth one, the largest image line; coils on both sides of a group's lines (16 at
-# most, fewer where LDS holds no more); a convolution before the last dimension, and as the last
+# radix, a smooth one, the longest line; coils on both sides of a group's lines (16 at most, fewer
+# where LDS holds no more), in several rounds where there are 256 lines of the image; a convolution
+# before the last dimension, and as the last
 CASES = [
     ((9, 13), (18, 26), 3, True),
-    ((9, 11), (18, 11), 17, True),
-    ((33, 24), (66, 48), 40, True),
+    ((9, 11), (18, 11), 16, True),
+    ((9, 11), (18, 11), 17, False),
+    ((128, 24), (143, 48), 40, True),
+    ((127, 24), (254, 48), 40, False),
+    ((128, 45), (130, 91), 17, True),
     ((31, 13), (62, 26), 5, True),
     ((19, 45), (38, 90), 16, True),
-    ((3, 1000), (6, 1001), 7, True),
-    ((2, 1024), (4, 2002), 4, True),
+    ((3, 385), (7, 770), 16, True),
+    ((3, 400), (7, 800), 11, True),
+    ((3, 401), (7, 819), 11, False),
+    ((2, 1024), (4, 2002), 4, False),
     ((7,), (14,), 9, True),
     ((5, 6, 7), (11, 12, 14), 6, True),
     ((13, 31), (26, 62), 5, False),

@@ -193,9 +193,16 @@ def _smooth(im, gs) -> bool:
     return ok
 
 
-def _combines(im, gs) -> bool:
-    """The adjoint's last pass can sum the coils: where the last dimension is no convolution (a
-    line's workspace then holds no chirp, as that of one value)."""
+def _combines(im, gs, B: int, C: int) -> bool:
+    """The adjoint's last pass sums the coils itself on a grid of any factors: where the last
+    dimension is no convolution (a line's workspace then holds no chirp, as that of one value),
+    and where a group per line of the image, which takes the coils in turn, is no slower than
+    the coils' images apart and summed by another kernel.  That is up to 800 values a line
+    (longer ones leave a group few coils at once: 8 coils, 490^2 -> 980^2 88 us apart, 94 combined,
+    385^2 -> 770^2 65 and 52), with a group for every CU or no more than one round of coils
+    (32 coils, 182^2 -> 364^2 42 and 48; 12 coils 28 and 24; 308^2 -> 616^2 119 and 85)."""
+    if int(gs[-1]) > 800 or (C > 16 and B * math.prod(int(n) for n in im[:-1]) < 256):
+        return False
     key = (int(im[-1]), int(gs[-1]), "combine")
     ok = _FUSED_OK.get(key)
     if ok is None:
@@ -275,7 +282,7 @@ def fft_grid_adj(grid: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, im
             raise ValueError(f"smaps shape {tuple(smaps.shape)} does not match data ({B}, {C}) + {im}")
     sc = plain(scaling_coef.to(device=grid.device, dtype=grid.dtype))
     smooth = _smooth(im, gs)
-    combine = smaps is not None and not _combines(im, gs)  # a convolution leaves the coils apart
+    combine = smaps is not None and not smooth and not _combines(im, gs, B, C)
     out = _out_or_new(out, (B, 1 if smaps is not None else C) + im, grid)
     image = torch.empty((B, C) + im, dtype=grid.dtype, device=grid.device) if combine else out
     ws, nws = _fft_workspace(grid.device, d, im, gs, B, C, smooth)
