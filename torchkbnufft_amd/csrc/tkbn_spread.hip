@@ -3784,9 +3784,6 @@ int tkbn_batch_interp_adj(const tkbn_batch* b, const void* table, void* workspac
 
 }  // extern "C"
 
-namespace tkbn {
-}  // namespace tkbn
-
 // ---- adjoint without device allocation -------------------------------------------
 // tkbn_interp_adj_noalloc keeps its workspace (plan-cache header, trajectory copy,
 // plan) in `scratch`, a static device array that every GPU the library runs on holds
