@@ -54,8 +54,11 @@ def require_gpu(*tensors: Tensor) -> torch.device:
 
 def plain(t: Tensor) -> Tensor:
     """``t`` contiguous, with a lazy conjugate or negative carried out: the kernels read the
-    memory as it lies, and ``contiguous()`` keeps those bits."""
-    return t.resolve_conj().resolve_neg().contiguous()
+    memory as it lies, and ``contiguous()`` keeps those bits.  (Asked for first: a dozen tensors
+    pass here in a pair of calls, and resolving what needs none costs 0.3 us more each.)"""
+    if t.is_conj() or t.is_neg():
+        t = t.resolve_conj().resolve_neg()
+    return t.contiguous()
 
 
 def real_dtype_of(t: Tensor) -> torch.dtype:
