@@ -61,6 +61,14 @@ def plain(t: Tensor) -> Tensor:
     return t.contiguous()
 
 
+def plain_as(t: Tensor, like: Tensor, dtype: torch.dtype) -> Tensor:
+    """``plain(t)`` on ``like``'s device in ``dtype`` (a ``to()`` that changes nothing costs more
+    than the comparison)."""
+    if t.dtype != dtype or t.device != like.device:
+        t = t.to(device=like.device, dtype=dtype)
+    return plain(t)
+
+
 def real_dtype_of(t: Tensor) -> torch.dtype:
     return {torch.complex64: torch.float32, torch.complex128: torch.float64}[t.dtype]
 

@@ -19,7 +19,7 @@ from torch import Tensor
 
 from .. import _lib
 from .._autograd._apply import run as _run
-from ._host import host_values, plain, require_gpu
+from ._host import host_values, plain, plain_as, require_gpu
 
 
 def _norm_scale(norm: Optional[str], grid_size) -> float:
@@ -49,7 +49,7 @@ def apod_pad(image: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, im_si
             smaps = smaps.expand(B, *smaps.shape[1:]).contiguous()
         if image.shape[1] not in (1, C):
             raise ValueError("image coil dimension must be 1 or match smaps")
-    sc = plain(scaling_coef.to(device=image.device, dtype=image.dtype))
+    sc = plain_as(scaling_coef, image, image.dtype)
     if sc.numel() != math.prod(im):
         raise ValueError("scaling_coef does not match im_size")
     grid = torch.empty((B, C) + gs, dtype=image.dtype, device=image.device)
@@ -88,7 +88,7 @@ def crop_deapod(grid: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, im_
             smaps = smaps.expand(B, *smaps.shape[1:]).contiguous()
         if tuple(smaps.shape) != (B, C) + im:
             raise ValueError(f"smaps shape {tuple(smaps.shape)} does not match data ({B}, {C}) + {im}")
-    sc = plain(scaling_coef.to(device=grid.device, dtype=grid.dtype))
+    sc = plain_as(scaling_coef, grid, grid.dtype)
     out = torch.empty((B, 1 if smaps is not None else C) + im, dtype=grid.dtype, device=grid.device)
     _crop_deapod_into(grid, smaps, sc, im, scale, out)
     return out
@@ -249,7 +249,7 @@ def fft_grid_fwd(image: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, i
             raise ValueError(f"smaps shape {tuple(smaps.shape)} does not match image {tuple(image.shape)}")
         if image.shape[1] not in (1, C):
             raise ValueError("image coil dimension must be 1 or match smaps")
-    sc = plain(scaling_coef.to(device=image.device, dtype=image.dtype))
+    sc = plain_as(scaling_coef, image, image.dtype)
     grid = _out_or_new(out, (B, C) + gs, image)
     smooth = _smooth(im, gs)
     ws, nws = _fft_workspace(image.device, d, im, gs, B, C, smooth)
@@ -280,7 +280,7 @@ def fft_grid_adj(grid: Tensor, smaps: Optional[Tensor], scaling_coef: Tensor, im
         smaps = plain(smaps)
         if tuple(smaps.shape) != (B, C) + im:
             raise ValueError(f"smaps shape {tuple(smaps.shape)} does not match data ({B}, {C}) + {im}")
-    sc = plain(scaling_coef.to(device=grid.device, dtype=grid.dtype))
+    sc = plain_as(scaling_coef, grid, grid.dtype)
     smooth = _smooth(im, gs)
     combine = smaps is not None and not smooth and not _combines(im, gs, B, C)
     out = _out_or_new(out, (B, 1 if smaps is not None else C) + im, grid)

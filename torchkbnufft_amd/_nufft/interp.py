@@ -16,7 +16,7 @@ import torch
 from torch import Tensor
 
 from .. import _lib
-from ._host import host_values, plain, real_dtype_of, require_gpu
+from ._host import host_values, plain, plain_as, real_dtype_of, require_gpu
 
 # adjoint mode used when the caller does not ask for one
 _DEFAULT_ADJ_MODE = _lib.TKBN_ADJ_ATOMIC
@@ -224,12 +224,12 @@ def _check_out(out: Optional[Tensor], shape: tuple, like: Tensor) -> Tensor:
 
 
 def _prep_tables(tables: List[Tensor], like: Tensor) -> List[Tensor]:
-    return [plain(t.to(device=like.device, dtype=like.dtype)) for t in tables]
+    return [plain_as(t, like, like.dtype) for t in tables]
 
 
 def _prep_omega(omega: Tensor, like: Tensor) -> Tensor:
     # the trajectory is evaluated in the data's real precision (tm, rint, floor)
-    return plain(omega.to(device=like.device, dtype=real_dtype_of(like)))
+    return plain_as(omega, like, real_dtype_of(like))
 
 
 def table_interp(
