@@ -19,11 +19,12 @@
 // one write and one read each, in place (a thread writes the addresses it read), with
 // one barrier per stage.  64 images of 320 x 320 -> 640 x 640 (row pass 157 MB, column pass
 // 315 MB, the filter's column pass 210 MB; a large copy runs at 5.1 TB/s): row pass 47 us
-// forward and 58 us adjoint, column pass 82 and 78 us, filter 108 us.  Stockham passes of
+// forward and 60 us adjoint, column pass 84 and 77 us, filter 98 us.  Stockham passes of
 // radices <= 8 with every value in LDS (six LDS writes and reads per element and nine
 // barriers at length 640) and twiddles evaluated by each group took 69 and 57, 92 and 92,
-// 148 us.  What is left over the copy's time is the butterflies' arithmetic (about 15
-// instructions per element and stage) that three groups per CU do not hide completely.
+// 148 us.  The vector units are busy 79 % of the filter's time, 52 to 54 % of the column passes'
+// (which move 4.0 and 4.3 TB/s) and 28 to 53 % of the row passes': the filter is bound by the
+// butterflies' arithmetic, the others by neither alone.
 // Grid sizes whose prime factors are 2, 3 and 5 have compiled or runtime plans of these
 // radices; the primes 7 to 17 add runtime butterflies of their own size, and a dimension with
 // a larger prime is transformed as a convolution (chirp kernels below).

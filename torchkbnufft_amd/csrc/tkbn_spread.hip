@@ -933,7 +933,8 @@ __global__ void __launch_bounds__((fwd_tiled_threads<T, JM, D>()))
 //   result is the reference's for every table.
 //   Every phase of the frame is evaluated in double and rounded once at the end: with float
 //   phases the results of few-row problems were further from 64-bit sums than those of the
-//   complex-weight kernels (12 rows, 256^2 adjoint: 1.26e-7 against 1.12e-7; now 1.07e-7).
+//   complex-weight kernels (12 rows, 256^2 adjoint, sums in float32: 1.26e-7 against 1.12e-7,
+//   with double phases 1.07e-7).
 // ---------------------------------------------------------------------------
 struct SepGeom {
   int L[2];            // table oversampling
@@ -2320,7 +2321,7 @@ static TileGeom make_coil_tile_geom(const tkbn_interp_desc* d) {
 // work target asks for the sample-lane kernels, whose fields they are, and so does a
 // problem one of whose separable workspaces (72 bytes a sample in the forward, 88 to 108 in
 // the adjoint, tables and tile lists beside) would pass 1 GiB.  Below 32 rows,
-// sample-lane against separable: spread 31 -> 18 us, gather 25 -> 17 us (one row, 512^2 grid,
+// sample-lane against separable: spread 31 -> 21 us, gather 25 -> 17 us (one row, 512^2 grid,
 // 206 000 samples); call pair 371 -> 207 us (8 trajectories x 8 rows, 384^2).
 constexpr int64_t kSepMaxBytes = 1LL << 30;
 static int64_t sep_fwd_bytes(const tkbn_interp_desc* d);
@@ -3312,7 +3313,7 @@ int interp_fwd_tiled(const tkbn_interp_desc* d, const void* grid, const void* om
 
 
 // ---------------------------------------------------------------------------
-// batches of uneven problems (complex64, sample-lane paths): one launch per stage
+// batches of uneven problems (complex64, separable and sample-lane paths): one launch per stage
 //   The caller builds every problem's plans with ordinary tkbn_interp_fwd / _adj calls
 //   (the same workspaces), then describes the problems once (tkbn_batch_create); the
 //   library writes a table of per-problem records (geometry, tile plans, pointers) that
@@ -3323,7 +3324,7 @@ int interp_fwd_tiled(const tkbn_interp_desc* d, const void* grid, const void* om
 // ---------------------------------------------------------------------------
 struct BatchProb {
   Geom<float> g;
-  TileGeom tf, ta;         // forward / adjoint sample-lane tile plans
+  TileGeom tf, ta;         // forward / adjoint tile plans (of either kind)
   const float2* grid_in;   // forward input grid
   float2* kdata_out;       // forward output
   const float2* kdata_in;  // adjoint input
@@ -3413,7 +3414,7 @@ __global__ void __launch_bounds__(256) batch_zero_hot_kernel(const BatchProb* __
   const int64_t t = li / q.ya, yc = li - t * q.ya;
   if (t >= q.ta.NB) return;
   if constexpr (D == 2) {
-    if (q.sep_a) {  // one chunk holds all rows (fewer than 32)
+    if (q.sep_a) {  // the first chunk's block clears all rows (fewer than 32)
       if (yc == 0) sep_zero_hot_item(q.g, q.ta, q.wa, q.grid_out, (int)t, 0, q.g.B * q.g.C);
       return;
     }
@@ -3880,7 +3881,11 @@ int64_t tkbn_interp_adj_workspace_bytes(const tkbn_interp_desc* desc, int32_t mo
   tkbn_interp_desc plain = *desc;
   for (int i = 0; i < 3; ++i) plain.tile[i] = 0;
   plain.work_target = 0;
-  if (!det && coil_variant_eligible(&plain)) n = std::max(n, sep_adj_bytes(desc));
+  if (!det && coil_variant_eligible(&plain)) {
+    // (a tuning that lists more tiles or pieces shows in the size, whichever plan is larger)
+    const int64_t untuned = adj_lane_bytes(&plain, det);
+    n = std::max(untuned, sep_adj_bytes(desc)) + std::max<int64_t>(0, n - untuned);
+  }
   if (reg3_eligible(desc)) {
     const int64_t nr = plan_cache_bytes(desc) + reg3_workspace_bytes(make_reg3_geom(desc, det));
     n = nr > n ? nr : n;
